@@ -15,6 +15,7 @@
 //                 the token's position), then scores, softmax and P.V over
 //                 one 128-position split of the cache           (:1200-1222)
 //   k_attn_comb   the splits merged per head                   (flash-decoding merge)
+//   k_attn_tile   instead of the two, a prompt's positions over one bf16 cache
 //   k_gemv_part   Wo . att per slice; the MoE router sums the slices into
 //                 the residual                                  (:1225-1232, :1546-1547)
 //   k_rms_rows    the final RMSNorm                            (:1556)
@@ -603,12 +604,34 @@ __device__ __forceinline__ void kv_store_f32(const KvFin& k, const AttnArgs& a, 
 
 // For a batch whose tokens may share a cache (a prefill chunk: the
 // positions of one prompt), every token's k and v rows are appended before
-// the attention reads the caches: one wave per (KV head, token).
+// the attention reads the caches: wave 0 of block (KV head, token).  With
+// a.qhl the block's other waves finish the KV head's query heads, two per
+// wave, for k_attn_tile: split for the matrix cores (bf16(q), bf16(q - hi))
+// into qhl[token][head][2][128].
 template <bool F32>
-__global__ void __launch_bounds__(64)
+__global__ void __launch_bounds__(320)
 k_kv_append(AttnArgs a) {
+    constexpr int HD = 128;
     const int kh = blockIdx.x, b = blockIdx.y;
     const int pos = a.pos[b];
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (w > 0) {
+        const int qpk = a.H / a.KH, j = threadIdx.x & 31, q = (threadIdx.x >> 5) - 2;
+        const int head = kh * qpk + (q < qpk ? q : 0), row = head * HD + 4 * j;
+        Fin4 f;
+        fin4_load(f, a, b, row, a.bq, row, qk_weight(a, true, head), true, pos, j);
+        float v[4];
+        fin4_value(v, f, a, b, row, a.qn ? a.qk_norm : 0, true, j);
+        uint32_t hi[2], lo[2];
+        split_bf16x2(v[0], v[1], hi[0], lo[0]);
+        split_bf16x2(v[2], v[3], hi[1], lo[1]);
+        uint16_t* o = a.qhl + ((size_t)b * a.H + head) * 2 * HD + 4 * j;
+        if (q < qpk) {
+            *(uint2*)o = make_uint2(hi[0], hi[1]);
+            *(uint2*)(o + HD) = make_uint2(lo[0], lo[1]);
+        }
+        return;
+    }
     const unsigned long long* kvp = a.kv + ((size_t)b * a.L + a.layer) * 2;
     KvFin k;
     kv_load(k, a, b, kh, pos, threadIdx.x);
@@ -1012,6 +1035,302 @@ k_attn_part_f32(AttnArgs a) {
     merge_waves<QPK>(a, b, kh, s, &red[0][0], QPK * HD, mls);
 }
 
+// ---------------------------------------------------- prefill attention
+//
+// Attention of a chunk of positions of one prompt (every token of the call
+// reads the same caches, whose rows k_kv_append has written): block (KV head,
+// 64 query rows = 64 / QPK tokens x QPK heads), 8 waves = 2 row groups of 32
+// query rows x 4 position strides: in step i wave (rg, ks) takes the
+// 32-position tile 4 i + ks of its rows' prefix with an online softmax, and
+// the 4 waves of a row group merge once at the end.  k_attn_part's
+// per-position form reads K and V, finishes the query heads and merges 4
+// waves for every (position, split); here a K or V row is read once per 64
+// query rows and the merge launch drops out.
+//
+// Scores by v_mfma_f32_32x32x16_bf16, K rows as A (lane l: position l % 32,
+// dimensions 16 kk + 8 (l / 32) .. + 7), the query rows as B (hi and lo bf16,
+// two products as k_attn_part's columns), so that lane l holds query row
+// l % 32 at positions 8 (v / 4) + 4 (l / 32) + v % 4: the softmax needs one
+// exchange, with lane l ^ 32.  P . V with V^T as A and the weights as B,
+// taken from the registers that computed them (contraction index j of half h
+// in step s is position 16 s + 8 (j / 4) + 4 h + j % 4);
+// ds_read_b64_tr_b16 reads 4 positions of 16 dimensions of V transposed.
+//
+// A step's 128 K and V rows (64 KB) go straight to LDS (global_load_lds),
+// two steps in two arrays: the rows of step i + 2 are requested when step i
+// is done, so a row has a whole step to arrive.  (Two arrays, so that the
+// compiler sees that a step's reads do not wait for the other's rows.)  The
+// 16-byte chunk c of K row r sits at chunk c ^ (r % 16), of V row r at c ^ 4
+// (r % 4): the reads of both fall in different banks.
+//
+// Bound: in a step the 8 waves run their products (64 MFMAs per SIMD, 2048
+// cycles) and their weights (about 1700 cycles of vector work) in phase, 1.9
+// us; a 512-token chunk of a 32/4-head model has at most 4 + the rows before
+// it / 128 steps, and about 11 us of launch, first rows and merge.  Measured
+// (append + attention launches): 512 tokens at 32/4 heads 28 us, per-position
+// form 70; the chunks of a 1531-token prompt 115 us per layer, 385 before;
+// 301 tokens at 32/8 heads 22 us, 54 before.  Staging each wave's own tile
+// with one step's rows in flight took 2.6 us per 32 positions instead of 1.9;
+// finishing the query rows here instead of in k_kv_append's launch 3 to 6 us
+// more per launch.
+constexpr int AT_ROWS = 64;             // query rows per block
+constexpr int AT_STEP = 128;            // positions per step
+
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+typedef float floatx16a __attribute__((ext_vector_type(16)));
+
+// 4 rows x 16 columns of bf16 in LDS, transposed over 16 lanes: lane i gives
+// the address of 4 columns (4 (i % 4) ..) of row i / 4 and receives column
+// i of rows 0..3
+__device__ __forceinline__ s16x4 lds_tr16(const uint16_t* p) {
+    return __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)(void*)p);
+}
+
+// e^-x weights as powers of two; at most -150 apart they are 0.  A NaN
+// score's weight is 0 (fmaxf drops the NaN), as expf_fast(NaN) is.
+__device__ __forceinline__ float exp2_w(float x) { return __builtin_amdgcn_exp2f(fmaxf(x, -150.0f)); }
+
+// A block barrier without fences: what must have completed before it is
+// waited for explicitly (a fence would also wait for the loads to LDS that
+// are meant to stay in flight).
+__device__ __forceinline__ void wave_meet() {
+    __asm__ volatile("" : : : "memory");
+    __builtin_amdgcn_s_barrier();
+    __asm__ volatile("" : : : "memory");
+}
+
+template <int QPK>
+__global__ void __launch_bounds__(512, 2)
+k_attn_tile(AttnArgs a, float* __restrict__ att) {
+    constexpr int HD = 128, TQ = AT_ROWS / QPK, RT = 32 / QPK, TILE = 32 * HD;
+    // two steps' rows: 4 tiles of K, then 4 of V; after the loop the outputs
+    // being merged
+    __shared__ __align__(16) uint16_t kv0[2 * AT_STEP * HD];
+    __shared__ __align__(16) uint16_t kv1[2 * AT_STEP * HD];
+    __shared__ float mls[8][32][2];
+    // per query row: which dimensions met a V value of +Inf (bit 0) or -Inf
+    // (bit 1) or NaN (both), 16 dimensions per word
+    __shared__ uint32_t taint[AT_ROWS][HD / 16];
+    static_assert(4 * 64 * 64 * 4 == sizeof(kv0), "a step's space holds the outputs of 4 waves");
+    const int kh = blockIdx.x, b0 = ((int)gridDim.y - 1 - (int)blockIdx.y) * TQ;   // longest prefixes first
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6), rg = w & 1, ks = w >> 1;
+    const int n = lane & 31, h = lane >> 5;
+    const unsigned long long* kvp = a.kv + ((size_t)b0 * a.L + a.layer) * 2;
+    const gptr<const uint16_t> src = (gptr<const uint16_t>)kvp[rg];     // what this wave loads: K (rg 0) or V rows
+
+    // row n of the row group is token tb; the positions of the block's 64
+    // rows (lane's first and last) bound its steps and its unmasked tiles
+    const int tb = b0 + rg * RT + n / QPK;
+    const int prow = a.pos[min(tb, a.B - 1)];
+    int pmax = a.pos[min(b0 + lane / QPK, a.B - 1)], pmin = pmax;
+#pragma unroll
+    for (int o = 32; o; o >>= 1) {
+        pmax = max(pmax, __shfl_xor(pmax, o, JM_WAVE));
+        pmin = min(pmin, __shfl_xor(pmin, o, JM_WAVE));
+    }
+    pmax = __builtin_amdgcn_readfirstlane(pmax);
+    pmin = __builtin_amdgcn_readfirstlane(pmin);
+    const int nstep = pmax / AT_STEP + 1;
+
+    // This wave's rows of step i: the K or V rows of tile 4 i + ks, load j
+    // rows 4 j .. 4 j + 3 (lane l row 4 j + l / 16, LDS chunk l % 16).  Rows
+    // past the prefixes repeat the last one (their weights are 0).
+    const uint32_t rstride = (uint32_t)a.KH * HD;
+    auto load_step = [&](int i, uint16_t* kv) __attribute__((always_inline)) {
+        const int t = min(4 * i + ks, pmax / 32);
+        const gptr<const uint16_t> base = src + ((size_t)(32 * t) * a.KH + kh) * HD;
+        uint16_t* const dst = kv + (4 * rg + ks) * TILE;
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+            const int r = 4 * j + (lane >> 4);
+            const int x = rg ? 4 * (lane >> 4) : (r & 15);
+            __builtin_amdgcn_global_load_lds(
+                (gptr<void>)(base + ((uint32_t)min(r, pmax - 32 * t) * rstride + 8 * ((lane & 15) ^ x))),
+                (__attribute__((address_space(3))) void*)(dst + 4 * j * HD), 16, 0, 0);
+        }
+    };
+
+    // the query rows, finished by k_kv_append
+    bf16x8 qh[8], ql[8];
+    {
+        const uint16_t* q = a.qhl + ((size_t)min(tb, a.B - 1) * a.H + kh * QPK + n % QPK) * 2 * HD + 8 * h;
+#pragma unroll
+        for (int kk = 0; kk < 8; kk++) {
+            qh[kk] = __builtin_bit_cast(bf16x8, *(const uint4*)(q + 16 * kk));
+            ql[kk] = __builtin_bit_cast(bf16x8, *(const uint4*)(q + HD + 16 * kk));
+        }
+    }
+    load_step(0, kv0);
+    (&taint[0][0])[tid] = 0;
+    static_assert(sizeof(taint) == 512 * 4, "a taint word per thread");
+    if (nstep > 1) load_step(1, kv1);
+
+    // scores as powers of two: q . k / sqrtf_fast(hd) times log2(e)
+    const float c2 = __fmul_rn(a.rsdiv, 1.4426950408889634f);
+    const int kx = h ^ (n & 15);            // K row n: dimensions 16 kk + 8 h .. at chunk (2 kk) ^ kx
+    // this lane's part of a transposed read: row 4 h + i / 4, 4 columns
+    // 16 (l / 16 % 2) + 4 (i % 4) of a 32-column block, i = l % 16
+    const int vrow = (lane & 15) >> 2;      // row % 4
+    const int vo = (4 * h + vrow) * HD + 8 * (2 * ((lane >> 4) & 1) + ((lane >> 1) & 1)) + 4 * (lane & 1);
+    floatx16a O[4] = {};
+    float m = -INFINITY, l = 0.0f;
+
+    auto step = [&](int i, uint16_t* kv) __attribute__((always_inline)) {
+        // this wave's rows of step i have arrived (8 loads of step i + 1 may
+        // be outstanding), then everyone's
+        if (i + 1 < nstep) __builtin_amdgcn_s_waitcnt(0x0F78);      // vmcnt(8)
+        else __builtin_amdgcn_s_waitcnt(0x0F70);                    // vmcnt(0)
+        wave_meet();
+        const int t = 4 * i + ks;
+        uint16_t* const kw = kv + ks * TILE;
+        uint16_t* const vw = kv + (4 + ks) * TILE;
+        if (AT_STEP * i + AT_STEP - 1 > pmin) {
+            // A weight of 0 does not hide a non-finite V value from the
+            // matrix product.  In a step that reaches past some row's prefix
+            // such values go into `taint`, for the rows whose prefix holds
+            // them, and out of the step.  (Block-uniform.)
+            uint32_t nf = 0;
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const uint4 u = *(const uint4*)(vw + 8 * (256 * rg + 64 * j + lane));
+                const uint32_t x[4] = {u.x, u.y, u.z, u.w};
+#pragma unroll
+                for (int e = 0; e < 4; e++)
+                    nf |= (uint32_t)((x[e] & 0x7F80u) == 0x7F80u) | (uint32_t)((x[e] & 0x7F800000u) == 0x7F800000u);
+            }
+            if (__syncthreads_or(nf != 0)) {
+#pragma unroll 1
+                for (int e = lane; e < TILE; e += 64) {
+                    const int r = e / HD, dim = (e % HD) ^ (32 * (r & 3));
+                    const uint32_t x = vw[e];
+                    if ((x & 0x7F80u) != 0x7F80u) continue;
+                    const uint32_t bits = (x & 0x7Fu) ? 3u : (x >> 15) ? 2u : 1u;
+#pragma unroll 1
+                    for (int q = 0; q < 32; q++)
+                        if (32 * t + r <= a.pos[min(b0 + rg * RT + q / QPK, a.B - 1)])
+                            atomicOr(&taint[32 * rg + q][dim / 16], bits << (2 * (dim % 16)));
+                }
+                __syncthreads();
+                if (rg == 0) {
+#pragma unroll 1
+                    for (int e = lane; e < TILE; e += 64)
+                        if ((vw[e] & 0x7F80u) == 0x7F80u) vw[e] = 0;
+                }
+                __syncthreads();
+            }
+        }
+        if (32 * t <= pmax) {
+            floatx16a S = {};
+#pragma unroll
+            for (int kk = 0; kk < 8; kk++) {
+                const bf16x8 k8 = __builtin_bit_cast(bf16x8, *(const uint4*)(kw + n * HD + 8 * ((2 * kk) ^ kx)));
+                S = __builtin_amdgcn_mfma_f32_32x32x16_bf16(k8, ql[kk], S, 0, 0, 0);
+                S = __builtin_amdgcn_mfma_f32_32x32x16_bf16(k8, qh[kk], S, 0, 0, 0);
+            }
+            if (32 * t + 31 > pmin) {
+#pragma unroll
+                for (int v = 0; v < 16; v++)
+                    if (32 * t + 8 * (v / 4) + 4 * h + v % 4 > prow) S[v] = -INFINITY;
+            }
+            float mt = S[0];
+#pragma unroll
+            for (int v = 1; v < 16; v++) mt = fmaxf(mt, S[v]);
+            mt = fmaxf(mt, __shfl_xor(mt, 32, JM_WAVE));
+            const float mn = fmaxf(m, __fmul_rn(mt, c2));
+            const float mref = mn == -INFINITY ? 0.0f : mn;         // a row with no score yet
+            if (__any(mn != m)) {
+                const float f = exp2_w(__fsub_rn(m, mref));
+                l = __fmul_rn(l, f);
+#pragma unroll
+                for (int nt = 0; nt < 4; nt++)
+#pragma unroll
+                    for (int v = 0; v < 16; v++) O[nt][v] = __fmul_rn(O[nt][v], f);
+                m = mn;
+            }
+            float p[16];
+#pragma unroll
+            for (int v = 0; v < 16; v++) {
+                p[v] = exp2_w(__builtin_fmaf(S[v], c2, -mref));
+                l = __fadd_rn(l, p[v]);
+            }
+#pragma unroll
+            for (int s = 0; s < 2; s++) {
+                uint32_t hi[4], lo[4];
+#pragma unroll
+                for (int e = 0; e < 4; e++) split_bf16x2(p[8 * s + 2 * e], p[8 * s + 2 * e + 1], hi[e], lo[e]);
+                const bf16x8 ph = __builtin_bit_cast(bf16x8, make_uint4(hi[0], hi[1], hi[2], hi[3]));
+                const bf16x8 pl = __builtin_bit_cast(bf16x8, make_uint4(lo[0], lo[1], lo[2], lo[3]));
+#pragma unroll
+                for (int nt = 0; nt < 4; nt++) {
+                    const s16x4 v0 = lds_tr16(vw + vo + 16 * s * HD + 32 * (nt ^ vrow));
+                    const s16x4 v1 = lds_tr16(vw + vo + (16 * s + 8) * HD + 32 * (nt ^ vrow));
+                    const bf16x8 va = __builtin_bit_cast(bf16x8, __builtin_shufflevector(v0, v1, 0, 1, 2, 3, 4, 5, 6, 7));
+                    O[nt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va, pl, O[nt], 0, 0, 0);
+                    O[nt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va, ph, O[nt], 0, 0, 0);
+                }
+            }
+        }
+        __builtin_amdgcn_s_waitcnt(0xC07F); // lgkmcnt(0): this wave's reads of the step, then
+        wave_meet();                        // everyone's, are done
+        if (i + 2 < nstep) load_step(i + 2, kv);
+    };
+#pragma unroll 1
+    for (int i = 0; i < nstep; i += 2) {
+        step(i, kv0);
+        if (i + 1 < nstep) step(i + 1, kv1);
+    }
+
+    // ---- the 4 waves of each row group merged with the rows' max
+    l = __fadd_rn(l, __shfl_xor(l, 32, JM_WAVE));
+    if (h == 0) {
+        mls[w][n][0] = m;
+        mls[w][n][1] = l;
+    }
+    __syncthreads();
+    float M = -INFINITY, L = 0.0f;
+#pragma unroll
+    for (int u = 0; u < 4; u++) M = fmaxf(M, mls[2 * u + rg][n][0]);
+    if (M == -INFINITY) M = 0.0f;
+#pragma unroll
+    for (int u = 0; u < 4; u++) L = __builtin_fmaf(mls[2 * u + rg][n][1], exp2_w(__fsub_rn(mls[2 * u + rg][n][0], M)), L);
+    // every wave's outputs to LDS (row group, then 32-dimension block, then
+    // wave), the rows' 32-dimension block ks summed by wave ks, over the
+    // waves in order
+    const float f = exp2_w(__fsub_rn(m, M));
+    float4* const mb = (float4*)(rg ? &kv1[0] : &kv0[0]) + lane;        // [nt][wave][4][64 lanes]
+#pragma unroll
+    for (int nt = 0; nt < 4; nt++)
+#pragma unroll
+        for (int q = 0; q < 4; q++)
+            mb[((nt * 4 + ks) * 4 + q) * 64] =
+                make_float4(__fmul_rn(O[nt][4 * q], f), __fmul_rn(O[nt][4 * q + 1], f), __fmul_rn(O[nt][4 * q + 2], f),
+                            __fmul_rn(O[nt][4 * q + 3], f));
+    __syncthreads();
+    const float r = __fdiv_rn(1.0f, L);
+    if (tb < a.B) {
+        float* out = att + ((size_t)tb * a.H + kh * QPK + n % QPK) * HD + 32 * ks + 4 * h;
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            float4 s = mb[((ks * 4 + 0) * 4 + q) * 64];
+#pragma unroll
+            for (int u = 1; u < 4; u++) {
+                const float4 x = mb[((ks * 4 + u) * 4 + q) * 64];
+                s = make_float4(__fadd_rn(s.x, x.x), __fadd_rn(s.y, x.y), __fadd_rn(s.z, x.z), __fadd_rn(s.w, x.w));
+            }
+            const uint32_t tw = taint[32 * rg + n][2 * ks + q / 2] >> (16 * (q % 2) + 8 * h);   // dimensions 8 q + 4 h ..
+            float o[4] = {s.x, s.y, s.z, s.w};
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const uint32_t x = (tw >> (2 * e)) & 3u;
+                const float add = x == 0 ? 0.0f : x == 1 ? INFINITY : x == 2 ? -INFINITY : __int_as_float(0x7FC00000);
+                o[e] = __fmul_rn(__fadd_rn(o[e], add), r);
+            }
+            *(float4*)(out + 8 * q) = make_float4(o[0], o[1], o[2], o[3]);
+        }
+    }
+}
+
 // Merge of the splits of one (query head, token): out = sum_s o_s e^(m_s - M)
 // / sum_s l_s e^(m_s - M), M the max over the splits.  The splits' weights
 // are computed in parallel (128 at a time) and staged in LDS; each thread
@@ -1095,11 +1414,30 @@ hipError_t launch_attn(const AttnArgs& a, int qpk, float* att, hipStream_t st) {
         hipError_t e0 = hipGetLastError();
         if (e0 != hipSuccess) return e0;
     }
+    const bool tile = !a.append && a.shared && !a.kv_f32 && (long long)a.B * a.KH >= JM_ATTN_TILE_MIN;
+    if (qpk != 1 && qpk != 2 && qpk != 4 && qpk != 8) return hipErrorInvalidValue;
     if (!a.append) {
-        if (a.kv_f32) hipLaunchKernelGGL(k_kv_append<true>, dim3((unsigned)a.KH, (unsigned)a.B), dim3(64), 0, st, a);
-        else hipLaunchKernelGGL(k_kv_append<false>, dim3((unsigned)a.KH, (unsigned)a.B), dim3(64), 0, st, a);
+        // (the partial outputs' buffer, unused by k_attn_tile, holds the query heads for it)
+        AttnArgs ap = a;
+        ap.qhl = tile ? (uint16_t*)a.part_o : nullptr;
+        const dim3 ga((unsigned)a.KH, (unsigned)a.B), gb(tile ? 64 * (1 + (qpk + 1) / 2) : 64);
+        if (a.kv_f32) hipLaunchKernelGGL(k_kv_append<true>, ga, gb, 0, st, ap);
+        else hipLaunchKernelGGL(k_kv_append<false>, ga, gb, 0, st, ap);
         hipError_t e0 = hipGetLastError();
         if (e0 != hipSuccess) return e0;
+    }
+    if (tile) {
+        AttnArgs ap = a;
+        ap.qhl = (uint16_t*)a.part_o;
+        const int tq = AT_ROWS / qpk;
+        const dim3 gt((unsigned)a.KH, (unsigned)((a.B + tq - 1) / tq));
+        switch (qpk) {
+            case 1: hipLaunchKernelGGL(k_attn_tile<1>, gt, dim3(512), 0, st, ap, att); break;
+            case 2: hipLaunchKernelGGL(k_attn_tile<2>, gt, dim3(512), 0, st, ap, att); break;
+            case 4: hipLaunchKernelGGL(k_attn_tile<4>, gt, dim3(512), 0, st, ap, att); break;
+            default: hipLaunchKernelGGL(k_attn_tile<8>, gt, dim3(512), 0, st, ap, att); break;
+        }
+        return hipGetLastError();
     }
     // Split s of (KV head kh, token b) is block (kh, b, S - 1 - s): the
     // splits are dispatched from the last one, which holds the fewest

@@ -162,7 +162,7 @@ int run_layers(const jm_store* s, int L) { return s->max_layers < 0 ? L : std::m
 
 // Every launch of one decode step on st (after the staging copy).
 int enqueue_step(jm_store* s, const jm_kernel_cfg* c, const jm_kernel_w* W, const float* xin, int B,
-                 float* hidden, float* logits, int* out_tok, int S, int qpk, bool append, bool capturing,
+                 float* hidden, float* logits, int* out_tok, int S, int qpk, bool append, bool shared, bool capturing,
                  hipStream_t st) {
     const int L = c->L, d = c->d, H = c->n_heads, KH = c->n_kv;
     const int nl = run_layers(s, L);
@@ -213,6 +213,7 @@ int enqueue_step(jm_store* s, const jm_kernel_cfg* c, const jm_kernel_w* W, cons
         at.pos = pos_dev; at.kv = s->tab; at.kv_f32 = s->kv_f32; at.L = L; at.layer = l;
         at.S = S; at.part_o = s->part_o; at.part_ml = s->part_ml;
         at.append = append ? 1 : 0;
+        at.shared = shared ? 1 : 0;
         // the grid covers the longest token's splits; the buffers hold S_cap
         // per (token, KV head), indexed with the call's S
         JM_HIP(jm::launch_attn(at, qpk, s->att, st), "attention launch");
@@ -381,6 +382,10 @@ int decode_impl(jm_store* s, const jm_kernel_cfg* c, const jm_kernel_w* W, const
     // (jm_prefill_layers), and there every row is appended by a launch of
     // its own first.  Checked over every k and v pointer of the call.
     const bool append = cache_pointers_distinct(s->tab_host, (size_t)2 * B * L);
+    // one prompt's positions: every token has token 0's caches
+    bool shared = !append;
+    for (int b = 1; b < B && shared; b++)
+        shared = memcmp(s->tab_host + (size_t)2 * b * L, s->tab_host, (size_t)2 * L * 8) == 0;
     int* pos_host = (int*)(s->tab_host + (size_t)2 * B * L);
     memcpy(pos_host, positions, (size_t)B * 4);
     const size_t tab_bytes = (size_t)B * L * 16 + (size_t)B * 4;
@@ -417,6 +422,7 @@ int decode_impl(jm_store* s, const jm_kernel_cfg* c, const jm_kernel_w* W, const
         key.dense_min = s->dense_min;
         key.ndig = s->ndig;
         key.append = append ? 1 : 0;
+        key.shared = shared ? 1 : 0;
         key.kv_f32 = s->kv_f32;
         if (!s->gexec || memcmp(&key, &s->gkey, sizeof key) != 0) {
             if (s->gexec) {
@@ -426,7 +432,7 @@ int decode_impl(jm_store* s, const jm_kernel_cfg* c, const jm_kernel_w* W, const
             }
             if (!s->cap_st) JM_HIP(hipStreamCreateWithFlags(&s->cap_st, hipStreamNonBlocking), "hipStreamCreate");
             JM_HIP(hipStreamBeginCapture(s->cap_st, hipStreamCaptureModeThreadLocal), "hipStreamBeginCapture");
-            const int rc = enqueue_step(s, c, W, xin, B, hidden, logits, out_tok, S, qpk, append, true, s->cap_st);
+            const int rc = enqueue_step(s, c, W, xin, B, hidden, logits, out_tok, S, qpk, append, shared, true, s->cap_st);
             hipGraph_t graph = nullptr;
             const hipError_t ec = hipStreamEndCapture(s->cap_st, &graph);
             if (rc) {
@@ -445,7 +451,7 @@ int decode_impl(jm_store* s, const jm_kernel_cfg* c, const jm_kernel_w* W, const
         JM_HIP(hipGraphLaunch(s->gexec, st), "hipGraphLaunch");
         return 0;
     }
-    return enqueue_step(s, c, W, xin, B, hidden, logits, out_tok, S, qpk, append, false, st);
+    return enqueue_step(s, c, W, xin, B, hidden, logits, out_tok, S, qpk, append, shared, false, st);
 }
 
 }  // namespace

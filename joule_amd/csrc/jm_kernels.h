@@ -247,10 +247,24 @@ struct AttnArgs {
     int L, layer;
     int append;               // 1: every token has its own cache; the attention appends its k and v
                               // rows itself.  0: k_kv_append appends every row first
+    int shared;               // 1: every token reads the same k cache and the same v cache (one prompt's positions)
     int S;                    // splits the partial buffers hold per (token, KV head)
     float* part_o;            // [B][KH][S][H/KH][128]
+    uint16_t* qhl;            // [B][H][2][128] finished query heads for k_attn_tile (launch_attn sets it)
     float* part_ml;           // [B][KH][S][H/KH][2]
 };
+// tokens x KV heads of one prompt's call over bf16 caches from which it takes
+// the query-tiled kernel (k_attn_tile).  Below, too few of its blocks (one
+// per KV head and 64 query rows) share the prefix.  A layer at prefixes of
+// 200 / 1000 / 4000 positions, per-position form vs tiled, us: 4 KV heads, 64
+// tokens 58.9 / 71.2 / 115.8 vs 61.2 / 72.2 / 118.0, 96 tokens 64.8 / 83.1 /
+// 150.1 vs 63.9 / 75.1 / 120.7; 8 KV heads, 32 tokens 48.9 / 60.1 / 100.3 vs
+// 49.8 / 63.6 / 108.9, 48 tokens 59.4 / 76.0 / 135.8 vs 60.7 / 73.4 / 118.5;
+// 16 KV heads, 16 tokens 41.2 / 50.2 / 86.9 vs 41.9 / 53.0 / 99.0, 20 tokens
+// 44.6 / 56.2 / 102.7 vs 44.2 / 55.6 / 103.0.
+#ifndef JM_ATTN_TILE_MIN
+#define JM_ATTN_TILE_MIN 320
+#endif
 // the projections finished (q out, k and v appended), partial attention,
 // then the merge into att [B][H*128]
 hipError_t launch_attn(const AttnArgs& a, int qpk, float* att, hipStream_t st);

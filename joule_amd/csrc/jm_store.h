@@ -68,6 +68,7 @@ struct DecKey {
     int dense_min;
     int ndig;
     int append;                 // the attention appends the k and v rows itself (no cache shared by two tokens)
+    int shared;                 // every token has the same caches
 };
 
 struct jm_store {
