@@ -111,10 +111,11 @@ int jm_store_reserve(jm_store* s, int max_B);
 int jm_store_info(const jm_store* s, int* L, int* E, int* d, int* m, int* topk, int* group);
 
 /* Batches with B * topk > 256 slots: an expert routed at least min_tokens
- * slots takes the MFMA branch (32-token tiles on the int8 matrix cores:
- * weights q - 8 against each activation's two int8 digits), the others the
- * wave-item GEMV kernels.  0 restores the default (8); a value above
- * B * topk keeps every expert on the GEMV kernels.  No counterpart in the
+ * slots takes the MFMA branch (32-token tiles on the fp6 matrix cores: the
+ * nibbles q against each activation's four base-16 digits), the others the
+ * wave-item GEMV kernels.  0 restores the default (8, or 3 in calls with fewer
+ * than 16 slots per expert); a value above B * topk keeps every expert on the
+ * GEMV kernels.  No counterpart in the
  * reference, whose batch is at most 16 tokens (decode_kernel.c:1522). */
 int jm_store_set_dense_min(jm_store* s, int min_tokens);
 

@@ -103,7 +103,9 @@ std::atomic<int> g_q4_gemm_min_t{JM_Q4_GEMM_MIN_T};
 // the array's name as an address: jm_store_create resolves the device
 // address once per device (hipGetSymbolAddress with that device current)
 // into scratch_ptr, and the calls lay the workspace out from there.
-static __device__ __align__(256) unsigned char scratch[JM_NOALLOC_SCRATCH_BYTES];
+// (An eighth more than the bound on the batches: ws_noalloc_bytes.)
+constexpr size_t SCRATCH_BYTES = (size_t)JM_NOALLOC_SCRATCH_BYTES / 8 * 9;
+static __device__ __align__(256) unsigned char scratch[SCRATCH_BYTES];
 
 namespace {
 
@@ -153,7 +155,7 @@ int check_group_shape(int d, int m, int group) {
 namespace {
 
 // Sizes of the Ws fields for B tokens, in field order.
-constexpr int WS_NF = 27;
+constexpr int WS_NF = 25;
 void ws_sizes(const jm_store* s, int B, size_t (&sz)[WS_NF]) {
     const int E = s->E, d = s->d, m = s->m, k = s->topk, G = s->group;
     const size_t nslot = (size_t)B * k;
@@ -174,21 +176,19 @@ void ws_sizes(const jm_store* s, int B, size_t (&sz)[WS_NF]) {
         (size_t)E * 4,                // first_slot
         nslot * 4,                    // comb
         (size_t)E * sizeof(jm::ExpertWork),   // work table
-        max_tiles * 8,                // dense tiles
+        (max_tiles + 1) * 16,         // dense tiles
         8,                            // n_tiles (tiles, small experts)
         (size_t)E * 4,                // small
         nslot * m * 4,                // act
         nslot * words_m * 4,          // adig
         nslot * (m / 32) * 4,         // ascale
         nslot * d * 4,                // y
-        nslot * m,                    // aqh
-        nslot * m,                    // aql
-        (size_t)B * d,                // xqh
-        (size_t)B * d,                // xql
-        (size_t)B * (d / G) * 4,      // xqs
-        nslot * (m / G) * 4,          // aqs
-        (size_t)B * (d / G) * 4,      // xqc
-        nslot * (m / G) * 4,          // aqc
+        nslot * m * 3,                // aq
+        (size_t)B * d * 3,            // xq
+        (size_t)B * (d / G) * 4,      // xc
+        nslot * (m / G) * 4,          // ac
+        (size_t)B * (d / G),          // xe
+        nslot * (m / G),              // ae
     };
     for (int i = 0; i < WS_NF; i++) sz[i] = v[i];
 }
@@ -203,6 +203,21 @@ size_t jm::ws_bytes(const jm_store* s, int B) {
     return total;
 }
 
+// jm_layer_ffn_batch_noalloc's bound was set when the dense branch's operands
+// took 2 bytes per value, a scale and a sum per group, and a tile 8 bytes; it is kept, so that the
+// batches the call takes and refuses are what they were.  The layout above is
+// at most an eighth larger (3 bytes per value, of 17 or more in all).
+size_t jm::ws_noalloc_bytes(const jm_store* s, int B) {
+    const size_t G = s->group, nslot = (size_t)B * s->topk;
+    size_t sz[WS_NF];
+    ws_sizes(s, B, sz);
+    size_t total = 0;
+    sz[12] = (nslot / JM_DENSE_TILE + s->E) * 8;      // dense tiles
+    for (int i = 0; i < WS_NF - 6; i++) total += align256(sz[i]);
+    return total + 2 * align256(nslot * s->m) + 2 * align256((size_t)B * s->d) + 2 * align256(B * (s->d / G) * 4) +
+           2 * align256(nslot * (s->m / G) * 4);
+}
+
 void jm::ws_layout(const jm_store* s, int B, char* base, Ws* w) {
     size_t sz[WS_NF];
     ws_sizes(s, B, sz);
@@ -211,9 +226,8 @@ void jm::ws_layout(const jm_store* s, int B, char* base, Ws* w) {
                            (void**)&w->active, (void**)&w->n_active, (void**)&w->first_slot,
                            (void**)&w->comb, (void**)&w->work, (void**)&w->tiles,
                            (void**)&w->n_tiles, (void**)&w->small, (void**)&w->act, (void**)&w->adig,
-                           (void**)&w->ascale, (void**)&w->y, (void**)&w->aqh, (void**)&w->aql,
-                           (void**)&w->xqh, (void**)&w->xql, (void**)&w->xqs, (void**)&w->aqs,
-                           (void**)&w->xqc, (void**)&w->aqc};
+                           (void**)&w->ascale, (void**)&w->y, (void**)&w->aq, (void**)&w->xq,
+                           (void**)&w->xc, (void**)&w->ac, (void**)&w->xe, (void**)&w->ae};
     static_assert(sizeof(Ws) == WS_NF * sizeof(void*), "a size for every workspace field");
     for (int i = 0; i < WS_NF; i++) {
         *slots[i] = base;
@@ -266,7 +280,7 @@ int create_dense_store(const jm_kernel_cfg* cfg, jm_store** out) {
     jm_store* s = new jm_store();
     memset(s, 0, sizeof *s);
     s->L = L; s->E = 0; s->d = d; s->m = m; s->topk = 0;
-    s->dense_min = JM_DENSE_MIN_DEFAULT;
+    s->dense_min = 0;
     s->ndig = JM_NDIG;
     s->max_layers = -1;
     s->device = dev;
@@ -352,17 +366,20 @@ int ffn_enqueue(jm_store* s, int layer, const float* x, int B, float* out, const
     r.first_slot = w.first_slot; r.comb = w.comb;
     r.work = w.work; r.umax = umax; r.rec = s->rec;
     r.key0 = (long long)layer * E;
-    r.dense_min = s->dense_min; r.tiles = w.tiles; r.n_tiles = w.n_tiles; r.small = w.small;
+    const int dense_min = s->dense_min ? s->dense_min
+                        : nslot < JM_DENSE_FEW_SLOTS * E ? JM_DENSE_MIN_FEW : JM_DENSE_MIN_DEFAULT;
+    r.tiles = w.tiles; r.n_tiles = w.n_tiles; r.small = w.small;
     r.skip_topk = dec && jm::gateup_topk(B, E);
     r.ndig = s->ndig;
-    // From the quad router's batch sizes on the dispatch path, the tokens'
-    // digits are encoded by the dispatch launch, on the CUs its dispatch
-    // block leaves idle, instead of by the router.  The decoder layer's
-    // normalised tokens reach it through y, which the down stage writes
-    // only later.
+    // On the dispatch path the dispatch launch encodes the tokens for the MFMA
+    // branch, on the CUs its dispatch block leaves idle, and from the quad
+    // router's batch sizes on also the digits, which the router then skips.
+    // The decoder layer's normalised tokens reach it through y, which the
+    // down stage writes only later.
     r.enc_late = !dec && B >= JM_ROUTER_QUAD_MIN_B;
     const bool layer_in = io.xpart || io.norm_w;
-    r.xn = r.enc_late && layer_in ? w.y : nullptr;
+    const bool mfma = !dec && s->mfma_ok && dense_min <= nslot;
+    r.xn = (r.enc_late || mfma) && layer_in ? w.y : nullptr;
     r.xenc = layer_in ? w.y : x;
     jm::ExpertArgs a;
     a.blob = s->blob; a.rec = s->rec; a.key0 = (long long)layer * E; a.E = E;
@@ -371,13 +388,12 @@ int ffn_enqueue(jm_store* s, int layer, const float* x, int B, float* out, const
     a.d = d; a.m = s->m; a.topk = k; a.group = G;
     a.tw = w.tw; a.xdig = w.xdig; a.xscale = w.xscale;
     a.act = w.act; a.adig = w.adig; a.ascale = w.ascale; a.y = w.y; a.out = out; a.resid = io.resid;
-    a.dense_min = s->mfma_ok ? s->dense_min : 0x7FFFFFFF;
+    a.dense_min = s->mfma_ok ? dense_min : 0x7FFFFFFF;
     r.dense_min = a.dense_min;
     a.tiles = w.tiles; a.n_tiles = w.n_tiles; a.small = w.small;
-    const bool mfma = !dec && a.dense_min <= nslot;
-    r.xqh = mfma ? w.xqh : nullptr; r.xql = w.xql; r.xqs = w.xqs; r.xqc = w.xqc;
-    a.xqh = w.xqh; a.xql = w.xql; a.xqs = w.xqs; a.xqc = w.xqc;
-    a.aqh = w.aqh; a.aql = w.aql; a.aqs = w.aqs; a.aqc = w.aqc;
+    r.xq = mfma ? w.xq : nullptr; r.xe = w.xe; r.xc = w.xc;
+    a.xq = w.xq; a.xe = w.xe; a.xc = w.xc;
+    a.aq = w.aq; a.ae = w.ae; a.ac = w.ac;
     a.logits = w.logits; a.renorm = s->renorm; a.top_w = w.top; a.tw_w = w.tw;
     a.ndig = s->ndig;
     const int max_tiles = nslot / JM_DENSE_TILE + E;
@@ -468,7 +484,7 @@ int jm_store_create(const jm_kernel_cfg* cfg, int group, const void* blob, uint6
     s->L = L; s->E = E; s->d = d; s->m = m; s->topk = k;
     s->renorm = cfg->norm_topk_prob ? 1 : 0;
     s->group = group;
-    s->dense_min = JM_DENSE_MIN_DEFAULT;
+    s->dense_min = 0;
     s->ndig = JM_NDIG;
     s->mfma_ok = jm::mfma_shape_ok(d, m) && sc16;
     s->max_layers = -1;
@@ -578,7 +594,7 @@ int jm_store_reserve(jm_store* s, int max_B) {
 int jm_store_set_dense_min(jm_store* s, int min_tokens) {
     if (int rc = check_store(s)) return rc;
     if (min_tokens < 0) return fail(JM_ERR_ARG, "min_tokens must be >= 0 (0 = default)");
-    s->dense_min = min_tokens == 0 ? JM_DENSE_MIN_DEFAULT : min_tokens;
+    s->dense_min = min_tokens;
     return 0;
 }
 
@@ -645,8 +661,8 @@ int jm_layer_ffn_batch_noalloc(jm_store* s, int layer, const float* x, int B, fl
     if (B == 0) return 0;
     if (!x || !out) return fail(JM_ERR_ARG, "x and out must be non-NULL");
     if (!aligned(x, 16) || !aligned(out, 16)) return fail(JM_ERR_ARG, "x and out must be 16-byte aligned");
-    const size_t need = jm::ws_bytes(s, B);
-    if (need > (size_t)JM_NOALLOC_SCRATCH_BYTES)
+    const size_t need = jm::ws_noalloc_bytes(s, B);
+    if (need > (size_t)JM_NOALLOC_SCRATCH_BYTES || jm::ws_bytes(s, B) > SCRATCH_BYTES)
         return fail(JM_ERR_SHAPE, "B=%d needs %zu bytes of workspace; the fixed no-allocation workspace holds %zu "
                     "(use jm_layer_ffn_batch, or fewer tokens per call)", B, need, (size_t)JM_NOALLOC_SCRATCH_BYTES);
     void* base = (s->device >= 0 && s->device < MAX_DEVICES) ? scratch_ptr[s->device] : nullptr;

@@ -1090,15 +1090,6 @@ __device__ __forceinline__ s16x4 lds_tr16(const uint16_t* p) {
 // score's weight is 0 (fmaxf drops the NaN), as expf_fast(NaN) is.
 __device__ __forceinline__ float exp2_w(float x) { return __builtin_amdgcn_exp2f(fmaxf(x, -150.0f)); }
 
-// A block barrier without fences: what must have completed before it is
-// waited for explicitly (a fence would also wait for the loads to LDS that
-// are meant to stay in flight).
-__device__ __forceinline__ void wave_meet() {
-    __asm__ volatile("" : : : "memory");
-    __builtin_amdgcn_s_barrier();
-    __asm__ volatile("" : : : "memory");
-}
-
 template <int QPK>
 __global__ void __launch_bounds__(512, 2)
 k_attn_tile(AttnArgs a, float* __restrict__ att) {

@@ -312,108 +312,16 @@ __device__ __forceinline__ int seg_or(int v) {
 
 // ------------------------------------------------- wave-level digit encode
 
-// --------------------------------------- int8 digit pairs (MFMA branch)
-//
-// The MFMA branch multiplies signed int8 weights (q - 8) by activations
-// written as two int8 digits per value: over a G-value group (the columns
-// one weight-scale group covers), a_j = rint(x_j / s) with s = max|x| / 32639,
-// and a_j = 256 hi_j + lo_j with hi_j, lo_j in [-128, 127] (|a_j| <= 32639 =
-// 127 * 256 + 127 keeps hi in range).  A group's integer dot with the
-// weights is exact: |sum_j a_j (q_j - 8)| <= G * 32639 * 8 < 2^24, so its
-// conversion to float is exact as well.
-constexpr int I8_R = 32639;
-
-// Position of value u (0..7) within its aligned 8-value run in the int8
-// operand order: the even values, then the odd ones.  That is the byte
-// order in which one dword of packed nibbles (value i in bits 4i..4i+3)
-// unpacks: its low nibbles, then its high nibbles.
-__host__ __device__ constexpr int i8_pos(int u) { return (u & 1) ? 4 + (u >> 1) : (u >> 1); }
-
-// Encode one group of G floats, value i held by lane i of an aligned G-lane
-// segment (G = 32 or 64): lane i writes its two digits to hi[p] and lo[p],
-// p = its value's place in the int8 operand order; lane 0 writes the scale
-// (NaN when the group holds a non-finite value, so that it propagates) and
-// the sum of the group's integers q = 256 h + l (exact: below 2^24), which
-// the matrix-core kernels fold into their products with unsigned weight
-// nibbles.  Only when `store`; every lane of the segment must call this.
-template <int G>
-__device__ __forceinline__ void encode_i8_group_wave(float v, bool store, int8_t* __restrict__ hi,
-                                                     int8_t* __restrict__ lo, float* __restrict__ scale,
-                                                     int* __restrict__ qsum) {
-    const int i = threadIdx.x & (G - 1);
-    const float a = fabsf(v);
-    const int bad = seg_or<G>(!(a <= 3.4028235e38f) ? 1 : 0);
-    const float mx = seg_max<G>(a);
-    const float inv = (mx > 0.0f && !bad) ? __fdiv_rn((float)I8_R, mx) : 0.0f;
-    const int q = (int)rintf(__fmul_rn(v, inv));
-    const int l = ((q + 128) & 255) - 128;
-    const int h = (q - l) >> 8;
-    const float qs = seg_sum<G>((float)q);
-    if (store) {
-        const int p = (i & ~7) + i8_pos(i & 7);
-        hi[p] = (int8_t)h;
-        lo[p] = (int8_t)l;
-        if (i == 0) {
-            *scale = bad ? __int_as_float(0x7FC00000) : __fdiv_rn(mx, (float)I8_R);
-            *qsum = (int)qs;
-        }
-    }
-}
-
-// Both encodings of one G-value group (one value per lane of a G-lane
-// segment) from one pair of segment reductions: the NDIG base-16 digits and
-// their scale, as encode_group_wave writes them, and with i8 the int8 digit
-// pairs, scale and integer sum, as encode_i8_group_wave writes them (the
-// same values as the two calls).  Only when `store`; every lane of the
-// segment must call this.
-template <int G, int NDIG>
-__device__ __forceinline__ void encode_group_both(float v, bool store, uint32_t* __restrict__ dig,
-                                                  float* __restrict__ scale, bool i8, int8_t* __restrict__ hi,
-                                                  int8_t* __restrict__ lo, float* __restrict__ qscale,
-                                                  int* __restrict__ qsum) {
-    const int i = threadIdx.x & (G - 1);
-    const float a = fabsf(v);
-    const int bad = seg_or<G>(!(a <= 3.4028235e38f) ? 1 : 0);
-    const float mx = seg_max<G>(a);
-    {
-        const float s = digit_scale<NDIG>(mx, bad != 0);
-        const float inv = (mx > 0.0f && !bad) ? __fdiv_rn((float)Digits<NDIG>::R, mx) : 0.0f;
-        int dg[NDIG];
-        split_digits<NDIG>((int)rintf(__fmul_rn(v, inv)), dg);
-#pragma unroll
-        for (int k = 0; k < NDIG; k++) {
-            const int word = seg_or<8>((dg[k] & 15) << (4 * (i & 7)));
-            if (store && (i & 7) == 0) dig[k * (G / 8) + (i >> 3)] = (uint32_t)word;
-        }
-        if (store && i == 0) *scale = s;
-    }
-    if (i8) {
-        const float inv = (mx > 0.0f && !bad) ? __fdiv_rn((float)I8_R, mx) : 0.0f;
-        const int q = (int)rintf(__fmul_rn(v, inv));
-        const int l = ((q + 128) & 255) - 128;
-        const int h = (q - l) >> 8;
-        const float qs = seg_sum<G>((float)q);
-        if (store) {
-            const int p = (i & ~7) + i8_pos(i & 7);
-            hi[p] = (int8_t)h;
-            lo[p] = (int8_t)l;
-            if (i == 0) {
-                *qscale = bad ? __int_as_float(0x7FC00000) : __fdiv_rn(mx, (float)I8_R);
-                *qsum = (int)qs;
-            }
-        }
-    }
-}
-
-// encode_group_both for NT groups at once, one value of each per lane: the
-// groups' reductions, divisions and digits first, with no branch among them,
-// then every store.  The NT dependency chains overlap instead of running one
-// after another between the stores' branches.  The same values as NT calls
-// of encode_group_both (every step is the same per group).
+// Encode NT groups of G floats at once (G = 32 or 64), one value of each per
+// lane of an aligned G-lane segment, as NDIG base-16 digits and a scale each:
+// the groups' reductions, divisions and digits first, with no branch among
+// them, then every store, so that the NT dependency chains overlap.  Lane j*8
+// of the segment writes word j of every digit k of group t to
+// dig[t][k*(G/8)+j]; lane 0 writes the scale.  Only when store[t]; every lane
+// of the segment must call this.
 template <int G, int NDIG, int NT>
 __device__ __forceinline__ void encode_groups_n(const float* v, const bool* store, uint32_t* const* dig,
-                                                float* const* scale, bool i8, int8_t* const* hi, int8_t* const* lo,
-                                                float* const* qscale, int* const* qsum) {
+                                                float* const* scale) {
     const int i = threadIdx.x & (G - 1);
     int bad[NT];
     float mx[NT];
@@ -434,19 +342,6 @@ __device__ __forceinline__ void encode_groups_n(const float* v, const bool* stor
 #pragma unroll
         for (int k = 0; k < NDIG; k++) word[t][k] = (uint32_t)seg_or<8>((dg[k] & 15) << (4 * (i & 7)));
     }
-    int hv[NT], lv[NT], qi[NT];
-    float qsc[NT];
-    if (i8) {
-#pragma unroll
-        for (int t = 0; t < NT; t++) {
-            const float inv = (mx[t] > 0.0f && !bad[t]) ? __fdiv_rn((float)I8_R, mx[t]) : 0.0f;
-            const int q = (int)rintf(__fmul_rn(v[t], inv));
-            lv[t] = ((q + 128) & 255) - 128;
-            hv[t] = (q - lv[t]) >> 8;
-            qi[t] = (int)seg_sum<G>((float)q);
-            qsc[t] = bad[t] ? __int_as_float(0x7FC00000) : __fdiv_rn(mx[t], (float)I8_R);
-        }
-    }
 #pragma unroll
     for (int t = 0; t < NT; t++) {
         if (!store[t]) continue;
@@ -455,15 +350,6 @@ __device__ __forceinline__ void encode_groups_n(const float* v, const bool* stor
             for (int k = 0; k < NDIG; k++) dig[t][k * (G / 8) + (i >> 3)] = word[t][k];
         }
         if (i == 0) *scale[t] = sc[t];
-        if (i8) {
-            const int p = (i & ~7) + i8_pos(i & 7);
-            hi[t][p] = (int8_t)hv[t];
-            lo[t][p] = (int8_t)lv[t];
-            if (i == 0) {
-                *qscale[t] = qsc[t];
-                *qsum[t] = qi[t];
-            }
-        }
     }
 }
 
@@ -475,7 +361,9 @@ __device__ __forceinline__ void encode_groups_n(const float* v, const bool* stor
 template <int G, int NDIG>
 __device__ __forceinline__ void encode_group_wave(float v, bool store, uint32_t* __restrict__ dig,
                                                   float* __restrict__ scale) {
-    encode_group_both<G, NDIG>(v, store, dig, scale, false, nullptr, nullptr, nullptr, nullptr);
+    uint32_t* const d = dig;
+    float* const s = scale;
+    encode_groups_n<G, NDIG, 1>(&v, &store, &d, &s);
 }
 
 // Digits of the 8 values in lanes 0..7 of the wave with the digit scale of
@@ -648,6 +536,15 @@ __device__ __forceinline__ void lds_barrier() {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// A block barrier without fences: what must have completed before it is
+// waited for explicitly (a fence would also wait for the loads to LDS that
+// are meant to stay in flight).
+__device__ __forceinline__ void wave_meet() {
+    __asm__ volatile("" : : : "memory");
+    __builtin_amdgcn_s_barrier();
+    __asm__ volatile("" : : : "memory");
 }
 
 __device__ __forceinline__ uint2 block_exclusive_scan2(uint2 v, unsigned* wsum, uint2* tot) {
@@ -861,7 +758,8 @@ __host__ __device__ constexpr int dispatch_lds_ints(int nslot, int E) {
 // global outputs are not read back), so its barriers order LDS alone.
 // With wn (STABLE false only: it may
 // alias the counts, which are dead once the segment starts are scanned),
-// wn[u] = the slot count of work entry u, for u < umax.
+// wn[u] = the slot count of work entry u (low 16 bits) and its expert (high
+// 16 bits), for u < umax.
 template <bool STABLE = true>
 __device__ __forceinline__ void dispatch_block(const int* top, int nslot, int E, int k, int* lds,
                                                int* __restrict__ seg_off, int* __restrict__ seg_slot,
@@ -971,7 +869,7 @@ __device__ __forceinline__ void dispatch_block(const int* top, int nslot, int E,
             const int u = total_e > 1 ? im : n_multi + is;
             if (u < umax) {
                 work[u] = wk;
-                if (wn) wn[u] = total_e;
+                if (wn) wn[u] = total_e | (tid << 16);
             }
         }
     }

@@ -25,11 +25,18 @@
 // combine done in the down kernel.  Larger calls take the dispatch path.
 #define JM_DEC_SLOTS 256
 // Dispatch path: experts with at least dense_min slots take the MFMA branch,
-// in tiles of this many tokens.  Its int8 operands (weights q - 8, and the
-// activations' two digits) store each run of 8 columns in the order
-// i8_pos gives (jm_device.h): the even columns, then the odd ones.
+// in tiles of this many tokens (fp6 matrix-core operands, jm_mx.h).
 #define JM_DENSE_TILE 32
+// By default (jm_store_set_dense_min): 8 slots, and 3 when a call has fewer
+// than 16 slots per expert, where the experts of 3 to 7 slots are many and
+// their tokens one by one bound the call (their tiles cost the same HBM bytes
+// and a thirty-second of the work).  us per block at 3 vs 8, Qwen3 shape: 33
+// tokens 117.6 vs 118.9, 52 116.9 vs 153.9, 80 124.2 vs 177.0, 128 124.3 vs
+// 169.4; OLMoE shape: 52 94.0 vs 123.2, 100 95.4 vs 107.1; 2 does as well as
+// 3; at 32 slots per expert (512 tokens) 182.8 vs 182.9.
 #define JM_DENSE_MIN_DEFAULT 8
+#define JM_DENSE_MIN_FEW 3
+#define JM_DENSE_FEW_SLOTS 16
 
 namespace jm {
 
@@ -48,10 +55,9 @@ struct ExpertArgs {
     int B;
     int d, m, topk;
     const float* tw;          // [B*k] routing weight of each slot
-    const int8_t* xqh;        // [B][d] tokens as int8 digit pairs (hi, lo) in int8 operand order (MFMA branch)
-    const int8_t* xql;
-    const float* xqs;         // [B][d/G] their scales
-    const int* xqc;           // [B][d/G] sums of their integers 256 h + l per group
+    const uint8_t* xq;        // [B][d / 64][192] tokens as fp6 digit planes (MFMA branch, jm_mx.h)
+    const uint8_t* xe;        // [B][d/G] their exponents
+    const float* xc;          // [B][d/G] their group corrections
     const uint32_t* xdig;     // [B][d/G][NDIG][G/8] token digits
     const float* xscale;      // [B][d/G]
     float* act;               // [B*k][m]   SiLU(gate)*up per slot
@@ -63,13 +69,13 @@ struct ExpertArgs {
     int group;
     // dispatch path, dense branch
     int dense_min;            // experts with at least this many slots take the MFMA kernels
-    const int2* tiles;        // [max tiles] (work entry, token tile) of the dense experts
+    const int4* tiles;        // [max tiles + 1] token tiles of the dense experts: (expert, first position in
+                              // seg_slot, tokens, 0)
     const int* n_tiles;       // [2] how many tiles; how many experts under dense_min (small)
     const int* small;         // [umax] work-table entries of the experts with 1..dense_min-1 slots
-    int8_t* aqh;              // [B*k][m] act as int8 digit pairs for the MFMA down
-    int8_t* aql;
-    float* aqs;               // [B*k][m/G] their scales
-    int* aqc;                 // [B*k][m/G] sums of their integers per group
+    uint8_t* aq;              // [B*k][m / 64][192] act for the MFMA down, as xq
+    uint8_t* ae;              // [B*k][m/G]
+    float* ac;                // [B*k][m/G]
     // decode path with the top-k in the gate/up kernel (gateup_topk): the
     // router scores, and where the table is written
     const float* logits;      // [B][E]
@@ -94,10 +100,9 @@ struct RouteArgs {
     float* logits;            // [B][E]
     uint32_t* xdig;           // [B][d/G][NDIG][G/8]
     float* xscale;            // [B][d/G]
-    int8_t* xqh;              // [B][d] tokens as int8 digit pairs for the MFMA branch (NULL: not needed)
-    int8_t* xql;
-    float* xqs;               // [B][d/G] their scales
-    int* xqc;                 // [B][d/G] sums of their integers per group
+    uint8_t* xq;              // [B][d / 64][192] tokens for the MFMA branch, encoded by the dispatch launch (NULL: not needed)
+    uint8_t* xe;              // [B][d/G] their exponents
+    float* xc;                // [B][d/G] their group corrections
     int* top;                 // [B*k]
     float* tw;                // [B*k]
     int* seg_off;             // [E+1]
@@ -111,14 +116,14 @@ struct RouteArgs {
     RecLoc rec;               // store record offsets
     long long key0;           // layer*E
     int dense_min;            // dispatch path: slots from which an expert takes the MFMA kernels
-    int2* tiles;              // dense tiles (work entry, token tile), in work-table order
+    int4* tiles;              // dense tiles (see ExpertArgs), in work-table order
     int* n_tiles;             // [2] dense tiles; experts under dense_min
     int* small;               // [umax] work-table entries of the experts under dense_min
     int skip_topk;            // 1: the top-k runs in the gate/up kernel
     int ndig;                 // digit planes the router writes to xdig (4 or 5)
-    int enc_late;             // 1: the dispatch launch encodes the tokens, not the router (k_router_quad only)
-    float* xn;                // [B][d] the router's staged tokens, for that encode (NULL: not written)
-    const float* xenc;        // [B][d] the tokens that encode reads (x, or xn)
+    int enc_late;             // 1: the dispatch launch writes the x digits, not the router (k_router_quad only)
+    float* xn;                // [B][d] the router's staged tokens, for the dispatch launch's encodes (NULL: not written)
+    const float* xenc;        // [B][d] the tokens those encodes read (x, or xn)
 };
 // from this many tokens the router serves 4 tokens per block from one read
 // of each group's table (k_router_quad), and on the dispatch path the
@@ -132,8 +137,9 @@ struct RouteArgs {
 // router scores + x digits (one wave per expert group and token), then the
 // top-k of every token (unless skip_topk)
 hipError_t launch_route_tok(const RouteArgs& a, hipStream_t st);
-// dispatch + work table from a.top (dispatch path); with enc_late, also the
-// tokens' digits from a.xenc, on the launch's blocks past the first
+// dispatch + work table from a.top (dispatch path); on the launch's blocks
+// past the first, the tokens of a.xenc as matrix-core records (a.xq) and, with
+// enc_late, as digits
 hipError_t launch_dispatch_work(const RouteArgs& a, hipStream_t st);
 // experts per layer in the router copy: E rounded up to whole groups of 8
 __host__ __device__ constexpr int router_experts_padded(int E) { return (E + 7) / 8 * 8; }
@@ -162,12 +168,12 @@ hipError_t launch_down_comb(const ExpertArgs& a, hipStream_t st);
 // dispatch path: gate/up and down over the work table, then the combine
 hipError_t launch_gateup(const ExpertArgs& a, int umax, hipStream_t st);
 hipError_t launch_down(const ExpertArgs& a, int umax, hipStream_t st);
-// dense branch: 1-D grids of (max_tiles + 1) x (row blocks); the blocks past
-// n_tiles[0] x (row blocks) run the wave items of the n_tiles[1] experts under
+// dense branch: at most two resident blocks per CU, each taking units (token
+// tile, row block) in turn, then the wave items of the n_tiles[1] experts under
 // dense_min (the small list), so no other launch is needed for them.
-// mfma_shape_ok: d and the intermediate multiples of 256, up to 2048, and at
-// most 1024 or a multiple of 1024 (the tile's token digits stay in LDS one
-// 1024-column phase at a time); otherwise the GEMV kernels take every expert
+// mfma_shape_ok: d a multiple of 512 and the intermediate of 256, up to 2048,
+// and at most 1024 or a multiple of 1024; otherwise the GEMV kernels take every
+// expert
 bool mfma_shape_ok(int d, int m);
 hipError_t launch_gateup_mfma(const ExpertArgs& a, int max_tiles, hipStream_t st);
 hipError_t launch_down_mfma(const ExpertArgs& a, int max_tiles, hipStream_t st);

@@ -1,37 +1,52 @@
-// Dense branch of the grouped Q4 expert product (gfx950 int8 MFMA), taken by
-// the experts whose segment holds at least `dense_min` tokens (prefill-sized
-// batches, skewed routing).  The same contraction as the wave-item kernels
-// in jm_experts.hip (decode_kernel.c:1365-1383), as tiled products:
+// Dense branch of the grouped Q4 expert product (gfx950 fp6 matrix cores),
+// taken by the experts whose segment holds at least `dense_min` tokens
+// (prefill-sized batches, skewed routing).  The same contraction as the
+// wave-item kernels in jm_experts.hip (decode_kernel.c:1365-1383), as tiled
+// products:
 //
 //   k_gateup_mfma  per (expert, 32-token tile, 128 intermediate rows):
 //                  G = X . Wg^T and U = X . Wu^T over d, then
-//                  act = (G / (1 + expf_fast(-G))) * U, written as int8
-//                  digit pairs for the down product (and as float)
-//   k_down_mfma    per (expert, 32-token tile, 512 hidden rows in two passes):
+//                  act = (G / (1 + expf_fast(-G))) * U, written for the down
+//                  product (and as float)
+//   k_down_mfma    per (expert, 32-token tile, 256 hidden rows):
 //                  y[slot] = w_slot * (act . Wd^T) over the intermediate
 //
-// Operands:
-//   weights  the signed nibbles q - 8 as int8, unpacked in registers from
-//            the packed record (each wave streams its own rows);
-//   tokens   two int8 digits per value with one float scale per token and
-//            Q4 group (jm_device.h: encode_i8_group_wave): the router kernel
-//            writes them for x, the gate/up epilogue for act.
-// v_mfma_i32_32x32x32_i8 tiles, tokens on the A side (i), weight rows on the
-// B side (n), in the lane layout of jm_mx.h; the lo plane's accumulator
-// starts at -8 times the tokens' group sums (wdigits takes q, not q - 8).
-// So a lane holds one weight row and 16 tokens: the row's group scale is one
-// value per lane, the tokens' scales 16.
+// Operands (jm_mx.h): the nibbles q as fp6, unpacked in registers from the
+// packed rows; the tokens as 4 fp6 digit planes with one power-of-two scale
+// per token and Q4 group, written by the dispatch launch for x and by the
+// gate/up epilogue for act.  Tokens are the rows (A, i) and weight rows the
+// columns (B, n) of v_mfma_scale_f32_32x32x64_f8f6f4, so a lane holds one
+// weight row and 16 tokens.  Four accumulating instructions give a stage's
+// (64 columns') sums already scaled per token; per element the epilogue is
+// one multiply-add by the row's group scale:
+//   acc += P * s_row
+// on top of the -8 of the Q4 code, for all groups at once: a product of
+// the tokens' group corrections (three bf16 terms) and the row scales (two).
 //
-// Per Q4 group of a lane's row and its 16 tokens the two digit products are
-// exact int32 sums (hi and lo), combined as 256 hi + lo (exact, below 2^24 in
-// magnitude), converted to float and accumulated as
-//   acc += (float(256 hi + lo) * s_token) * s_row.
+// A wave takes 32 tokens x 64 weight rows (two 32-row blocks, which share the
+// token operands), a block 4 waves; two blocks share a CU and stay for several
+// units (tile, row block).  Tokens go to LDS in super-stages of 256 columns (24
+// KB, global_load_lds, 4 tokens x 256 bytes per load), weights straight to
+// registers (16 rows x 64 bytes per load, brought into the operand layout by
+// two lane-row swaps), both one super-stage ahead across units: a unit's
+// tile entry, slots, corrections and first operands are requested during the
+// unit before.
 //
-// The whole contraction of a tile's 32 tokens (both digit planes) stays in
-// LDS for the block's lifetime, so the main loop has no barriers: each wave
-// streams its weight rows through a ring of register stages and reads its
-// token operands from LDS.
-#include <atomic>
+// Bound.  512 Zipf-routed Qwen3 tokens (1122 gate/up units, 214 MB of records):
+// a block's super-stage takes 2.7 to 4 us, of which its arithmetic alone is 1.2
+// (per wave 330 vector instructions and 32 MFMAs of 34 cycles) and the rest the
+// records' arrival, 3 to 4.2 TB/s while every block streams; the unit's SwiGLU
+// and encode take 3 to 5; and 1122 units on 512 resident blocks leave the third
+// round a fifth full.  Gate/up 134 -> 99 us, down 64 -> 56 (203 OLMoE tokens: 80
+// -> 66 and 46 -> 38).  The form before (int8 digit pairs, exact int32 group
+// sums, 4 instructions per element for two float scales) moved 56 16-byte LDS
+// reads and writes per wave and super-stage, 3584 LDS cycles of the 3600 that a
+// pair of waves took.  Measured on the way: blocks of one unit 117 and 69 (each
+// waited 7 to 14 us for its chain of loads), three such blocks per CU 108 and
+// 64 (168 registers, spills), tokens staged 32 bytes per lane pair 113 (64
+// address cycles per load instead of 16); the units' column order rotated by
+// expert and row block made no difference.
+#include <algorithm>
 #include <type_traits>
 
 #include "jm_device.h"
@@ -43,506 +58,638 @@ namespace jm {
 
 constexpr int MT = JM_DENSE_TILE;   // tokens per tile (32)
 static_assert(MT == 32, "the tile's tokens are the 32 A rows of one MFMA");
-constexpr int MTHREADS = 512;       // 8 waves per block
+constexpr int MTHREADS = 256;       // 4 waves per block
 constexpr int NWAVE = MTHREADS / 64;
-constexpr int GU_ROWS = 128;        // intermediate rows of a gate/up block (both matrices)
-constexpr int DN_ROWS = 256;        // hidden rows of one pass of a down block (8 waves x 32)
-constexpr int DN_BLOCK_ROWS = 512;  // hidden rows of a down block: two passes over its staged act digits
+constexpr int WROWS = 64;           // weight rows per wave: two 32-row blocks
+constexpr int GU_ROWS = 128;        // intermediate rows of a gate/up block (each wave: 32 of both matrices)
+constexpr int DN_ROWS = 256;        // hidden rows of a down block (4 waves x 64)
 constexpr int KMAX = 2048;          // longest contraction the kernels take
-constexpr int KPAD = 16;            // bytes of padding per LDS token row (bank spread)
-constexpr int KPH_MAX = 1024;       // columns of a token phase (the tokens' LDS holds one phase)
-constexpr int SSC = 256;            // columns of a weight super-stage: 128 bytes (one cache line) per row
-constexpr int WRS = 144;            // LDS bytes per row of a wave's weight buffer (128 + bank spread)
-constexpr int WBUF = 32 * WRS;      // one super-stage of a wave's 32 rows
+constexpr int SSC = 256;            // columns of a super-stage: 128 bytes (one cache line) per weight row
+constexpr int PIECE = 64 * 16;      // LDS bytes of one record piece of a stage (16 bytes per lane)
+constexpr int RING = 4 * 6 * PIECE; // LDS bytes of a super-stage's token operands
 
-struct TileInfo {
-    int slot0;      // first position of the tile in seg_slot
-    int nt;         // tokens in the tile (1..MT)
-    int e;          // expert id
+// The tokens' buffers, one super-stage each: separate arrays, so that the
+// compiler sees that reading one does not wait for the loads into another.
+struct Rings {
+    uint8_t* r[3];      // the third for an odd count of super-stages
+    uint8_t* corr;      // [steps][3][PIECE] the unit's correction operands
 };
 
-__device__ __forceinline__ TileInfo tile_at(const ExpertArgs& a, int t) {
-    const int2 tl = a.tiles[t];
-    const ExpertWork wk = a.work[tl.x];
-    TileInfo ti;
-    ti.slot0 = wk.s0 + tl.y * MT;
-    ti.nt = min(MT, wk.n - tl.y * MT);
-    ti.e = wk.e;
-    return ti;
-}
-
-// LDS layout of a block with contraction length K:
-//   q    the tile's token digits of one phase (kph columns): token i's plane
-//        p (0 hi, 1 lo) at q + (p * MT + i) * (kph + KPAD), in int8 operand
-//        order; kph + KPAD = 16 mod 256 bytes puts the 16 token rows of a
-//        ds_read_b128 half-wave in distinct banks
-//   s    the tokens' scales over all of K: group g, token i at s[g * MT + i]
-//   c    -8 times the tokens' group sums of 256 h + l, laid out as s
-//   tok  the tile's token (gate/up) or slot (down) rows, then its slot ids
-//        (gate/up) or routing weights (down)
-//   w    per wave, two super-stage buffers of its 32 weight rows (WRS bytes
-//        per row)
-struct Lay {
-    int kph;
-    size_t s, c, tok, w, total;
-    __host__ __device__ constexpr Lay(int K, int G)
-        : kph(K < KPH_MAX ? K : KPH_MAX),
-          s((size_t)2 * MT * ((K < KPH_MAX ? K : KPH_MAX) + KPAD)),
-          c(s + (size_t)(K / G) * MT * 4),
-          tok(c + (size_t)(K / G) * MT * 4),
-          w(tok + 2 * MT * 4),
-          total(tok + 2 * MT * 4 + (size_t)NWAVE * 2 * WBUF) {}
+// Where a wave's product's operands come from: K columns in nss super-stages,
+// two 32-row blocks of weight rows.
+struct Operands {
+    const uint8_t* recb;    // the tokens' records, at the first column (uniform)
+    uint32_t reco[2];       // the offsets of tokens 8 w + l / 16 and 8 w + 4 + l / 16 of the tile
+    const uint8_t* expb;    // their exponents, and the offset of token l % 32
+    uint32_t expo;
+    const uint8_t* w[2];    // each row block's first row's packed bytes, at the first column (uniform)
+    const uint8_t* sc[2];   // and its scales
+    uint32_t wrow, srow;    // bytes per packed row, per row of scales
+    int nss, ng;            // super-stages, groups
 };
 
-// Stage the tile's digit planes, columns [c0, c0 + kph), into q: token i's
-// rows are row src[i] of hi/lo [.][K].  All threads; no branches, so each
-// thread's loads of a batch are all in flight together (indices past the
-// end repeat the last piece, stored again to the same place).
-__device__ __forceinline__ void stage_phase(const int8_t* __restrict__ hi, const int8_t* __restrict__ lo,
-                                            const int* src, int K, int c0, int kph, int8_t* q) {
-    constexpr int BATCH = 8;
-    // an opaque thread index: the addresses below are recomputed at each
-    // staging instead of being kept live across the caller's main loop
-    int tid = threadIdx.x;
-    __asm__ volatile("" : "+v"(tid));
-    const int KP = kph + KPAD;
-    const int pieces = kph / 16;                  // 16-byte pieces per token row
-    const int total = 2 * MT * pieces;
-    // u / pieces as a multiply-high: exact for u * pieces < 2^32
-    const unsigned magic = 0xFFFFFFFFu / (unsigned)pieces + 1u;
-    for (int base = 0; base < total; base += MTHREADS * BATCH) {
-        uint4 v[BATCH];
-        int dst[BATCH];
-#pragma unroll
-        for (int j = 0; j < BATCH; j++) {
-            const unsigned u = (unsigned)min(base + j * MTHREADS + tid, total - 1);
-            const int r = (int)__umulhi(u, magic);                // plane * MT + token
-            const int pc = (int)u - r * pieces;
-            v[j] = *(const uint4*)((r >= MT ? lo : hi) + (size_t)src[r & (MT - 1)] * K + c0 + pc * 16);
-            dst[j] = r * KP + pc * 16;
-        }
-#pragma unroll
-        for (int j = 0; j < BATCH; j++) *(uint4*)(q + dst[j]) = v[j];
-    }
+// A value that is the same in every lane, as a scalar
+__device__ __forceinline__ int scalar(int v) { return __builtin_amdgcn_readfirstlane(v); }
+__device__ __forceinline__ unsigned long long scalar(unsigned long long v) {
+    return (unsigned long long)(uint32_t)scalar((int)(v >> 32)) << 32 | (uint32_t)scalar((int)v);
 }
 
-// The tile's token scales and group-sum corrections of ng groups (padding
-// tokens, i >= nt: 0); token row r's groups start at r * stride.
-__device__ __forceinline__ void stage_scales(const float* __restrict__ sc, const int* __restrict__ qc, const int* src,
-                                             int nt, int ng, int stride, float* s, int* c) {
-    for (int u = threadIdx.x; u < ng * MT; u += MTHREADS) {
-        const int g = u / MT, i = u % MT;
-        const size_t o = (size_t)src[i] * stride + g;
-        s[u] = i < nt ? sc[o] : 0.0f;
-        c[u] = i < nt ? -8 * qc[o] : 0;
-    }
+// A lane's address from a uniform base and a 32-bit lane offset, both opaque
+// to the optimiser: the base then stays in scalar registers and the load adds
+// them (hoisted out of the super-stage loop, or as its induction variables,
+// the lanes' 64-bit addresses take 40 vector registers and spill).
+__device__ __forceinline__ gptr<const uint8_t> lane_at(const uint8_t* p, uint32_t o) {
+    unsigned long long u = scalar((unsigned long long)p);
+    __asm__ volatile("" : "+s"(u), "+v"(o));
+    return (gptr<const uint8_t>)u + o;
 }
 
-// A wave's weight stream.  A super-stage is SSC columns of the wave's 32
-// rows: one 128-byte line per row, read as 4 coalesced loads per lane (load
-// k: lane L takes row 8 k + L / 8, bytes 16 (L % 8) of the line), then
-// written to the wave's own LDS buffer and read back per stage in the MFMA
-// layout (lane n % 32 its row).  Two super-stages are in flight.  With the
-// lines come this lane's row's scales of the super-stage's groups (4 stages
-// x 64 / G groups).
+template <typename T>
+__device__ __forceinline__ T load_as(gptr<const uint8_t> p) {
+    typedef uint32_t words __attribute__((ext_vector_type(sizeof(T) / 4)));
+    return __builtin_bit_cast(T, *(gptr<const words>)p);
+}
+
+// A wave's weights of one super-stage: w[row block][half line][16-row half].
+// Lane l of w[rb][u][b] holds row 16 b + l % 16, bytes 64 u + 16 (l / 16) ..
+// + 15 of the 128-byte line: 16 rows x 64 bytes per load.  Each half line is
+// requested for the next super-stage as soon as its registers are unpacked.
 template <int G>
-struct WStream {
-    static constexpr int NSC = 4 * 64 / G;        // scales per super-stage
+struct WStage {
+    static constexpr int NSC = SSC / G;           // scales per row
     typedef typename std::conditional<NSC == 4, uint2, uint4>::type ScT;
-    uint4 wb[2][4];                               // [0]: the next super-stage, [1]: the one after
-    ScT sc[2];
-    const uint8_t* wbase;                         // the wave's first row
-    const uint8_t* srow;                          // this lane's row's scales
-    size_t rowb;                                  // bytes per row
-    int nss;                                      // super-stages over K
-    __device__ __forceinline__ void load(int slot, int S) {
-        S = S < nss ? S : nss - 1;
-        const int L = threadIdx.x & 63;
+    typedef typename std::conditional<NSC == 4, uint32_t, uint2>::type ExT;
+    uint4 w[2][2][2];
+    ScT sc[2];                                    // row l % 32's scales
+    ExT ex;                                       // token l % 32's exponents
+    __device__ __forceinline__ void load_half(const Operands& op, int S, int u) {
+        const int l = threadIdx.x & 63;
 #pragma unroll
-        for (int k = 0; k < 4; k++)
-            wb[slot][k] = *(const uint4*)(wbase + (size_t)(8 * k + L / 8) * rowb + (size_t)S * (SSC / 2) + 16 * (L % 8));
-        sc[slot] = *(const ScT*)(srow + (size_t)S * NSC * 2);
+        for (int rb = 0; rb < 2; rb++) {
+            const uint32_t o = (uint32_t)(l & 15) * op.wrow + 16 * (l >> 4);
+#pragma unroll
+            for (int b = 0; b < 2; b++)
+                w[rb][u][b] = load_as<uint4>(
+                    lane_at(op.w[rb] + (size_t)S * (SSC / 2) + (size_t)b * 16 * op.wrow, o) + 64 * u);
+        }
     }
-    // write the next super-stage's lines to LDS buffer wl and return its
-    // scales; the one after moves up and super-stage S is requested behind it
-    __device__ __forceinline__ ScT advance(uint8_t* wl, int S) {
-        const int L = threadIdx.x & 63;
+    __device__ __forceinline__ void load_scales(const Operands& op, int S) {
+        const int l = threadIdx.x & 63;
 #pragma unroll
-        for (int k = 0; k < 4; k++) *(uint4*)(wl + (8 * k + L / 8) * WRS + 16 * (L % 8)) = wb[0][k];
-        const ScT r = sc[0];
-#pragma unroll
-        for (int k = 0; k < 4; k++) wb[0][k] = wb[1][k];
-        sc[0] = sc[1];
-        load(1, S);
-        return r;
+        for (int rb = 0; rb < 2; rb++)
+            sc[rb] = load_as<ScT>(lane_at(op.sc[rb] + (size_t)S * NSC * 2, (uint32_t)(l & 31) * op.srow));
+        ex = load_as<ExT>(lane_at(op.expb + S * NSC, op.expo));
     }
 };
 
 // scale u (0..NSC-1) of a super-stage's packed fp16 scales, as float
 template <int G>
-__device__ __forceinline__ float sc_at(const typename WStream<G>::ScT& v, int u) {
+__device__ __forceinline__ float sc_at(const typename WStage<G>::ScT& v, int u) {
     uint32_t w;
     if (G == 64) w = u < 2 ? ((const uint2&)v).x : ((const uint2&)v).y;
     else w = u < 2 ? ((const uint4&)v).x : u < 4 ? ((const uint4&)v).y : u < 6 ? ((const uint4&)v).z : ((const uint4&)v).w;
     return fp16_hw((uint16_t)(w >> (16 * (u & 1))));
 }
 
-// A wave's token operands of one stage: both sub-steps, both digit planes.
-// Stage columns (relative to the token phase) start at c; lane half h.
-//   G = 64: one group; sub-step u takes values 32 h + 16 u + 0..15.
-//   G = 32: two groups; sub-step u (= group u) takes values 32 u + 16 h + 0..15.
-struct AOps {
-    int4v ah0, ah1, al0, al1;
-};
-
-template <int G>
-__device__ __forceinline__ AOps load_aops(const int8_t* qh, const int8_t* ql, int c, int h) {
-    const int o0 = G == 64 ? c + 32 * h : c + 16 * h;
-    const int o1 = G == 64 ? o0 + 16 : o0 + 32;
-    return AOps{*(const int4v*)(qh + o0), *(const int4v*)(qh + o1), *(const int4v*)(ql + o0),
-                *(const int4v*)(ql + o1)};
-}
-
-// The weight operands of one stage from the wave's LDS buffer (row n, lane
-// half h), as int8 (q - 8): sub-step 0 and 1 (see AOps).
-template <int G>
-__device__ __forceinline__ void load_bops(const uint8_t* wl, int n, int h, int cs, int4v& b0, int4v& b1) {
-    const uint8_t* r = wl + n * WRS + 32 * cs;
-    if (G == 64) {
-        const uint4 w = *(const uint4*)(r + 16 * h);
-        b0 = wdigits(w.x, w.y);
-        b1 = wdigits(w.z, w.w);
-    } else {
-        const uint2 w0 = *(const uint2*)(r + 8 * h), w1 = *(const uint2*)(r + 16 + 8 * h);
-        b0 = wdigits(w0.x, w0.y);
-        b1 = wdigits(w1.x, w1.y);
+// This wave's 8 tokens' records of super-stage S to the ring buffer: 768
+// bytes each as three 256-byte groups, a load 4 tokens x 256 bytes (lane l:
+// token l / 16).  [group][token][16 chunks of 16 bytes], chunk c of token i at
+// c ^ (i % 16): a stage's reads, the same chunk of 32 tokens, fall in
+// different banks.
+__device__ __forceinline__ void stage_tokens(const Operands& op, int S, uint8_t* ring) {
+    const int w = scalar((int)(threadIdx.x >> 6)), l = threadIdx.x & 63;
+#pragma unroll
+    for (int q = 0; q < 2; q++) {
+        const uint32_t i = 8 * w + 4 * q + (l >> 4);
+        const gptr<const uint8_t> src = lane_at(op.recb + (size_t)S * (4 * F6_STAGE), op.reco[q] + 16 * ((l ^ i) & 15));
+#pragma unroll
+        for (int g = 0; g < 3; g++)
+            __builtin_amdgcn_global_load_lds((gptr<void>)(src + 256 * g),
+                                             (__attribute__((address_space(3))) void*)(ring + (32 * g + 8 * w + 4 * q) * 256), 16, 0, 0);
     }
 }
 
-// The 16 tokens' scales of one group (this lane's half h)
-struct SxOps {
-    float4 s[4];
-};
-
-__device__ __forceinline__ SxOps load_sx(const float* s, int g, int h) {
-    const float* sg = s + (size_t)g * MT + 4 * h;
-    return SxOps{{*(const float4*)(sg), *(const float4*)(sg + 8), *(const float4*)(sg + 16),
-                  *(const float4*)(sg + 24)}};
-}
-
-// The 16 tokens' corrections of one group (this lane's half h), in the
-// accumulator layout: register v holds token 8 (v / 4) + 4 h + v % 4.
-__device__ __forceinline__ int16v load_corr(const int* c, int g, int h) {
-    const int* cg = c + (size_t)g * MT + 4 * h;
-    const int8v a = __builtin_shufflevector(*(const int4v*)cg, *(const int4v*)(cg + 8), 0, 1, 2, 3, 4, 5, 6, 7);
-    const int8v b = __builtin_shufflevector(*(const int4v*)(cg + 16), *(const int4v*)(cg + 24), 0, 1, 2, 3, 4, 5, 6, 7);
-    return __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7, 8, 9, 10, 11, 12, 13, 14, 15);
-}
-
-// The integer products of one stage: per group of the stage, hi and lo
-// digit planes.  The lo products accumulate onto o.il, which the caller sets
-// to the group's corrections: with unsigned nibbles q, 256 ih + il is then
-// the exact sum of (256 h + l) (q - 8).
-template <int G>
-struct IOps {
-    int16v ih[64 / G], il[64 / G];
-};
-
-template <int G>
-__device__ __forceinline__ void stage_mfma(IOps<G>& o, const AOps& a, const int4v& b0, const int4v& b1) {
-    if (G == 64) {
-        o.ih[0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a.ah0, b0, int16v{}, 0, 0, 0);
-        o.il[0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a.al0, b0, o.il[0], 0, 0, 0);
-        o.ih[0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a.ah1, b1, o.ih[0], 0, 0, 0);
-        o.il[0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a.al1, b1, o.il[0], 0, 0, 0);
-    } else {
-        o.ih[0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a.ah0, b0, int16v{}, 0, 0, 0);
-        o.il[0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a.al0, b0, o.il[0], 0, 0, 0);
-        o.ih[G == 64 ? 0 : 1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a.ah1, b1, int16v{}, 0, 0, 0);
-        o.il[G == 64 ? 0 : 1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a.al1, b1, o.il[G == 64 ? 0 : 1], 0, 0, 0);
-    }
-}
-
-// acc += 256 * ih + il of one group, times each token's scale, times the
-// row's scale
-__device__ __forceinline__ void group_acc(floatx16& acc, const int16v& ih, const int16v& il, const SxOps& sx,
-                                          float ws) {
+// The unit's group corrections on their way to LDS (three bf16 terms each, in
+// the operand order of the correction product): wave w holds steps w, w + 4,
+// ... of 16 groups, lane l groups 16 st + 8 (l / 32) .. + 7 of token l % 32.
+template <int CSTEPS>
+struct CorrTok {
+    static_assert(CSTEPS <= NWAVE, "a step per wave");
+    float4 c[2];
+    __device__ __forceinline__ void load(const float* corr, int ng) {
+        const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
 #pragma unroll
-    for (int k = 0; k < 4; k++) {
-        const float sv[4] = {sx.s[k].x, sx.s[k].y, sx.s[k].z, sx.s[k].w};
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const int v = 4 * k + j;
-            const int iv = ih[v] * 256 + il[v];
-            acc[v] = __builtin_fmaf(__fmul_rn((float)iv, sv[j]), ws, acc[v]);
+        for (int q = 0; q < 2; q++) {
+            const int g = 16 * w + 8 * (l >> 5) + 4 * q;
+            c[q] = *(const float4*)(corr + (g < ng ? g : 0));
         }
     }
-}
-
-// Where a block's token digits come from, for the phase restaging.
-struct TokSrc {
-    const int8_t* hi;
-    const int8_t* lo;
-    const int* rows;
-    int K;
-};
-
-// The contraction of one wave: its 32 weight rows (lane n = l % 32 holds
-// row n) against the tile's 32 tokens over K columns, into acc.  The token
-// digits of the first phase and all the scales are in LDS, and the weight
-// stream's first two super-stages are in flight.  Stage c's token operands
-// are read one stage ahead; for G = 64 stage c's MFMAs are issued before
-// stage c - 1's scale epilogue (products alternate by stage parity), so
-// each wave has independent MFMA and VALU work at every point.  At each
-// token phase boundary the block restages the tokens (two barriers).
-template <int G, bool AHEAD = true>
-__device__ __forceinline__ void wave_product(floatx16& acc, WStream<G>& ws, uint8_t* wl, int8_t* q,
-                                             const float* s, const int* cc, const TokSrc& ts, const Lay& ly) {
-    constexpr int NG = 64 / G;                    // groups per stage
-    constexpr bool PIPE = G == 64;
-    const int lane = threadIdx.x & 63;
-    const int n = lane & 31, h = lane >> 5;
-    const int KP = ly.kph + KPAD;
-    const int8_t* qh = q + (size_t)n * KP;
-    const int8_t* ql = q + (size_t)(MT + n) * KP;
-    const int sspp = ly.kph / SSC;                // super-stages per token phase
-    const int nss = ws.nss;
-    AOps ab[2];
-    IOps<G> pr[PIPE ? 2 : 1];
-    float wsp[PIPE ? 2 : 1][NG];
-    // AHEAD (G = 64): the next stage's weight operands (within a
-    // super-stage) and this stage's token scales (for the epilogue of the
-    // stage before) are requested one stage ahead, so that the stage's
-    // MFMAs and epilogue wait on no LDS read of their own stage
-    int4v bn0, bn1;
-    SxOps sxn;
-    const int nph = (nss + sspp - 1) / sspp;
-#pragma unroll 1
-    for (int ph = 0; ph < nph; ph++) {
-      if (ph > 0) {
-        __syncthreads();                          // every wave is done with the previous phase
-        stage_phase(ts.hi, ts.lo, ts.rows, ts.K, ph * ly.kph, ly.kph, q);
-        __syncthreads();
-      }
-      const int s_end = min(nss, (ph + 1) * sspp);
-#pragma unroll 1
-      for (int S = ph * sspp; S < s_end; S++) {
-        const bool pstart = S % sspp == 0, pend = S + 1 == s_end;
-        uint8_t* wbuf = wl + (S & 1) * WBUF;
-        const typename WStream<G>::ScT scs = ws.advance(wbuf, S + 2);
-        const int cp = (S % sspp) * SSC;          // the super-stage's first column within the phase
-        if (PIPE && pstart) ab[0] = load_aops<G>(qh, ql, cp, h);
-        if (PIPE && AHEAD) load_bops<G>(wbuf, n, h, 0, bn0, bn1);
+    __device__ __forceinline__ void store(int ng, uint8_t* cl) const {
+        const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
+        if (16 * w >= ng) return;
+        uint32_t t[3][4];
 #pragma unroll
-        for (int cs = 0; cs < 4; cs++) {
-            __builtin_amdgcn_sched_barrier(0);
-            const int c = 4 * S + cs;             // stage index over K
-            const int cur = cs & 1, prv = cur ^ 1;
-            const int pc = PIPE ? cur : 0, pp = PIPE ? prv : 0;
-            if (PIPE && !AHEAD) {
-                if (!(cs == 3 && pend)) ab[prv] = load_aops<G>(qh, ql, cp + 64 * (cs + 1), h);
-                SxOps sxp;
-                if (c > 0) sxp = load_sx(s, c - 1, h);
-                int4v b0, b1;
-                load_bops<G>(wbuf, n, h, cs, b0, b1);
-                pr[pc].il[0] = load_corr(cc, c, h);
-                stage_mfma<G>(pr[pc], ab[cur], b0, b1);
-                wsp[pc][0] = sc_at<G>(scs, cs);
-                if (c > 0) group_acc(acc, pr[pp].ih[0], pr[pp].il[0], sxp, wsp[pp][0]);
-            } else if (PIPE) {
-                const int4v b0 = bn0, b1 = bn1;
-                pr[pc].il[0] = load_corr(cc, c, h);
-                const SxOps sxp = sxn;
-                // requests for the next stage
-                if (!(cs == 3 && pend)) ab[prv] = load_aops<G>(qh, ql, cp + 64 * (cs + 1), h);
-                if (cs < 3) load_bops<G>(wbuf, n, h, cs + 1, bn0, bn1);
-                sxn = load_sx(s, c, h);
-                stage_mfma<G>(pr[pc], ab[cur], b0, b1);
-                wsp[pc][0] = sc_at<G>(scs, cs);
-                if (c > 0) group_acc(acc, pr[pp].ih[0], pr[pp].il[0], sxp, wsp[pp][0]);
-            } else {
-                ab[cur] = load_aops<G>(qh, ql, cp + 64 * cs, h);
-                int4v b0, b1;
-                load_bops<G>(wbuf, n, h, cs, b0, b1);
+        for (int q = 0; q < 2; q++) {
+            const bool in = 16 * w + 8 * (l >> 5) + 4 * q < ng;
+            const float v[4] = {in ? c[q].x : 0.0f, in ? c[q].y : 0.0f, in ? c[q].z : 0.0f, in ? c[q].w : 0.0f};
 #pragma unroll
-                for (int u = 0; u < NG; u++) pr[0].il[u] = load_corr(cc, NG * c + u, h);
-                stage_mfma<G>(pr[0], ab[cur], b0, b1);
-#pragma unroll
-                for (int u = 0; u < NG; u++) wsp[0][u] = sc_at<G>(scs, NG * cs + u);
-#pragma unroll
-                for (int u = 0; u < NG; u++)
-                    group_acc(acc, pr[0].ih[u], pr[0].il[u], load_sx(s, NG * c + u, h), wsp[0][u]);
+            for (int e = 0; e < 2; e++) {
+                const float a = v[2 * e], b = v[2 * e + 1];
+                uint32_t hi, lo;
+                split_bf16x2(a, b, hi, lo);
+                t[0][2 * q + e] = hi;
+                t[1][2 * q + e] = lo;
+                t[2][2 * q + e] = pack_bf16x2(
+                    __fsub_rn(__fsub_rn(a, __uint_as_float(hi << 16)), __uint_as_float(lo << 16)),
+                    __fsub_rn(__fsub_rn(b, __uint_as_float(hi & 0xFFFF0000u)), __uint_as_float(lo & 0xFFFF0000u)));
             }
         }
-      }
+#pragma unroll
+        for (int k = 0; k < 3; k++)
+            *(uint4*)(cl + (3 * w + k) * PIECE + 16 * l) = make_uint4(t[k][0], t[k][1], t[k][2], t[k][3]);
     }
-    if (PIPE) {
-        // the last stage's epilogue (stage 4 nss - 1 is odd: its products sit in buffer 1)
-        group_acc(acc, pr[PIPE ? 1 : 0].ih[0], pr[PIPE ? 1 : 0].il[0], AHEAD ? sxn : load_sx(s, 4 * nss - 1, h),
-                  wsp[PIPE ? 1 : 0][0]);
+};
+
+// The row scales of one row block for the correction product: lane l groups
+// 16 st + 8 (l / 32) .. + 7 of row l % 32, steps st of 16 groups.
+template <int CSTEPS>
+struct CorrScales {
+    uint2 v[CSTEPS][2];
+    __device__ __forceinline__ void load(const Operands& op, const uint8_t* sc) {
+        const int l = threadIdx.x & 63;
+#pragma unroll
+        for (int st = 0; st < CSTEPS; st++)
+#pragma unroll
+            for (int q = 0; q < 2; q++) {
+                const int g = 16 * st + 8 * (l >> 5) + 4 * q;
+                v[st][q] = load_as<uint2>(lane_at(sc, (uint32_t)(l & 31) * op.srow + 2 * (g < op.ng ? g : 0)));
+            }
     }
+};
+
+// acc += sum over the groups of correction x row scale
+template <int CSTEPS>
+__device__ __forceinline__ void add_corr(floatx16& acc, const Operands& op, const CorrScales<CSTEPS>& sc, const uint8_t* cl) {
+    const int l = threadIdx.x & 63, h = l >> 5;
+#pragma unroll
+    for (int st = 0; st < CSTEPS; st++) {
+        if (16 * st >= op.ng) break;
+        uint32_t hi[4], lo[4];
+#pragma unroll
+        for (int q = 0; q < 2; q++) {
+            const bool in = 16 * st + 8 * h + 4 * q < op.ng;
+            const uint32_t x = in ? sc.v[st][q].x : 0u, y = in ? sc.v[st][q].y : 0u;
+            split_bf16x2(fp16_hw((uint16_t)x), fp16_hw((uint16_t)(x >> 16)), hi[2 * q], lo[2 * q]);
+            split_bf16x2(fp16_hw((uint16_t)y), fp16_hw((uint16_t)(y >> 16)), hi[2 * q + 1], lo[2 * q + 1]);
+        }
+        const bf16x8 wh = __builtin_bit_cast(bf16x8, make_uint4(hi[0], hi[1], hi[2], hi[3]));
+        const bf16x8 wl = __builtin_bit_cast(bf16x8, make_uint4(lo[0], lo[1], lo[2], lo[3]));
+        const bf16x8 c0 = __builtin_bit_cast(bf16x8, *(const uint4*)(cl + (3 * st + 0) * PIECE + 16 * l));
+        const bf16x8 c1 = __builtin_bit_cast(bf16x8, *(const uint4*)(cl + (3 * st + 1) * PIECE + 16 * l));
+        const bf16x8 c2 = __builtin_bit_cast(bf16x8, *(const uint4*)(cl + (3 * st + 2) * PIECE + 16 * l));
+        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(c2, wh, acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(c1, wl, acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(c1, wh, acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(c0, wl, acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(c0, wh, acc, 0, 0, 0);
+    }
+}
+
+// Two dwords of each of the 4 sixteen-lane rows exchanged: x = rows (x0, x1,
+// x2, x3), y likewise -> (x0, y0, x2, y2) and (x1, y1, x3, y3)
+__device__ __forceinline__ void swap16(uint32_t& x, uint32_t& y) {
+    const auto p = __builtin_amdgcn_permlane16_swap(x, y, false, false);
+    x = p[0];
+    y = p[1];
+}
+// -> (x0, x1, y0, y1) and (x2, x3, y2, y3)
+__device__ __forceinline__ void swap32(uint32_t& x, uint32_t& y) {
+    const auto p = __builtin_amdgcn_permlane32_swap(x, y, false, false);
+    x = p[0];
+    y = p[1];
+}
+
+__device__ __forceinline__ int8v f6_operand(const uint32_t (&d)[4]) {
+    uint32_t f[6];
+    f6_spread(d[0], d[1], f[0], f[1], f[2]);
+    f6_spread(d[2], d[3], f[3], f[4], f[5]);
+    return int8v{(int)f[0], (int)f[1], (int)f[2], (int)f[3], (int)f[4], (int)f[5], 0, 0};
+}
+
+// The weight operands of one row block from half a line (64 bytes: two
+// stages) of each row.  G = 64: both stages', b[stage].  G = 32: stage S's two
+// groups, b[group], each group's 32 columns in both lane halves.
+template <int G, int S>
+__device__ __forceinline__ void load_bops(const uint4 (&w)[2], int8v (&b)[2]) {
+    const uint32_t x[4] = {w[0].x, w[0].y, w[0].z, w[0].w}, y[4] = {w[1].x, w[1].y, w[1].z, w[1].w};
+    uint32_t d0[4], d1[4];
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        uint32_t p = x[k], q = y[k];
+        swap16(p, q);                             // p: chunks 0, 2 of rows 0..15, 16..31; q: chunks 1, 3
+        if (G == 64) {
+            swap32(p, q);                         // chunks (0, 1) and (2, 3) in the lane halves
+            d0[k] = p;
+            d1[k] = q;
+        } else {
+            uint32_t p2 = p, q2 = q;
+            swap32(p, p2);                        // chunk 0 and chunk 2 in both halves
+            swap32(q, q2);                        // chunk 1 and chunk 3
+            d0[k] = S ? p2 : p;
+            d1[k] = S ? q2 : q;
+        }
+    }
+    b[0] = f6_operand(d0);
+    b[1] = f6_operand(d1);
+}
+
+// P (+)= A . B with the token exponent in byte SA of sa and the plane's
+// scale in byte SB of sb
+template <int SA, int SB>
+__device__ __forceinline__ floatx16 mfma_f6(const int8v& a, const int8v& b, const floatx16& c, uint32_t sa, uint32_t sb) {
+    return __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a, b, c, 2, 2, SA, (int)sa, SB, (int)sb);
+}
+
+// One stage's products: P[rb][group] from the stage's token operands in LDS
+template <int G, int CS>
+__device__ __forceinline__ void stage_mfma(floatx16 (&P)[2][64 / G], const uint8_t* ring, const int8v (&b)[2][64 / G],
+                                           const typename WStage<G>::ExT& ex, uint32_t sb) {
+    // piece k, half h: chunk 12 CS + 2 k + h of token l % 32 (opaque: the
+    // addresses are made here instead of being kept in registers)
+    const int l = threadIdx.x & 63;
+    uint32_t at = (l & 31) * 256 + 16 * ((l >> 5) ^ (l & 15));
+    __asm__ volatile("" : "+v"(at));
+    uint4 p[6];
+#pragma unroll
+    for (int k = 0; k < 6; k++) {
+        const int c = 12 * CS + 2 * k;
+        p[k] = *(const uint4*)(ring + (c >> 4) * (32 * 256) + (at ^ (16 * (c & 15))));
+    }
+    const int8v a0 = {(int)p[0].x, (int)p[0].y, (int)p[0].z, (int)p[0].w, (int)p[4].x, (int)p[4].y, 0, 0};
+    const int8v a1 = {(int)p[1].x, (int)p[1].y, (int)p[1].z, (int)p[1].w, (int)p[4].z, (int)p[4].w, 0, 0};
+    const int8v a2 = {(int)p[2].x, (int)p[2].y, (int)p[2].z, (int)p[2].w, (int)p[5].x, (int)p[5].y, 0, 0};
+    const int8v a3 = {(int)p[3].x, (int)p[3].y, (int)p[3].z, (int)p[3].w, (int)p[5].z, (int)p[5].w, 0, 0};
+    if constexpr (G == 64) {
+#pragma unroll
+        for (int rb = 0; rb < 2; rb++) P[rb][0] = mfma_f6<CS, 0>(a0, b[rb][0], floatx16{}, ex, sb);
+#pragma unroll
+        for (int rb = 0; rb < 2; rb++) P[rb][0] = mfma_f6<CS, 1>(a1, b[rb][0], P[rb][0], ex, sb);
+#pragma unroll
+        for (int rb = 0; rb < 2; rb++) P[rb][0] = mfma_f6<CS, 2>(a2, b[rb][0], P[rb][0], ex, sb);
+#pragma unroll
+        for (int rb = 0; rb < 2; rb++) P[rb][0] = mfma_f6<CS, 3>(a3, b[rb][0], P[rb][0], ex, sb);
+    } else {
+        const uint32_t e = CS < 2 ? ex.x : ex.y;
+        constexpr int B0 = 2 * (CS & 1);
+#pragma unroll
+        for (int rb = 0; rb < 2; rb++) {
+            P[rb][0] = mfma_f6<B0, 0>(a0, b[rb][0], floatx16{}, e, sb);
+            P[rb][1] = mfma_f6<B0 + 1, 0>(a2, b[rb][1], floatx16{}, e, sb);
+        }
+#pragma unroll
+        for (int rb = 0; rb < 2; rb++) {
+            P[rb][0] = mfma_f6<B0, 1>(a1, b[rb][0], P[rb][0], e, sb);
+            P[rb][1] = mfma_f6<B0 + 1, 1>(a3, b[rb][1], P[rb][1], e, sb);
+        }
+    }
+}
+
+__device__ __forceinline__ void group_acc(floatx16& acc, const floatx16& P, float ws) {
+#pragma unroll
+    for (int v = 0; v < 16; v++) acc[v] = __builtin_fmaf(P[v], ws, acc[v]);
+}
+
+// What acc depends on comes before what follows in the source (else the
+// operands of later stages are read first, into registers there are not).
+__device__ __forceinline__ void pin(floatx16 (&acc)[2]) {
+    __asm__ volatile("" : "+v"(acc[0]), "+v"(acc[1]) : : "memory");
+}
+
+// 16-group steps of the correction product: of 256 or 768 columns for one or
+// three super-stages, else of up to KMAX
+constexpr int corr_steps(int G, int nss) { return ((nss ? nss * SSC : KMAX) / G + 15) / 16; }
+
+// A wave's running state over a block's units (a unit: one token tile against
+// the block's rows): the operands of the unit being computed and the next
+// super-stage's weights.
+template <int G, int NSS>
+struct Pipe {
+    using W = WStage<G>;
+    static constexpr int NG = 64 / G;
+    static constexpr int CSTEPS = corr_steps(G, NSS);
+    // the correction's scales are kept from the unit before, or (more than
+    // the registers hold) read when they are needed
+    static constexpr bool CS_AHEAD = CSTEPS <= 2;
+    W w;
+    floatx16 acc[2];
+    CorrScales<CSTEPS> cs[2];
+    CorrTok<CSTEPS> ct;
+
+    // the next unit's corrections on their way
+    __device__ __forceinline__ void next_corr(const Operands& op, const float* corr) {
+        if constexpr (CS_AHEAD) {
+#pragma unroll
+            for (int rb = 0; rb < 2; rb++) cs[rb].load(op, op.sc[rb]);
+        }
+        ct.load(corr, op.ng);
+    }
+
+    // the first unit's operands
+    __device__ __forceinline__ void start(const Operands& op, const Rings& rg, const float* corr) {
+        next_corr(op, corr);
+        stage_tokens(op, 0, rg.r[0]);
+        w.load_half(op, 0, 0);
+        w.load_half(op, 0, 1);
+        w.load_scales(op, 0);
+        ct.store(op.ng, rg.corr);
+    }
+
+    // Super-stage S from `ring`; the next one's operands (nop's super-stage
+    // nS) are requested into nring and the weight registers.  hook() runs
+    // once every wave's operands of S are there.
+    template <class Hook>
+    __device__ __forceinline__ void step(const uint8_t* ring, uint8_t* nring, Hook&& hook) {
+        const uint32_t h = (threadIdx.x >> 5) & 1;
+        // the planes' scales: 2^6 for the two operands' eighths, times 16^plane
+        const uint32_t sb = G == 64 ? 0x918D8985u : h ? 0x9189u : 0x8D85u;
+        // this super-stage's tokens and weights have arrived (waited for by
+        // count the tokens alone would do, but the compiler then waits for
+        // the next ones' loads to LDS before it takes the weights; and the
+        // block barrier does not wait for loads to LDS), and every wave is
+        // done with the one before, whose buffer may be filled again
+        __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_waitcnt(0x0070);       // vmcnt(0), lgkmcnt(0)
+        wave_meet();
+        int nS;
+        const Operands nop = hook(nS);
+        if (nring) stage_tokens(nop, nS, nring);
+        __builtin_amdgcn_sched_barrier(0);
+        const typename W::ScT sc[2] = {w.sc[0], w.sc[1]};
+        const typename W::ExT ex = w.ex;
+        auto stage = [&](auto cs_, const int8v (&b)[2][NG]) __attribute__((always_inline)) {
+            constexpr int CS = decltype(cs_)::value;
+            floatx16 P[2][NG];
+            stage_mfma<G, CS>(P, ring, b, ex, sb);
+#pragma unroll
+            for (int rb = 0; rb < 2; rb++)
+#pragma unroll
+                for (int g = 0; g < NG; g++) group_acc(acc[rb], P[rb][g], sc_at<G>(sc[rb], NG * CS + g));
+        };
+        auto half = [&](auto u) __attribute__((always_inline)) {
+            constexpr int U = decltype(u)::value;
+            if constexpr (G == 64) {
+                int8v t0[2], t1[2];
+                load_bops<G, 0>(w.w[0][U], t0);
+                load_bops<G, 0>(w.w[1][U], t1);
+                __builtin_amdgcn_sched_barrier(0);
+                w.load_half(nop, nS, U);
+                if (U == 1) w.load_scales(nop, nS);
+                __builtin_amdgcn_sched_barrier(0);
+                const int8v b0[2][NG] = {{t0[0]}, {t1[0]}}, b1[2][NG] = {{t0[1]}, {t1[1]}};
+                stage(std::integral_constant<int, 2 * U>{}, b0);
+                stage(std::integral_constant<int, 2 * U + 1>{}, b1);
+                pin(acc);
+            } else {
+                int8v b[2][NG];
+                load_bops<G, 0>(w.w[0][U], b[0]);
+                load_bops<G, 0>(w.w[1][U], b[1]);
+                stage(std::integral_constant<int, 2 * U>{}, b);
+                pin(acc);                     // (one stage's operands at a time: registers)
+                load_bops<G, 1>(w.w[0][U], b[0]);
+                load_bops<G, 1>(w.w[1][U], b[1]);
+                __builtin_amdgcn_sched_barrier(0);
+                w.load_half(nop, nS, U);
+                if (U == 1) w.load_scales(nop, nS);
+                __builtin_amdgcn_sched_barrier(0);
+                stage(std::integral_constant<int, 2 * U + 1>{}, b);
+                pin(acc);
+            }
+        };
+        half(std::integral_constant<int, 0>{});
+        half(std::integral_constant<int, 1>{});
+    }
+
+    // The unit's super-stages (NSS 0: an even count, or 1 or 3), then the next
+    // unit's first operands on their way.  early() runs in the first
+    // super-stage, late(nop) in the second (in the only one, after early's
+    // loads): they find the next unit and fill in its operands.
+    template <class Early, class Late>
+    __device__ __forceinline__ void unit(const Operands& op, Operands& nop, const Rings& rg, Early&& early, Late&& late) {
+        auto first = [&]() __attribute__((always_inline)) {
+#pragma unroll
+            for (int rb = 0; rb < 2; rb++) {
+                if constexpr (!CS_AHEAD) cs[rb].load(op, op.sc[rb]);
+                acc[rb] = floatx16{};
+                add_corr(acc[rb], op, cs[rb], rg.corr);
+            }
+            early();
+        };
+        if constexpr (NSS == 1) {
+            step(rg.r[0], nullptr, [&](int& nS) __attribute__((always_inline)) -> Operands {
+                first();
+                late(nop);
+                nS = 0;
+                return nop;
+            });
+            wave_meet();                      // every wave is done with the only buffer
+            stage_tokens(nop, 0, rg.r[0]);
+        } else if constexpr (NSS == 3) {
+            step(rg.r[0], rg.r[1], [&](int& nS) __attribute__((always_inline)) -> Operands { first(); nS = 1; return op; });
+            step(rg.r[1], rg.r[2], [&](int& nS) __attribute__((always_inline)) -> Operands { late(nop); nS = 2; return op; });
+            step(rg.r[2], rg.r[0], [&](int& nS) __attribute__((always_inline)) -> Operands { nS = 0; return nop; });
+        } else {
+#pragma unroll 1
+            for (int S = 0; S < op.nss; S += 2) {
+                step(rg.r[0], rg.r[1], [&](int& nS) __attribute__((always_inline)) -> Operands {
+                    if (S == 0) first();
+                    nS = S + 1;
+                    return op;
+                });
+                const bool last = S + 2 == op.nss;
+                step(rg.r[1], rg.r[0], [&](int& nS) __attribute__((always_inline)) -> Operands {
+                    if (S == 0) late(nop);
+                    nS = last ? 0 : S + 2;
+                    return last ? nop : op;
+                });
+            }
+        }
+    }
+};
+
+// The kernels' blocks stay for several units: unit u of the grid's gridDim.x
+// blocks is tile u / nrb, row block u % nrb, then u + gridDim.x; past the
+// tiles' units come the small experts' items.  A tile's entry, its slots and
+// its first operands are requested during the unit before, so that only the
+// block's first unit waits for that chain of loads.
+__device__ __forceinline__ int4 tile_at(const ExpertArgs& a, int t) {
+    const int4 ti = a.tiles[t];
+    return make_int4(scalar(ti.x), scalar(ti.y), scalar(ti.z), 0);
+}
+
+// this lane's slot of a tile: token l % 32 (padding: the first)
+__device__ __forceinline__ int tile_slot(const ExpertArgs& a, const int4& ti) {
+    const int i = threadIdx.x & 31;
+    return a.seg_slot[ti.y + (i < ti.z ? i : 0)];
+}
+
+// rows: the tokens' row of lane l % 32, K columns
+template <int G>
+__device__ __forceinline__ void set_tokens(Operands& op, const uint8_t* rec, const uint8_t* exps, int row, int K) {
+    const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
+    op.recb = rec;                                // (below 4 GB: at most JM_MAX_SLOTS rows of KMAX columns)
+#pragma unroll
+    for (int q = 0; q < 2; q++) op.reco[q] = (uint32_t)f6_rec_bytes(__shfl(row, 8 * w + 4 * q + (l >> 4), JM_WAVE), K);
+    op.expb = exps;
+    op.expo = (uint32_t)row * (K / G);
+    op.wrow = K / 2;
+    op.srow = K / G * 2;
+    op.nss = K / SSC;
+    op.ng = K / G;
 }
 
 // ------------------------------------------------------------------ gate/up
 
 template <int G>
-__device__ __forceinline__ void gateup_tile(const ExpertArgs& a, const TileInfo& ti, int rblk, unsigned char* sm) {
-    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-    const int d = a.d, m = a.m, ng = d / G;
-    const Lay ly(d, G);
-    const int mat = w & 1, rq = w >> 1;           // this wave: gate (0) or up (1), rows 32 rq .. 32 rq + 31
-    const int r0 = rblk * GU_ROWS;                // the block's first intermediate row
-    int8_t* q = (int8_t*)sm;
-    float* s = (float*)(sm + ly.s);
-    int* cc = (int*)(sm + ly.c);
-    int* tok = (int*)(sm + ly.tok);
-    uint8_t* wl = sm + ly.w + (size_t)w * 2 * WBUF;
-    int* slots = tok + MT;
-    if (tid < MT) {
-        const int sl = a.seg_slot[ti.slot0 + (tid < ti.nt ? tid : 0)];   // padding: the first slot
-        slots[tid] = sl;
-        tok[tid] = sl / a.topk;
-    }
-    unsigned long long so, po;
-    a.rec.get(mat, a.key0 + ti.e, so, po);
-    const int n = lane & 31;
-    const int wrow0 = r0 + 32 * rq;               // the wave's first row
-    WStream<G> ws;
-    ws.wbase = a.blob + po + (size_t)wrow0 * (d / 2);
-    ws.srow = a.blob + so + (size_t)(wrow0 + n) * ng * 2;
-    ws.rowb = d / 2;
-    ws.nss = d / SSC;
-    ws.load(0, 0);
-    ws.load(1, 1);
-    __syncthreads();
-    stage_phase(a.xqh, a.xql, tok, d, 0, ly.kph, q);
-    stage_scales(a.xqs, a.xqc, tok, ti.nt, ng, ng, s, cc);
-    __syncthreads();
-    floatx16 acc = {};
-    wave_product<G>(acc, ws, wl, q, s, cc, TokSrc{a.xqh, a.xql, tok, d}, ly);
-
-    // SwiGLU: both matrices' sums to LDS (over the token digits), then one
-    // wave per (token, 64-row piece) forms act, its digits and scale
-    __syncthreads();
-    const int h = lane >> 5;
-    constexpr int RP = GU_ROWS + 4;               // padded LDS row of one token's sums
-    float* gu = (float*)sm;                       // [2][MT][RP]
+__device__ __forceinline__ void gateup_op(Operands& op, const ExpertArgs& a, const int4& ti, int rblk, int sl) {
+    const int w = scalar((int)(threadIdx.x >> 6));
+    set_tokens<G>(op, a.xq, a.xe, sl / a.topk, a.d);
 #pragma unroll
-    for (int v = 0; v < 16; v++) {
-        const int i = 8 * (v / 4) + 4 * h + (v % 4);
-        gu[((size_t)mat * MT + i) * RP + 32 * rq + n] = acc[v];
-    }
-    __syncthreads();
-    const int mg = m / G;
-    for (int it = w; it < MT * (GU_ROWS / 64); it += NWAVE) {
-        const int i = it / (GU_ROWS / 64), piece = it % (GU_ROWS / 64);
-        if (i >= ti.nt) continue;                 // wave-uniform
-        const int slot = slots[i];
-        const int rr = 64 * piece + lane;         // row within the block
-        // SiLU(g) * u, dividing as the reference does (decode_kernel.c:1375)
-        const float g = gu[(size_t)i * RP + rr], u = gu[((size_t)MT + i) * RP + rr];
-        const float av = swiglu(g, u);
-        const int row = r0 + rr;
-        a.act[(size_t)slot * m + row] = av;
-        const int g0 = row / G;                   // this lane's group (a G-lane segment)
-        encode_i8_group_wave<G>(av, true, a.aqh + (size_t)slot * m + (size_t)g0 * G,
-                                a.aql + (size_t)slot * m + (size_t)g0 * G, a.aqs + (size_t)slot * mg + g0,
-                                a.aqc + (size_t)slot * mg + g0);
+    for (int mat = 0; mat < 2; mat++) {           // gate rows, then the same up rows
+        unsigned long long so, po;
+        a.rec.get(mat, a.key0 + ti.x, so, po);
+        op.w[mat] = a.blob + scalar(po) + (size_t)(rblk * GU_ROWS + 32 * w) * op.wrow;
+        op.sc[mat] = a.blob + scalar(so) + (size_t)(rblk * GU_ROWS + 32 * w) * op.srow;
     }
 }
 
+constexpr int ACT_RP = GU_ROWS + 4;               // padded LDS row of one token's act values
+
+// The unit's act values: SiLU(g) * u (dividing as the reference does,
+// decode_kernel.c:1375) to LDS, then 16 consecutive rows of one token per
+// thread: the float values and their record for the down product.
+template <int G>
+__device__ __forceinline__ void gateup_out(const ExpertArgs& a, const floatx16 (&acc)[2], const int4& ti, int rblk, int sl,
+                                           float* act) {
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, n = lane & 31, h = lane >> 5;
+    const int m = a.m, r0 = rblk * GU_ROWS;
+#pragma unroll
+    for (int v = 0; v < 16; v++) act[(8 * (v / 4) + 4 * h + (v % 4)) * ACT_RP + 32 * w + n] = swiglu(acc[0][v], acc[1][v]);
+    __builtin_amdgcn_s_waitcnt(0xC07F);           // lgkmcnt(0)
+    wave_meet();
+    const int it = tid >> 3, rr = 16 * (tid & 7);
+    const bool live = it < ti.z;
+    const int slot = __shfl(sl, it, JM_WAVE);
+    float v[16];
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        const float4 f = *(const float4*)(act + it * ACT_RP + rr + 4 * q);
+        v[4 * q] = f.x; v[4 * q + 1] = f.y; v[4 * q + 2] = f.z; v[4 * q + 3] = f.w;
+        if (live) *(float4*)(a.act + (size_t)slot * m + r0 + rr + 4 * q) = f;
+    }
+    f6_encode16<G>(v, (r0 + rr) / 16, live, a.aq + f6_rec_bytes(slot, m), a.ae + (size_t)slot * (m / G),
+                   a.ac + (size_t)slot * (m / G));
+}
+
 // The experts under dense_min (n_tiles[1] entries of the small list) as
-// wave items, run by the blocks past the tiles (first = the first such
-// block, nblk = how many): virtual block v of 8 waves takes the 8
-// consecutive items 8 (v % vpe) + w of small entry v / vpe.  The blocks are
-// dispatched after the tiles' and fill the grid's last round.  The grid
-// always has at least (row blocks) x (small experts) of them: an expert
-// under dense_min frees a whole tile of max_tiles = slots / 32 + E.
+// wave items, the units after the tiles' (first = this block's first of them,
+// nblk = the blocks of the grid): virtual block v takes the 4 consecutive items
+// 4 (v % vpe) + w of small entry v / vpe.
 template <int G, int LPR, int NDIG>
 __device__ __forceinline__ void small_gateup(const ExpertArgs& a, int first, int nblk, unsigned char* sm) {
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int vpe = a.m / wi::GU_ROWS / NWAVE;
     const int nv = a.n_tiles[1] * vpe;
-    // per group of 4 waves, the act-scale slots of wi::gateup_item
-    float (*gm)[2][4] = (float (*)[2][4])sm;
-    int (*gb)[2][4] = (int (*)[2][4])(sm + 2 * sizeof(float[2][4]));
+    // the act-scale slots of wi::gateup_item
+    float (&gm)[2][4] = *(float (*)[2][4])sm;
+    int (&gb)[2][4] = *(int (*)[2][4])(sm + sizeof(float[2][4]));
 #pragma unroll 1
     for (int v = first; v < nv; v += nblk) {
-        wi::gateup_item<G, NDIG, LPR, 1, false>(a, a.top, a.small[v / vpe], (v % vpe) * NWAVE + w, gm[w >> 2],
-                                                   gb[w >> 2]);
+        wi::gateup_item<G, NDIG, LPR, 1, false>(a, a.top, a.small[v / vpe], (v % vpe) * NWAVE + w, gm, gb);
         __syncthreads();                          // the slots serve the next item
     }
 }
 
-// 1-D grid: block f < n_tiles x (m / GU_ROWS) is tile f % n_tiles, row
-// block f / n_tiles; the rest run the small experts' items.
 template <int G, int LPR, int NDIG>
-__global__ void __launch_bounds__(MTHREADS, 1)
+__global__ void __launch_bounds__(MTHREADS, 2)
 k_gateup_mfma(ExpertArgs a) {
-    extern __shared__ __align__(16) unsigned char sm[];
-    const int nt = a.n_tiles[0], ntb = nt * (a.m / GU_ROWS);
-    const int f = blockIdx.x;
-    if (f < ntb) {
-        gateup_tile<G>(a, tile_at(a, f % nt), f / nt, sm);
-        return;
+    __shared__ __align__(16) uint8_t ring0[RING];
+    __shared__ __align__(16) uint8_t ring1[RING];
+    __shared__ __align__(16) uint8_t corr_l[corr_steps(G, 0) * 3 * PIECE];
+    __shared__ __align__(16) float act[MT * ACT_RP];
+    const Rings rg{{ring0, ring1, nullptr}, corr_l};
+    const int nrb = a.m / GU_ROWS, nb = gridDim.x;
+    int u = blockIdx.x;
+    int4 ti = tile_at(a, u / nrb);
+    const int ntb = scalar(a.n_tiles[0]) * nrb;
+    if (u < ntb) {
+        int sl = tile_slot(a, ti);
+        Operands op;
+        gateup_op<G>(op, a, ti, u % nrb, sl);
+        Pipe<G, 0> p;
+        p.start(op, rg, a.xc + (size_t)(sl / a.topk) * op.ng);
+#pragma unroll 1
+        for (;;) {
+            const int un = u + nb < ntb ? u + nb : u;         // past the last, the last again
+            int4 tn = a.tiles[un / nrb];
+            int sn = 0;
+            Operands nop;
+            p.unit(op, nop, rg,
+                [&]() __attribute__((always_inline)) {
+                    tn = make_int4(scalar(tn.x), scalar(tn.y), scalar(tn.z), 0);
+                    sn = tile_slot(a, tn);
+                },
+                [&](Operands& o) __attribute__((always_inline)) { gateup_op<G>(o, a, tn, un % nrb, sn); });
+            p.next_corr(nop, a.xc + (size_t)(sn / a.topk) * nop.ng);
+            gateup_out<G>(a, p.acc, ti, u % nrb, sl, act);
+            if (un == u) break;
+            p.ct.store(nop.ng, corr_l);
+            u = un;
+            ti = tn;
+            sl = sn;
+            op = nop;
+        }
+        u += nb;
+        __builtin_amdgcn_s_waitcnt(0x0F70);       // vmcnt(0): nothing on its way to LDS
+        __syncthreads();
     }
-    small_gateup<G, LPR, NDIG>(a, f - ntb, (int)gridDim.x - ntb, sm);
+    small_gateup<G, LPR, NDIG>(a, u - ntb, nb, ring0);
 }
 
 // --------------------------------------------------------------------- down
 
 template <int G>
-__device__ __forceinline__ void down_tile(const ExpertArgs& a, const TileInfo& ti, int rblk, unsigned char* sm) {
-    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-    const int d = a.d, m = a.m, ng = m / G;
-    const Lay ly(m, G);
-    int8_t* q = (int8_t*)sm;
-    float* s = (float*)(sm + ly.s);
-    int* cc = (int*)(sm + ly.c);
-    int* tok = (int*)(sm + ly.tok);
-    float* tws = (float*)(tok + MT);
-    uint8_t* wl = sm + ly.w + (size_t)w * 2 * WBUF;
-    if (tid < MT) {
-        const int sl = a.seg_slot[ti.slot0 + (tid < ti.nt ? tid : 0)];   // padding: the first slot
-        tok[tid] = sl;
-        tws[tid] = a.tw[sl];
-    }
+__device__ __forceinline__ void down_op(Operands& op, const ExpertArgs& a, const int4& ti, int rblk, int sl) {
+    const int w = scalar((int)(threadIdx.x >> 6));
+    set_tokens<G>(op, a.aq, a.ae, sl, a.m);
     unsigned long long so, po;
-    a.rec.get(2, a.key0 + ti.e, so, po);
-    const int n = lane & 31, h = lane >> 5;
-    WStream<G> ws;
-    ws.rowb = m / 2;
-    ws.nss = m / SSC;
-    auto start = [&](int pass) __attribute__((always_inline)) {
-        const int wrow0 = rblk * DN_BLOCK_ROWS + pass * DN_ROWS + 32 * w;
-        ws.wbase = a.blob + po + (size_t)wrow0 * (m / 2);
-        ws.srow = a.blob + so + (size_t)(wrow0 + n) * ng * 2;
-        ws.load(0, 0);
-        ws.load(1, 1);
-        return wrow0 + n;
-    };
-    int row = start(0);
-    __syncthreads();
-    stage_phase(a.aqh, a.aql, tok, m, 0, ly.kph, q);
-    stage_scales(a.aqs, a.aqc, tok, ti.nt, ng, ng, s, cc);
-    __syncthreads();
-    // the staged act digits serve DN_BLOCK_ROWS / DN_ROWS passes over the rows
-#pragma unroll 1
-    for (int pass = 0; pass < DN_BLOCK_ROWS / DN_ROWS; pass++) {
-        floatx16 acc = {};
-        wave_product<G>(acc, ws, wl, q, s, cc, TokSrc{a.aqh, a.aql, tok, m}, ly);
-        const int r = row;
-        if (pass + 1 < DN_BLOCK_ROWS / DN_ROWS) row = start(pass + 1);
+    a.rec.get(2, a.key0 + ti.x, so, po);
 #pragma unroll
-        for (int v = 0; v < 16; v++) {
-            const int i = 8 * (v / 4) + 4 * h + (v % 4);
-            if (i < ti.nt) a.y[(size_t)tok[i] * d + r] = __fmul_rn(tws[i], acc[v]);
+    for (int rb = 0; rb < 2; rb++) {
+        op.w[rb] = a.blob + scalar(po) + (size_t)(rblk * DN_ROWS + WROWS * w + 32 * rb) * op.wrow;
+        op.sc[rb] = a.blob + scalar(so) + (size_t)(rblk * DN_ROWS + WROWS * w + 32 * rb) * op.srow;
+    }
+}
+
+// The unit's weighted rows of y.
+__device__ __forceinline__ void down_out(const ExpertArgs& a, const floatx16 (&acc)[2], const int4& ti, int rblk, int sl,
+                                         float tw) {
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, n = lane & 31, h = lane >> 5;
+    const int row = rblk * DN_ROWS + WROWS * w + n;
+#pragma unroll
+    for (int v = 0; v < 16; v++) {
+        const int i = 8 * (v / 4) + 4 * h + (v % 4);
+        const int slot = __shfl(sl, i, JM_WAVE);
+        const float t = __shfl(tw, i, JM_WAVE);
+        if (i < ti.z) {
+            float* const y = a.y + (size_t)slot * a.d + row;
+            y[0] = __fmul_rn(t, acc[0][v]);
+            y[32] = __fmul_rn(t, acc[1][v]);
         }
     }
 }
 
 // The small experts' down items (wi::down_item, no barriers) on the blocks
-// past the tiles, 8 consecutive items of one entry per virtual block.
+// past the tiles, 4 consecutive items of one entry per virtual block.
 template <int G, int LPR, int NDIG>
 __device__ __forceinline__ void small_down(const ExpertArgs& a, int first, int nblk) {
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -553,76 +700,106 @@ __device__ __forceinline__ void small_down(const ExpertArgs& a, int first, int n
         wi::down_item<G, NDIG, LPR, 1>(a, a.small[v / vpe], (v % vpe) * NWAVE + w);
 }
 
-// 1-D grid as k_gateup_mfma's, with row blocks of DN_BLOCK_ROWS hidden rows.
-template <int G, int LPR, int NDIG>
-__global__ void __launch_bounds__(MTHREADS, 1)
+// NSS: super-stages of the contraction (Pipe::unit)
+template <int G, int LPR, int NDIG, int NSS>
+__global__ void __launch_bounds__(MTHREADS, 2)
 k_down_mfma(ExpertArgs a) {
-    extern __shared__ __align__(16) unsigned char sm[];
-    const int nt = a.n_tiles[0], ntb = nt * (a.d / DN_BLOCK_ROWS);
-    const int f = blockIdx.x;
-    if (f < ntb) {
-        down_tile<G>(a, tile_at(a, f % nt), f / nt, sm);
-        return;
+    __shared__ __align__(16) uint8_t ring0[RING];
+    __shared__ __align__(16) uint8_t ring1[NSS == 1 ? 16 : RING];
+    __shared__ __align__(16) uint8_t ring2[NSS == 3 ? RING : 16];
+    __shared__ __align__(16) uint8_t corr_l[corr_steps(G, NSS) * 3 * PIECE];
+    const Rings rg{{ring0, ring1, ring2}, corr_l};
+    const int nrb = a.d / DN_ROWS, nb = gridDim.x;
+    int u = blockIdx.x;
+    int4 ti = tile_at(a, u / nrb);
+    const int ntb = scalar(a.n_tiles[0]) * nrb;
+    if (u < ntb) {
+        int sl = tile_slot(a, ti);
+        float tw = a.tw[sl];
+        Operands op;
+        down_op<G>(op, a, ti, u % nrb, sl);
+        Pipe<G, NSS> p;
+        p.start(op, rg, a.ac + (size_t)sl * op.ng);
+#pragma unroll 1
+        for (;;) {
+            const int un = u + nb < ntb ? u + nb : u;         // past the last, the last again
+            int4 tn = a.tiles[un / nrb];
+            int sn = 0;
+            Operands nop;
+            p.unit(op, nop, rg,
+                [&]() __attribute__((always_inline)) {
+                    tn = make_int4(scalar(tn.x), scalar(tn.y), scalar(tn.z), 0);
+                    sn = tile_slot(a, tn);
+                },
+                [&](Operands& o) __attribute__((always_inline)) { down_op<G>(o, a, tn, un % nrb, sn); });
+            const float twn = a.tw[sn];
+            p.next_corr(nop, a.ac + (size_t)sn * nop.ng);
+            down_out(a, p.acc, ti, u % nrb, sl, tw);
+            if (un == u) break;
+            p.ct.store(nop.ng, corr_l);
+            u = un;
+            ti = tn;
+            sl = sn;
+            tw = twn;
+            op = nop;
+        }
+        u += nb;
+        __builtin_amdgcn_s_waitcnt(0x0F70);       // vmcnt(0): nothing on its way to LDS
+        __syncthreads();
     }
-    small_down<G, LPR, NDIG>(a, f - ntb, (int)gridDim.x - ntb);
+    small_down<G, LPR, NDIG>(a, u - ntb, nb);
 }
 
 // ------------------------------------------------------ plain Q4 product
 
 // out[t][row] = X[t] . dequant(W[row]) for one Q4 matrix (the plugin
 // product q4_gemm_f32, expert_ffn.c:200-215, at prefill-sized T): block
-// (32-token tile, npass x 256 rows, K split z), 8 waves x 32 rows per pass
-// over the tile's staged digits, as the down kernel without routing.  The
-// digits of X come from k_prep_i8.  With gridDim.z > 1 split z covers the
-// columns [z kl, z kl + kl) (whole Q4 groups and super-stages) and writes
-// its partial sums to out + z T m, which k_sum_splits adds in split order.
-template <int G>
-__global__ void __launch_bounds__(MTHREADS, 1)
+// (32-token tile, 256 rows, K split z), 4 waves x 64 rows, as a unit of the
+// down kernel without routing.  The records of X come from k_prep_f6.
+// With gridDim.z > 1 split z covers the columns [z kl, z kl + kl) (whole Q4
+// groups and super-stages) and writes its partial sums to out + z T m, which
+// k_sum_splits adds in split order.
+template <int G, int NSS>
+__global__ void __launch_bounds__(MTHREADS, 2)
 k_q4_gemm_mfma(const uint8_t* __restrict__ packed, const uint16_t* __restrict__ scales,
-               const int8_t* __restrict__ xqh, const int8_t* __restrict__ xql, const float* __restrict__ xqs,
-               const int* __restrict__ xqc, int T, int m, int d, int kl, int npass, float* __restrict__ out) {
-    extern __shared__ __align__(16) unsigned char sm[];
-    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-    const int ng = d / G;                         // groups per row (the scales' row stride)
+               const uint8_t* __restrict__ xq, const uint8_t* __restrict__ xe, const float* __restrict__ xc, int T, int m,
+               int d, int kl, float* __restrict__ out) {
+    __shared__ __align__(16) uint8_t ring0[RING];
+    __shared__ __align__(16) uint8_t ring1[NSS == 1 ? 16 : RING];
+    __shared__ __align__(16) uint8_t ring2[NSS == 3 ? RING : 16];
+    __shared__ __align__(16) uint8_t corr_l[corr_steps(G, NSS) * 3 * PIECE];
+    const Rings rg{{ring0, ring1, ring2}, corr_l};
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int w = scalar(tid >> 6);
+    const int ng = d / G;                         // groups per row
     const int k0 = (int)blockIdx.z * kl;          // the split's first column
-    const Lay ly(kl, G);
     const int t0 = blockIdx.x * MT;
     const int nt = min(MT, T - t0);
     float* const o = out + (size_t)blockIdx.z * T * m;
-    int8_t* q = (int8_t*)sm;
-    float* s = (float*)(sm + ly.s);
-    int* cc = (int*)(sm + ly.c);
-    int* tok = (int*)(sm + ly.tok);
-    uint8_t* wl = sm + ly.w + (size_t)w * 2 * WBUF;
-    if (tid < MT) tok[tid] = t0 + (tid < nt ? tid : 0);   // padding: the tile's first token
-    const int n = lane & 31, h = lane >> 5;
-    WStream<G> ws;
-    ws.rowb = d / 2;
-    ws.nss = kl / SSC;
-    auto start = [&](int pass) __attribute__((always_inline)) {
-        const int wrow0 = (blockIdx.y * npass + pass) * DN_ROWS + 32 * w;
-        ws.wbase = packed + (size_t)wrow0 * (d / 2) + k0 / 2;
-        ws.srow = (const uint8_t*)scales + ((size_t)(wrow0 + n) * ng + k0 / G) * 2;
-        ws.load(0, 0);
-        ws.load(1, 1);
-        return wrow0 + n;
-    };
-    int row = start(0);
-    __syncthreads();
-    stage_phase(xqh + k0, xql + k0, tok, d, 0, ly.kph, q);
-    stage_scales(xqs + k0 / G, xqc + k0 / G, tok, nt, kl / G, ng, s, cc);
-    __syncthreads();
-#pragma unroll 1
-    for (int pass = 0; pass < npass; pass++) {
-        floatx16 acc = {};
-        // (operands one stage ahead would spill this kernel's registers)
-        wave_product<G, false>(acc, ws, wl, q, s, cc, TokSrc{xqh + k0, xql + k0, tok, d}, ly);
-        const int r = row;
-        if (pass + 1 < npass) row = start(pass + 1);
+    const int i0 = lane & 31, h = lane >> 5;
+    const int t = i0 < nt ? i0 : 0;               // padding: the tile's first token
+    const int row0 = blockIdx.y * DN_ROWS + WROWS * w;
+    Operands op;
+    set_tokens<G>(op, xq + f6_rec_bytes(t0, d) + (size_t)k0 * 3, xe + (size_t)t0 * ng + k0 / G, t, d);
 #pragma unroll
-        for (int v = 0; v < 16; v++) {
-            const int i = 8 * (v / 4) + 4 * h + (v % 4);
-            if (i < nt) o[(size_t)(t0 + i) * m + r] = acc[v];
+    for (int rb = 0; rb < 2; rb++) {
+        op.w[rb] = packed + (size_t)(row0 + 32 * rb) * op.wrow + k0 / 2;
+        op.sc[rb] = (const uint8_t*)scales + (size_t)(row0 + 32 * rb) * op.srow + (size_t)(k0 / G) * 2;
+    }
+    op.nss = kl / SSC;
+    op.ng = kl / G;
+    Pipe<G, NSS> p;
+    p.start(op, rg, xc + (size_t)(t0 + t) * ng + k0 / G);
+    Operands nop = op;
+    p.unit(op, nop, rg, []() __attribute__((always_inline)) {}, [](Operands&) __attribute__((always_inline)) {});
+    __builtin_amdgcn_s_waitcnt(0x0F70);           // vmcnt(0): nothing on its way to LDS
+#pragma unroll
+    for (int v = 0; v < 16; v++) {
+        const int i = 8 * (v / 4) + 4 * h + (v % 4);
+        if (i < nt) {
+            float* const y = o + (size_t)(t0 + i) * m + row0 + i0;
+            y[0] = p.acc[0][v];
+            y[32] = p.acc[1][v];
         }
     }
 }
@@ -649,86 +826,60 @@ k_sum_splits(const float4* __restrict__ part, long long n4, int ns, float4* __re
     out[i] = r;
 }
 
-// Int8 digit pairs and scales of T rows of d floats, one G-lane segment per
-// Q4 group (the encoding of the block's router kernels).
+// The records, exponents and corrections of T rows of d floats, 16 columns per
+// thread (as the dispatch launch encodes the block's tokens).
 template <int G>
 __global__ void __launch_bounds__(256)
-k_prep_i8(const float* __restrict__ X, int T, int d, int8_t* __restrict__ hi, int8_t* __restrict__ lo,
-          float* __restrict__ sc, int* __restrict__ qc) {
-    const long long seg = ((long long)blockIdx.x * blockDim.x + threadIdx.x) / G;
-    const int ng = d / G;
-    const bool ok = seg < (long long)T * ng;
-    const long long sg = ok ? seg : 0;
-    const int t = (int)(sg / ng), g = (int)(sg % ng);
-    const size_t o = (size_t)t * d + (size_t)g * G;
-    const float v = ok ? X[o + (threadIdx.x & (G - 1))] : 0.0f;
-    encode_i8_group_wave<G>(v, ok, hi + o, lo + o, sc + (size_t)t * ng + g, qc + (size_t)t * ng + g);
+k_prep_f6(const float* __restrict__ X, int T, int d, uint8_t* __restrict__ rec, uint8_t* __restrict__ exps,
+          float* __restrict__ corr) {
+    const long long u = (long long)blockIdx.x * 256 + threadIdx.x;
+    const int nblk = d / 16, ng = d / G;
+    const long long b = u / nblk;
+    const int c16 = (int)(u % nblk);
+    const bool ok = b < T;
+    const size_t row = ok ? b : 0;
+    const float4* xp = (const float4*)(X + row * d + 16 * c16);
+    float v[16];
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        const float4 f = xp[q];
+        v[4 * q] = f.x; v[4 * q + 1] = f.y; v[4 * q + 2] = f.z; v[4 * q + 3] = f.w;
+    }
+    f6_encode16<G>(v, c16, ok, rec + f6_rec_bytes(row, d), exps + row * ng, corr + row * ng);
 }
 
-// Contractions the kernels take: multiples of the weight super-stage, and
-// one token phase or whole phases; row counts of whole blocks.
-static bool mfma_k_ok(int K) { return K % SSC == 0 && K <= KMAX && (K <= KPH_MAX || K % KPH_MAX == 0); }
+// Contractions the kernels take: whole super-stages up to 1024 columns, or
+// whole 1024s; row counts of whole blocks.
+static bool mfma_k_ok(int K) { return K % SSC == 0 && K <= KMAX && (K <= 1024 || K % 1024 == 0); }
 
 bool mfma_shape_ok(int d, int m) {
-    return d % DN_BLOCK_ROWS == 0 && m % GU_ROWS == 0 && mfma_k_ok(d) && mfma_k_ok(m);
+    return d % 512 == 0 && m % GU_ROWS == 0 && mfma_k_ok(d) && mfma_k_ok(m);
 }
-
-namespace {
-
-template <int G>
-constexpr size_t gateup_lds(int d) {
-    return Lay(d, G).total > (size_t)2 * MT * (GU_ROWS + 4) * 4 ? Lay(d, G).total
-                                                                 : (size_t)2 * MT * (GU_ROWS + 4) * 4;
-}
-
-// Dynamic LDS above 64 KiB must be allowed per kernel: once per device,
-// for the largest contraction the kernels take.
-constexpr int MAX_DEV = 64;
-std::atomic<unsigned> g_lds_set[MAX_DEV];
-
-hipError_t allow_lds() {
-    int dev = 0;
-    hipError_t e = hipGetDevice(&dev);
-    if (e != hipSuccess) return e;
-    if (dev < 0 || dev >= MAX_DEV) return hipErrorInvalidDevice;
-    if (g_lds_set[dev].load(std::memory_order_acquire)) return hipSuccess;
-#define JM_MF(N) \
-        {(const void*)k_gateup_mfma<64, 32, N>, gateup_lds<64>(KMAX)}, {(const void*)k_gateup_mfma<64, 64, N>, gateup_lds<64>(KMAX)}, \
-        {(const void*)k_gateup_mfma<32, 32, N>, gateup_lds<32>(KMAX)}, {(const void*)k_gateup_mfma<32, 64, N>, gateup_lds<32>(KMAX)}, \
-        {(const void*)k_down_mfma<64, 32, N>, Lay(KMAX, 64).total}, {(const void*)k_down_mfma<64, 64, N>, Lay(KMAX, 64).total}, \
-        {(const void*)k_down_mfma<32, 32, N>, Lay(KMAX, 32).total}, {(const void*)k_down_mfma<32, 64, N>, Lay(KMAX, 32).total}
-    const struct { const void* f; size_t b; } k[18] = {
-        JM_MF(4), JM_MF(5),
-        {(const void*)k_q4_gemm_mfma<64>, Lay(KMAX, 64).total}, {(const void*)k_q4_gemm_mfma<32>, Lay(KMAX, 32).total}};
-#undef JM_MF
-    for (const auto& x : k) {
-        e = hipFuncSetAttribute(x.f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)x.b);
-        if (e != hipSuccess) return e;
-    }
-    g_lds_set[dev].store(1u, std::memory_order_release);
-    return hipSuccess;
-}
-
-}  // namespace
 
 // Lanes per row segment of the small experts' wave items: rows of C columns
 // (C / 32 chunks of 16 bytes; C <= KMAX, so one chunk per lane).
 static int item_lanes(int C) { return C / 32 <= 32 ? 32 : 64; }
 
-// Grids of max_tiles x (row blocks) blocks, one row of blocks more: the
-// blocks past the device's tile count run the small experts' wave items.
+// Two blocks per CU (registers and LDS), or as many as there can be units:
+// max_tiles tiles and one more row of blocks for the small experts' items.
+static unsigned unit_blocks(int max_tiles, int row_blocks) {
+    static const int ncu = [] {
+        int dev = 0, n = 0;
+        if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
+            n = 0;
+        return n > 0 ? n : 256;
+    }();
+    return (unsigned)std::min<long long>(2 * ncu, (long long)(max_tiles + 1) * row_blocks);
+}
+
 hipError_t launch_gateup_mfma(const ExpertArgs& a, int max_tiles, hipStream_t st) {
     if (max_tiles == 0) return hipSuccess;
     if (!mfma_shape_ok(a.d, a.m) || (a.group != 64 && a.group != 32)) return hipErrorInvalidValue;
-    if (!a.small || (a.m / wi::GU_ROWS) % NWAVE) return hipErrorInvalidValue;
-    hipError_t e = allow_lds();
-    if (e != hipSuccess) return e;
-    const int rb = a.m / GU_ROWS;
-    const dim3 grid((unsigned)((max_tiles + 1) * rb));
+    if (!a.small || (a.m / wi::GU_ROWS) % NWAVE || (a.ndig != 4 && a.ndig != 5)) return hipErrorInvalidValue;
+    const dim3 grid(unit_blocks(max_tiles, a.m / GU_ROWS));
     const bool l64 = item_lanes(a.d) == 64;
-    if (a.ndig != 4 && a.ndig != 5) return hipErrorInvalidValue;
-#define JM_GM(GG, L) do { if (a.ndig == 5) hipLaunchKernelGGL((k_gateup_mfma<GG, L, 5>), grid, dim3(MTHREADS), gateup_lds<GG>(a.d), st, a); \
-                          else hipLaunchKernelGGL((k_gateup_mfma<GG, L, 4>), grid, dim3(MTHREADS), gateup_lds<GG>(a.d), st, a); } while (0)
+#define JM_GM(GG, L) do { if (a.ndig == 5) hipLaunchKernelGGL((k_gateup_mfma<GG, L, 5>), grid, dim3(MTHREADS), 0, st, a); \
+                          else hipLaunchKernelGGL((k_gateup_mfma<GG, L, 4>), grid, dim3(MTHREADS), 0, st, a); } while (0)
     if (a.group == 64) {
         if (l64) JM_GM(64, 64);
         else JM_GM(64, 32);
@@ -743,15 +894,14 @@ hipError_t launch_gateup_mfma(const ExpertArgs& a, int max_tiles, hipStream_t st
 hipError_t launch_down_mfma(const ExpertArgs& a, int max_tiles, hipStream_t st) {
     if (max_tiles == 0) return hipSuccess;
     if (!mfma_shape_ok(a.d, a.m) || (a.group != 64 && a.group != 32)) return hipErrorInvalidValue;
-    if (!a.small || (a.d / wi::DN_ROWS) % NWAVE) return hipErrorInvalidValue;
-    hipError_t e = allow_lds();
-    if (e != hipSuccess) return e;
-    const int rb = a.d / DN_BLOCK_ROWS;
-    const dim3 grid((unsigned)((max_tiles + 1) * rb));
+    if (!a.small || (a.d / wi::DN_ROWS) % NWAVE || (a.ndig != 4 && a.ndig != 5)) return hipErrorInvalidValue;
+    const dim3 grid(unit_blocks(max_tiles, a.d / DN_ROWS));
     const bool l64 = item_lanes(a.m) == 64;
-    if (a.ndig != 4 && a.ndig != 5) return hipErrorInvalidValue;
-#define JM_DM(GG, L) do { if (a.ndig == 5) hipLaunchKernelGGL((k_down_mfma<GG, L, 5>), grid, dim3(MTHREADS), Lay(a.m, GG).total, st, a); \
-                          else hipLaunchKernelGGL((k_down_mfma<GG, L, 4>), grid, dim3(MTHREADS), Lay(a.m, GG).total, st, a); } while (0)
+    const int nss = a.m / SSC;
+#define JM_DN(GG, L, N) do { if (nss == 1) hipLaunchKernelGGL((k_down_mfma<GG, L, N, 1>), grid, dim3(MTHREADS), 0, st, a); \
+                             else if (nss == 3) hipLaunchKernelGGL((k_down_mfma<GG, L, N, 3>), grid, dim3(MTHREADS), 0, st, a); \
+                             else hipLaunchKernelGGL((k_down_mfma<GG, L, N, 0>), grid, dim3(MTHREADS), 0, st, a); } while (0)
+#define JM_DM(GG, L) do { if (a.ndig == 5) JM_DN(GG, L, 5); else JM_DN(GG, L, 4); } while (0)
     if (a.group == 64) {
         if (l64) JM_DM(64, 64);
         else JM_DM(64, 32);
@@ -760,6 +910,7 @@ hipError_t launch_down_mfma(const ExpertArgs& a, int max_tiles, hipStream_t st) 
         else JM_DM(32, 32);
     }
 #undef JM_DM
+#undef JM_DN
     return hipGetLastError();
 }
 
@@ -787,7 +938,7 @@ int q4_gemm_splits(int T, int m, int d) {
 
 size_t q4_gemm_mfma_ws(int T, int m, int d, int group) {
     const int ns = q4_gemm_splits(T, m, d);
-    return pad256((size_t)T * d) * 2 + pad256((size_t)T * (d / group) * 4) * 2 +
+    return pad256(f6_rec_bytes(T, d)) + pad256((size_t)T * (d / group)) + pad256((size_t)T * (d / group) * 4) +
            (ns > 1 ? pad256((size_t)ns * T * m * 4) : 0);
 }
 
@@ -795,31 +946,22 @@ hipError_t launch_q4_gemm_mfma(const uint8_t* packed, const uint16_t* scales, co
                                int group, void* ws, float* out, hipStream_t st) {
     if (T == 0 || m == 0) return hipSuccess;
     if (!q4_gemm_mfma_ok(m, d, group)) return hipErrorInvalidValue;
-    hipError_t e = allow_lds();
-    if (e != hipSuccess) return e;
-    int8_t* hi = (int8_t*)ws;
-    int8_t* lo = hi + pad256((size_t)T * d);
-    float* sc = (float*)(lo + pad256((size_t)T * d));
-    int* qc = (int*)((char*)sc + pad256((size_t)T * (d / group) * 4));
-    float* part = (float*)((char*)qc + pad256((size_t)T * (d / group) * 4));
-    const long long lanes = (long long)T * d;
-    const unsigned pblocks = (unsigned)((lanes + 255) / 256);
+    uint8_t* xq = (uint8_t*)ws;
+    uint8_t* xe = xq + pad256(f6_rec_bytes(T, d));
+    float* xc = (float*)(xe + pad256((size_t)T * (d / group)));
+    float* part = (float*)((char*)xc + pad256((size_t)T * (d / group) * 4));
+    const unsigned pblocks = (unsigned)(((long long)T * (d / 16) + 255) / 256);
     const int ns = q4_gemm_splits(T, m, d);
     const int kl = d / ns;
     float* dst = ns > 1 ? part : out;
-    // two passes per block when the rows allow and the grid still fills the chip
-    const int tiles = (T + MT - 1) / MT;
-    const int npass = (m % (2 * DN_ROWS) == 0 && (long long)tiles * (m / (2 * DN_ROWS)) >= 256) ? 2 : 1;
-    const dim3 grid((unsigned)tiles, (unsigned)(m / (DN_ROWS * npass)), (unsigned)ns);
-    if (group == 64) {
-        hipLaunchKernelGGL(k_prep_i8<64>, dim3(pblocks), dim3(256), 0, st, X, T, d, hi, lo, sc, qc);
-        hipLaunchKernelGGL(k_q4_gemm_mfma<64>, grid, dim3(MTHREADS), Lay(kl, 64).total, st, packed, scales, hi, lo, sc,
-                           qc, T, m, d, kl, npass, dst);
-    } else {
-        hipLaunchKernelGGL(k_prep_i8<32>, dim3(pblocks), dim3(256), 0, st, X, T, d, hi, lo, sc, qc);
-        hipLaunchKernelGGL(k_q4_gemm_mfma<32>, grid, dim3(MTHREADS), Lay(kl, 32).total, st, packed, scales, hi, lo, sc,
-                           qc, T, m, d, kl, npass, dst);
-    }
+    const dim3 grid((unsigned)((T + MT - 1) / MT), (unsigned)(m / DN_ROWS), (unsigned)ns);
+#define JM_QG(GG, N) hipLaunchKernelGGL((k_q4_gemm_mfma<GG, N>), grid, dim3(MTHREADS), 0, st, packed, scales, xq, xe, xc, T, m, d, kl, dst)
+#define JM_QGG(GG) do { hipLaunchKernelGGL(k_prep_f6<GG>, dim3(pblocks), dim3(256), 0, st, X, T, d, xq, xe, xc); \
+                        if (kl / SSC == 1) JM_QG(GG, 1); else if (kl / SSC == 3) JM_QG(GG, 3); else JM_QG(GG, 0); } while (0)
+    if (group == 64) JM_QGG(64);
+    else JM_QGG(32);
+#undef JM_QGG
+#undef JM_QG
     if (ns > 1) {
         const long long n4 = (long long)T * m / 4;
         hipLaunchKernelGGL(k_sum_splits, dim3((unsigned)((n4 + 255) / 256)), dim3(256), 0, st, (const float4*)part, n4,

@@ -32,6 +32,7 @@
 #include "jm_chain.h"
 #include "jm_device.h"
 #include "jm_kernels.h"
+#include "jm_mx.h"
 
 namespace jm {
 
@@ -92,31 +93,21 @@ hipError_t launch_bf16_exact(const float* in, long long n, unsigned* flag, hipSt
 
 
 // Where the encodes of NT groups go: entry t receives group p of token b
-// (its x digits and their scale; for the MFMA branch also its digit pairs,
-// their scale and integer sum).
+// (its x digits and their scale).
 template <int G, int NDIG, int NT>
 struct EncDst {
     uint32_t* dig[NT];
     float* sc[NT];
-    int8_t* hi[NT];
-    int8_t* lo[NT];
-    float* qs[NT];
-    int* qc[NT];
-    __device__ __forceinline__ void set(int t, const RouteArgs& a, size_t b, int p, bool i8) {
-        const size_t ng = (size_t)(a.d / G), g = b * ng + p, o = b * a.d + (size_t)p * G;
+    __device__ __forceinline__ void set(int t, const RouteArgs& a, size_t b, int p) {
+        const size_t g = b * (size_t)(a.d / G) + p;
         dig[t] = a.xdig + g * (NDIG * (G / 8));
         sc[t] = a.xscale + g;
-        hi[t] = a.xqh + (i8 ? o : 0);
-        lo[t] = a.xql + (i8 ? o : 0);
-        qs[t] = a.xqs + g;
-        qc[t] = a.xqc + g;
     }
 };
 
 // x digits of token b staged in xT (chain order), wave eg's share of the
-// token's groups over ngrp waves: one G-value group per G-lane segment (and,
-// for the MFMA branch, the same group as int8 digit pairs), two groups at a
-// time so that their reduction chains interleave.  Run before the router
+// token's groups over ngrp waves: one G-value group per G-lane segment, two
+// groups at a time so that their reduction chains interleave.  Run before the router
 // chains: it needs only the staged token, so it runs while the table's
 // chunks arrive.
 template <int G, int NDIG, int d>
@@ -126,7 +117,6 @@ __device__ __forceinline__ void encode_token_share(const RouteArgs& a, int b, in
     constexpr int PPW = JM_WAVE / G;
     const int lane = threadIdx.x & 63;
     const int sub = lane / G;
-    const bool i8 = a.xqh != nullptr;
     for (int base = eg * PPW; base < ng; base += 2 * ngrp * PPW) {
         float v[2];
         bool ok[2];
@@ -138,9 +128,9 @@ __device__ __forceinline__ void encode_token_share(const RouteArgs& a, int b, in
             const int pp = ok[u] ? p : 0;
             const int j = pp * G + (lane & (G - 1));
             v[u] = ok[u] ? xT[(size_t)(j & 7) * TP + (j >> 3)] : 0.0f;
-            dst.set(u, a, (size_t)b, pp, i8);
+            dst.set(u, a, (size_t)b, pp);
         }
-        encode_groups_n<G, NDIG, 2>(v, ok, dst.dig, dst.sc, i8, dst.hi, dst.lo, dst.qs, dst.qc);
+        encode_groups_n<G, NDIG, 2>(v, ok, dst.dig, dst.sc);
     }
 }
 
@@ -260,6 +250,11 @@ k_router_grp(RouteArgs a) {
             xv[i].w = __fmul_rn(__fmul_rn(xv[i].w, inv), bf16_bits_to_f32(w.y >> 16));
         }
     }
+    if (LAYER && eg == 0 && a.xn) {
+        float4* xo = (float4*)(a.xn + (size_t)b * d);
+#pragma unroll
+        for (int i = 0; i < XV; i++) xo[lane + 64 * i] = xv[i];
+    }
     stage_chain_order<XV, TP>(xv, xT);
     __syncthreads();
     encode_token_share<G, NDIG, d>(a, b, eg, ngrp, xT);
@@ -274,8 +269,8 @@ k_router_grp(RouteArgs a) {
 // runs its group's chains for the 4 tokens from one read of its table
 // chunks, each token's chain in the same order as k_router_grp's, so the
 // scores are the same bits.  The table is read once per 4 tokens instead of
-// once per token.  The x digits and the MFMA-branch digit pairs of the 4 tokens
-// are shared out over the grid's waves as k_router_grp shares them.
+// once per token.  The x digits of the 4 tokens are shared out over the grid's
+// waves as k_router_grp shares them.
 constexpr int RQ_T = 4;             // tokens per block
 template <int G, int NDIG, int DV, bool WBF16, bool LAYER>
 __global__ void __launch_bounds__(256)
@@ -383,9 +378,8 @@ k_router_quad(RouteArgs a) {
     }
     __syncthreads();
     const int nt = min(RQ_T, a.B - b0);           // tokens of this block (>= 1)
-    // x digits (one G-value group per G-lane segment) and the MFMA digit
-    // pairs of the block's tokens, this wave's share over the grid's nvg
-    // waves, before the chains: they need only the staged tokens, so they
+    // x digits (one G-value group per G-lane segment) of the block's tokens,
+    // this wave's share over the grid's nvg waves, before the chains: they need only the staged tokens, so they
     // run while the table's chunks are still arriving.  The tokens of a
     // group are encoded together (unconditionally, the stores guarded), so
     // that their reduction chains interleave.  With enc_late the dispatch
@@ -394,7 +388,6 @@ k_router_quad(RouteArgs a) {
     constexpr int ng = d / G;
     constexpr int PPW = JM_WAVE / G;
     const int sub = lane / G;
-    const bool i8 = a.xqh != nullptr;
     for (int base = a.enc_late ? ng : eg * PPW; base < ng; base += nvg * PPW) {
         const int p = base + sub;
         const bool ok = p < ng;
@@ -407,9 +400,9 @@ k_router_quad(RouteArgs a) {
         for (int t = 0; t < RQ_T; t++) {
             st[t] = ok && t < nt;
             v[t] = st[t] ? xT[t][(size_t)(j & 7) * TP + (j >> 3)] : 0.0f;
-            dst.set(t, a, (size_t)b0 + (t < nt ? t : 0), pp, i8);
+            dst.set(t, a, (size_t)b0 + (t < nt ? t : 0), pp);
         }
-        encode_groups_n<G, NDIG, RQ_T>(v, st, dst.dig, dst.sc, i8, dst.hi, dst.lo, dst.qs, dst.qc);
+        encode_groups_n<G, NDIG, RQ_T>(v, st, dst.dig, dst.sc);
     }
     if (chains) {
         float acc[RQ_T];
@@ -439,25 +432,40 @@ k_router_quad(RouteArgs a) {
     }
 }
 
-// The dispatch launch's token encode (enc_late): the x digits and, for the
-// MFMA branch, the digit pairs of every token, from a.xenc (the tokens as the
-// router scored them).  Item (ENC_T tokens, group position) per wave, one
-// G-value group per G-lane segment, the tokens' loads issued together; the
-// same values as the router's encode.  Two tokens per item measured best:
-// at 512 tokens the block took 1.2 us less than with 4 (0.9 us at 64); with
-// 1 token per item it took as long at 512 and 0.4 us more at 64 tokens (when
-// the encode moved here from 64 tokens on).
-// (The 4 encodes of a 4-token item through
-// encode_groups_n made the 512-token block about 0.5 us slower.)
+// The dispatch launch's token encodes, on its waves past the dispatch block
+// (wave gw of nw), of the tokens as the router scored them (a.xenc):
+//   enc_late  the x digits: item (ENC_T tokens, group position) per wave, one
+//             G-value group per G-lane segment, the tokens' loads issued
+//             together; the same values as the router's encode.  Two tokens
+//             per item measured best: at 512 tokens the block took 1.2 us less
+//             than with 4; with 1 as long
+//   a.xq      the matrix-core records, 16 columns per thread
 constexpr int ENC_T = 2;
 template <int G, int NDIG>
 __device__ __forceinline__ void encode_late(const RouteArgs& a, int gw, int nw) {
     constexpr int PPW = JM_WAVE / G;
     const int lane = threadIdx.x & 63, sub = lane / G;
     const int d = a.d, ng = d / G, ngw = ng / PPW;
-    const int nq = (a.B + ENC_T - 1) / ENC_T;
-    const bool i8 = a.xqh != nullptr;
-    for (int it = gw; it < nq * ngw; it += nw) {
+    const int nf6 = a.xq ? (int)(((long long)a.B * (d / 16) + 63) / 64) : 0;
+    const int ndig = a.enc_late ? (a.B + ENC_T - 1) / ENC_T * ngw : 0;
+#pragma unroll 1
+    for (int it = gw; it < nf6; it += nw) {
+        const long long u = (long long)it * 64 + lane;      // whole groups: d / 16 is a multiple of G / 16
+        const int nblk = d / 16;
+        const int b = (int)(u / nblk), c16 = (int)(u % nblk);
+        const bool ok = b < a.B;
+        const float4* xp = (const float4*)(a.xenc + (size_t)(ok ? b : 0) * d + 16 * c16);
+        float v[16];
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            const float4 f = xp[q];
+            v[4 * q] = f.x; v[4 * q + 1] = f.y; v[4 * q + 2] = f.z; v[4 * q + 3] = f.w;
+        }
+        f6_encode16<G>(v, c16, ok, a.xq + f6_rec_bytes(ok ? b : 0, d), a.xe + (size_t)(ok ? b : 0) * ng,
+                       a.xc + (size_t)(ok ? b : 0) * ng);
+    }
+#pragma unroll 1
+    for (int it = nw - 1 - gw; it < ndig; it += nw) {
         const int q = it / ngw;
         const int p = (it - q * ngw) * PPW + sub;
         const int b0 = q * ENC_T;
@@ -469,18 +477,18 @@ __device__ __forceinline__ void encode_late(const RouteArgs& a, int gw, int nw) 
             v[t] = a.xenc[b * d + (size_t)p * G + (lane & (G - 1))];
         }
         EncDst<G, NDIG, ENC_T> dst;
+        bool st[ENC_T];
 #pragma unroll
         for (int t = 0; t < ENC_T; t++) {
-            const bool st = t < nt;
-            dst.set(t, a, (size_t)b0 + (st ? t : 0), p, i8);
-            encode_group_both<G, NDIG>(st ? v[t] : 0.0f, st, dst.dig[t], dst.sc[t], i8, dst.hi[t], dst.lo[t],
-                                       dst.qs[t], dst.qc[t]);
+            st[t] = t < nt;
+            dst.set(t, a, (size_t)b0 + (st[t] ? t : 0), p);
+            encode_group_wave<G, NDIG>(st[t] ? v[t] : 0.0f, st[t], dst.dig[t], dst.sc[t]);
         }
     }
 }
 
 // Dispatch and work table of all slots from the top-k table (dispatch
-// path), on block 0; with enc_late, the blocks past it encode the tokens.
+// path), on block 0; the blocks past it encode the tokens.
 template <int G, int NDIG>
 __global__ void __launch_bounds__(1024)
 k_dispatch_work(RouteArgs a) {
@@ -492,8 +500,9 @@ k_dispatch_work(RouteArgs a) {
     }
     ExpertRec rec;
     if ((int)threadIdx.x < a.E) rec = load_expert_rec(a.rec, a.key0, threadIdx.x);
-    // the work entries' slot counts come back in LDS (over the expert
-    // counts, dead by then); the scan below uses the dispatch's scan scratch
+    // the work entries' slot counts and experts come back in LDS (over the
+    // expert counts, dead by then), and the segment starts are there (off);
+    // the scan below uses the dispatch's scan scratch
     int* const wn = lds_i;
     unsigned* const wsum = (unsigned*)(lds_i + 3 * a.E + 1);
     dispatch_block<false>(a.top, a.B * a.topk, a.E, a.topk, lds_i, a.seg_off, a.seg_slot, a.active,
@@ -502,15 +511,18 @@ k_dispatch_work(RouteArgs a) {
     // the experts under dense_min (their wave items run on the MFMA grids)
     lds_barrier();
     const int u = threadIdx.x;
-    int ct = 0, sm = 0;
+    int ct = 0, sm = 0, n = 0, e = 0;
     if (u < a.umax) {
-        const int n = wn[u];
+        n = wn[u] & 0xFFFF;
+        e = wn[u] >> 16;
         ct = n >= a.dense_min ? (n + JM_DENSE_TILE - 1) / JM_DENSE_TILE : 0;
         sm = n > 0 && n < a.dense_min;
     }
     uint2 tot;
     const uint2 ex = block_exclusive_scan2(make_uint2((unsigned)ct, (unsigned)sm), wsum, &tot);
-    for (int j = 0; j < ct; j++) a.tiles[ex.x + j] = make_int2(u, j);
+    const int s0 = lds_i[a.E + e];
+    for (int j = 0; j < ct; j++)
+        a.tiles[ex.x + j] = make_int4(e, s0 + j * JM_DENSE_TILE, min(JM_DENSE_TILE, n - j * JM_DENSE_TILE), 0);
     if (sm) a.small[ex.y] = u;
     if (threadIdx.x == 0) {
         a.n_tiles[0] = (int)tot.x;
@@ -550,13 +562,11 @@ hipError_t launch_route_tok(const RouteArgs& a, hipStream_t st) {
 constexpr int ENC_LATE_MAX_BLOCKS = 1024;
 
 hipError_t launch_dispatch_work(const RouteArgs& a, hipStream_t st) {
-    int nenc = 0;
-    if (a.enc_late) {
-        if (a.group != 32 && a.group != 64) return hipErrorInvalidValue;
-        if (a.ndig != 4 && a.ndig != 5) return hipErrorInvalidValue;
-        const long long items = (long long)((a.B + ENC_T - 1) / ENC_T) * (a.d / 64);
-        nenc = (int)std::min<long long>(ENC_LATE_MAX_BLOCKS, (items + 15) / 16);
-    }
+    if (a.group != 32 && a.group != 64) return hipErrorInvalidValue;
+    if (a.ndig != 4 && a.ndig != 5) return hipErrorInvalidValue;
+    const long long dig = a.enc_late ? (long long)((a.B + ENC_T - 1) / ENC_T) * (a.d / 64) : 0;
+    const long long f6 = a.xq ? ((long long)a.B * (a.d / 16) + 63) / 64 : 0;
+    const int nenc = (int)std::min<long long>(ENC_LATE_MAX_BLOCKS, (dig + f6 + 15) / 16);
     const dim3 grid((unsigned)(1 + nenc));
     const size_t lds = (size_t)dispatch_lds_ints(a.B * a.topk, a.E) * 4;
     if (a.group == 64) {

@@ -26,21 +26,19 @@ struct Ws {
     int* first_slot;            // [E]
     int* comb;                  // [B*k]
     ExpertWork* work;           // [E]
-    int2* tiles;                // [B*k/32 + E] dense tiles (dispatch path)
+    int4* tiles;                // [B*k/32 + E + 1] dense tiles (dispatch path)
     int* n_tiles;               // [2] dense tiles, experts under dense_min
     int* small;                 // [E] work-table entries of the experts under dense_min
     float* act;                 // [B*k][m]
     uint32_t* adig;             // [B*k][m/8][NDIG] act digits
     float* ascale;              // [B*k][m/32]
     float* y;                   // [B*k][d]
-    int8_t* aqh;                // [B*k][m] act as int8 digit pairs for the MFMA down
-    int8_t* aql;
-    int8_t* xqh;                // [B][d] tokens as int8 digit pairs for the MFMA gate/up
-    int8_t* xql;
-    float* xqs;                 // [B][d/G] scales of the token digit pairs
-    float* aqs;                 // [B*k][m/G] scales of the act digit pairs
-    int* xqc;                   // [B][d/G] sums of the token digit pairs' integers per group
-    int* aqc;                   // [B*k][m/G] the same for act
+    uint8_t* aq;                // [B*k][m / 64][192] act as fp6 digit planes for the MFMA down (jm_mx.h)
+    uint8_t* xq;                // [B][d / 64][192] tokens likewise for the MFMA gate/up
+    float* xc;                  // [B][d/G] group corrections of the tokens
+    float* ac;                  // [B*k][m/G] and of act
+    uint8_t* xe;                // [B][d/G] exponents of the tokens' groups
+    uint8_t* ae;                // [B*k][m/G] and of act's
 };
 
 }  // namespace jm
@@ -91,7 +89,7 @@ struct jm_store {
     // optional per-stage events (jm_store_profile)
     int prof;
     hipEvent_t ev[JM_STAGES + 1];
-    int dense_min;              // segment size from which an expert takes the MFMA branch
+    int dense_min;              // segment size from which an expert takes the MFMA branch (0: the default)
     int ndig;                   // activation digit planes of the GEMV kernels (jm_store_set_act_digits)
     bool mfma_ok;               // the shape and the records' alignment allow the MFMA branch
     // ---- batch decode (jm_decode_layers_batch) ----
@@ -149,6 +147,8 @@ int store_reserve(jm_store* s, int B);
 // Bytes of the workspace layout for B tokens of the store's shape, and the
 // fields laid out from base (256-byte aligned).
 size_t ws_bytes(const jm_store* s, int B);
+// The size that decides which batches jm_layer_ffn_batch_noalloc takes.
+size_t ws_noalloc_bytes(const jm_store* s, int B);
 void ws_layout(const jm_store* s, int B, char* base, Ws* w);
 
 // Decoder-layer extras of the MoE block around its input and output.
