@@ -295,6 +295,164 @@ k_gemm_bf16(GemvArgs a) {
     }
 }
 
+// The same product where the blocks outnumber the CUs: block (256-row tile,
+// 64-token tile, column range), 4 waves of 64 tokens x 64 rows each, which
+// read 6 operands from LDS per 8 MFMAs where k_gemm_bf16's 32 x 32 waves read
+// 12, and two blocks per CU instead of one, so that one multiplies while the
+// other waits for its stage.  The stage is 64 columns, so that a weight row's
+// part is a whole 128-byte line (32-column stages fetched each line twice:
+// 152 us against 141 for the case below), in one LDS buffer.  At 301 tokens,
+// us per launch, against k_gemm_bf16: rows x columns 24576 x 4096 141 vs 191
+// (860 TFLOP/s executed), 4096 x 12288 112 vs 140, 6144 x 4096 45 vs 56, 4096
+// x 4096 42 vs 50.  What bounds it: a stage's loads, LDS writes and reads take
+// about 2.05 us for a pair of blocks, of which the MFMAs are 0.85; reading the
+// next stage's operands ahead from a third LDS buffer measured 158 for the
+// first case, and two stages in registers no better.
+constexpr int GW_R = 256;           // weight rows per block
+
+struct GwStage {
+    float4 x[2][2];                 // 8 columns of two tokens
+    uint4 nw;                       // their norm weights (bf16)
+    uint4 w[GW_R / 32];             // 8 columns of weight rows 32 apart
+};
+
+// Offset in bf16 of 8-column chunk c of row r of a staged operand: rows of 128
+// bytes, the chunk rotated by the row so that the rows one read phase touches
+// at one chunk, and the whole rows a write phase touches, spread over every
+// bank.
+__device__ __forceinline__ int gw_at(int r, int c) { return r * GM_KS + 8 * (c ^ ((r >> 1) & 7) ^ (4 * (r & 1))); }
+
+template <bool NORM>
+__global__ void __launch_bounds__(256, 2)
+k_gemm_bf16_wide(GemvArgs a) {
+    typedef float floatx16 __attribute__((ext_vector_type(16)));
+    constexpr int NW = GW_R / 32;
+    __shared__ __align__(16) uint16_t xh[GM_T * GM_KS], xl[GM_T * GM_KS], wl[GW_R * GM_KS];
+    __shared__ float ss_l[GM_T][8];
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    // the first row tile also sums each token's squares (the RMSNorm of the
+    // layer input, for the consumer) from the values it stages
+    const bool want_ss = a.rss && blockIdx.x == 0;
+    float ss[2] = {};
+    const int row0 = blockIdx.x * GW_R, tb0 = blockIdx.y * GM_T;
+    // block z takes the z-th of gridDim.z equal column ranges and writes
+    // slice z of part (and of rss)
+    const int K = a.K, nstage = K / GM_KS / (int)gridDim.z, kz = blockIdx.z;
+    const int kcol0 = kz * nstage * GM_KS;
+    // the row tile lies in one matrix (row counts are multiples of GW_R)
+    const uint16_t* wm;
+    int wr0;
+    if (row0 < a.rows[0]) { wm = a.w[0]; wr0 = row0; }
+    else if (row0 < a.rows[0] + a.rows[1]) { wm = a.w[1]; wr0 = row0 - a.rows[0]; }
+    else { wm = a.w[2]; wr0 = row0 - a.rows[0] - a.rows[1]; }
+    // staging: tokens sr and sr + 32, columns 8 sc .. 8 sc + 7; the same
+    // columns of weight rows sr + 32 i
+    const int sr = tid >> 3, sc = tid & 7;
+    const bool live[2] = {tb0 + sr < a.B, tb0 + sr + 32 < a.B};
+    const float* xrow[2];
+#pragma unroll
+    for (int q = 0; q < 2; q++) xrow[q] = a.x + (size_t)(live[q] ? tb0 + sr + 32 * q : 0) * K + kcol0 + 8 * sc;
+    const uint16_t* wrow = wm + (size_t)(wr0 + sr) * K + kcol0 + 8 * sc;
+    const int sto = gw_at(sr, sc);                // (rows 32 apart rotate alike)
+
+    // every load is unconditional (past the last stage: the last stage again)
+    auto load_stage = [&](GwStage& r, int s) __attribute__((always_inline)) {
+        s = s < nstage ? s : nstage - 1;
+#pragma unroll
+        for (int q = 0; q < 2; q++) {
+            const float4* xs = (const float4*)(xrow[q] + s * GM_KS);
+            r.x[q][0] = xs[0];
+            r.x[q][1] = xs[1];
+        }
+        r.nw = NORM ? *(const uint4*)(a.norm_w + kcol0 + s * GM_KS + 8 * sc) : make_uint4(0, 0, 0, 0);
+#pragma unroll
+        for (int i = 0; i < NW; i++) r.w[i] = *(const uint4*)(wrow + (size_t)(32 * i) * K + s * GM_KS);
+    };
+    auto store_stage = [&](const GwStage& r) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < NW; i++) *(uint4*)&wl[32 * i * GM_KS + sto] = r.w[i];
+#pragma unroll
+        for (int q = 0; q < 2; q++) {
+            float v[8] = {r.x[q][0].x, r.x[q][0].y, r.x[q][0].z, r.x[q][0].w,
+                          r.x[q][1].x, r.x[q][1].y, r.x[q][1].z, r.x[q][1].w};
+            if (NORM) {
+#pragma unroll
+                for (int e = 0; e < 8; e++) ss[q] = __builtin_fmaf(v[e], v[e], ss[q]);
+                const uint32_t nn[4] = {r.nw.x, r.nw.y, r.nw.z, r.nw.w};
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    v[2 * e] = __fmul_rn(v[2 * e], bf16_bits_to_f32(nn[e] & 0xFFFFu));
+                    v[2 * e + 1] = __fmul_rn(v[2 * e + 1], bf16_bits_to_f32(nn[e] >> 16));
+                }
+            }
+            uint32_t hi[4], lo[4];
+#pragma unroll
+            for (int e = 0; e < 4; e++) split_bf16x2(v[2 * e], v[2 * e + 1], hi[e], lo[e]);
+            const unsigned keep = live[q] ? 0xFFFFFFFFu : 0u;     // tokens past B stage zeros
+            *(uint4*)&xh[32 * q * GM_KS + sto] = make_uint4(hi[0] & keep, hi[1] & keep, hi[2] & keep, hi[3] & keep);
+            *(uint4*)&xl[32 * q * GM_KS + sto] = make_uint4(lo[0] & keep, lo[1] & keep, lo[2] & keep, lo[3] & keep);
+        }
+    };
+
+    const int wn0 = 64 * w;                       // this wave's first weight row within the block's tile
+    floatx16 acc[2][2] = {};
+    auto mfma_stage = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int k2 = 0; k2 < GM_KS / 16; k2++) {
+            const int off = gw_at(lane & 31, 2 * k2 + (lane >> 5));     // (rows 32 apart rotate alike)
+            bf16x8 ah[2], al[2], b[2];
+#pragma unroll
+            for (int i = 0; i < 2; i++) {
+                ah[i] = *(const bf16x8*)&xh[32 * i * GM_KS + off];
+                al[i] = *(const bf16x8*)&xl[32 * i * GM_KS + off];
+            }
+#pragma unroll
+            for (int j = 0; j < 2; j++) b[j] = *(const bf16x8*)&wl[(wn0 + 32 * j) * GM_KS + off];
+#pragma unroll
+            for (int i = 0; i < 2; i++)
+#pragma unroll
+                for (int j = 0; j < 2; j++)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah[i], b[j], acc[i][j], 0, 0, 0);
+#pragma unroll
+            for (int i = 0; i < 2; i++)
+#pragma unroll
+                for (int j = 0; j < 2; j++)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(al[i], b[j], acc[i][j], 0, 0, 0);
+        }
+    };
+    // stage s + 1 streams into registers while stage s (in LDS) is multiplied
+    GwStage r;
+    load_stage(r, 0);
+    for (int s = 0; s < nstage; s++) {
+        store_stage(r);
+        load_stage(r, s + 1);
+        __syncthreads();
+        mfma_stage();
+        __syncthreads();
+    }
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+#pragma unroll
+        for (int v = 0; v < 16; v++) {
+            const int t = tb0 + 32 * i + 8 * (v / 4) + 4 * (lane >> 5) + (v % 4);
+            if (t >= a.B) continue;
+            float* out = a.part + ((size_t)kz * a.B + t) * a.N + row0 + wn0 + (lane & 31);
+#pragma unroll
+            for (int j = 0; j < 2; j++) out[32 * j] = acc[i][j][v];
+        }
+    if (NORM && want_ss) {
+#pragma unroll
+        for (int q = 0; q < 2; q++) ss_l[sr + 32 * q][sc] = ss[q];
+        __syncthreads();
+        if (tid < GM_T && tb0 + tid < a.B) {
+            float t = 0.0f;
+#pragma unroll
+            for (int i = 0; i < 8; i++) t = __fadd_rn(t, ss_l[tid][i]);
+            a.rss[(size_t)kz * a.B + tb0 + tid] = t;
+        }
+    }
+}
+
 bool gemm_shape_ok(const GemvArgs& a) {
     return a.K % (2 * GM_KS) == 0 && a.rows[0] % GM_R == 0 && a.rows[1] % GM_R == 0 && a.rows[2] % GM_R == 0;
 }
@@ -309,13 +467,13 @@ static int device_cus() {
     return ncu;
 }
 
-// Column ranges (K slices) of the GEMM, 1, 2 or 4: one block per CU runs at
+// Column ranges (K slices) of k_gemm_bf16, 1, 2 or 4: one block per CU runs at
 // a time, so a grid of (N / 128) x (B / 64) tiles that leaves CUs idle in
 // its last round is split along K into more, shorter blocks.  Time is
 // modelled as rounds x (1 / slices + 0.15), the constant a block's fixed
 // part (prologue, output stores); ties keep fewer slices (fewer partial
 // outputs to write and sum).
-int gemm_slices(const GemvArgs& a) {
+static int gemm_slices_narrow(const GemvArgs& a) {
     const int ncu = device_cus();
     const long long tiles = (long long)(a.N / GM_R) * ((a.B + GM_T - 1) / GM_T);
     const int nstage = a.K / GM_KS;
@@ -333,11 +491,50 @@ int gemm_slices(const GemvArgs& a) {
     return best;
 }
 
+// Which kernel takes a, and in how many column ranges.  Both are priced in
+// microseconds as they measured here, for the 64-column stages of a block and
+// the blocks a CU gets: k_gemm_bf16 0.74 per stage and 3 per block, one block
+// at a time; the wide tile 2.05 per stage of two blocks sharing a CU or 1.25
+// of one alone, 8 per such round and 4 once.  Each further slice is written
+// and read again at about 5 TB/s.  The wide tile has to be 5% ahead: measured
+// where it is not, us narrow vs wide, 512 tokens 5120 x 2048 39 vs 41 and 2048
+// x 4096 28 vs 33.
+struct GemmPlan {
+    bool wide;
+    int kz;
+};
+
+static GemmPlan gemm_plan(const GemvArgs& a) {
+    const int ncu = device_cus(), tt = (a.B + GM_T - 1) / GM_T, nstage = a.K / GM_KS;
+    GemmPlan p{false, gemm_slices_narrow(a)};
+    // (the wide kernel sums squares only where it applies a norm weight)
+    if (a.rows[0] % GW_R != 0 || a.rows[1] % GW_R != 0 || a.rows[2] % GW_R != 0 || (a.rss && !a.norm_w)) return p;
+    const double slice = (double)a.B * a.N * 4 / 5e6;
+    const long long nb = ((long long)(a.N / GM_R) * tt * p.kz + ncu - 1) / ncu;
+    double best = 0.95 * ((double)nb * (0.74 * nstage / p.kz + 3.0) + slice * p.kz);
+    for (int kz : {1, 2, 4}) {
+        if (nstage % (2 * kz) != 0) continue;
+        const long long n = ((long long)(a.N / GW_R) * tt * kz + ncu - 1) / ncu;
+        const double t = (double)nstage / kz * (2.05 * (n / 2) + 1.25 * (n % 2)) + 8.0 * ((n + 1) / 2) + 4.0 + slice * kz;
+        if (t < best) {
+            best = t;
+            p = {true, kz};
+        }
+    }
+    return p;
+}
+
+int gemm_slices(const GemvArgs& a) { return gemm_plan(a).kz; }
+
 hipError_t launch_gemm_bf16(const GemvArgs& a, hipStream_t st) {
     if (a.B == 0 || a.N == 0) return hipSuccess;
     if (!gemm_shape_ok(a)) return hipErrorInvalidValue;
-    const dim3 grid((unsigned)(a.N / GM_R), (unsigned)((a.B + GM_T - 1) / GM_T), (unsigned)gemm_slices(a));
-    hipLaunchKernelGGL(k_gemm_bf16, grid, dim3(512), 0, st, a);
+    const GemmPlan p = gemm_plan(a);
+    const int rb = p.wide ? GW_R : GM_R;
+    const dim3 grid((unsigned)(a.N / rb), (unsigned)((a.B + GM_T - 1) / GM_T), (unsigned)p.kz);
+    if (!p.wide) hipLaunchKernelGGL(k_gemm_bf16, grid, dim3(512), 0, st, a);
+    else if (a.norm_w) hipLaunchKernelGGL(k_gemm_bf16_wide<true>, grid, dim3(256), 0, st, a);
+    else hipLaunchKernelGGL(k_gemm_bf16_wide<false>, grid, dim3(256), 0, st, a);
     return hipGetLastError();
 }
 
