@@ -67,7 +67,7 @@ ROOT = Path(__file__).resolve().parent
 sys.path.insert(0, str(ROOT))
 
 PEAK_HBM_GBS = 8000.0
-PEAK_MFMA_I8_TOPS = 5000.0     # dense int8 MFMA (the dense branch's operands)
+PEAK_MFMA_I8_TOPS = 5000.0     # dense int8 MFMA, the yardstick of mfma_frac_of_int8_peak (the operands are 6-bit floats)
 ZIPF_ALPHA = 0.28              # Zipf(1.1) bias strength: per-expert counts about 5..200 over 512 tokens
 
 # HBM traffic of the block's kernels: two rocprofv3 --pmc runs of this
@@ -657,7 +657,7 @@ def plugin_q4_gemm(group, m=768, d=2048, sizes=(1, 2, 4, 6, 7, 8, 12, 16, 20, 24
     at each token count T (inputs and the packed matrix resident on the GPU;
     the workspace cached after the first call), with the library's own
     choice of kernel and with each of the two kernels forced (the v_dot8
-    digit kernel, the int8 matrix cores), from which the crossover is read.
+    digit kernel, the matrix cores), from which the crossover is read.
 
     `us_per_call` is the GPU's time per call: a bounded spin kernel
     (torch.cuda._sleep) holds the stream while the host enqueues the `reps`

@@ -125,7 +125,7 @@ int jm_store_set_dense_min(jm_store* s, int min_tokens);
  * group's largest magnitude / R, R = 30583 for 4 digits, 489335 for 5).  4
  * (the default; 0 restores it) keeps about 15 bits per group, 5 about 19 bits
  * at more dot products per row.  Router indices and weights do not depend on
- * it.  The MFMA branch's int8 digit pairs are not affected.  No counterpart in
+ * it.  The MFMA branch's digit planes are not affected.  No counterpart in
  * the reference, whose activations are float32. */
 int jm_store_set_act_digits(jm_store* s, int ndig);
 /* The store's digit planes (4 or 5), -1 for a NULL store. */
@@ -434,7 +434,7 @@ int jm_q4_gemv_f32(float* out, const float* x, const uint8_t* packed, const uint
 
 /* out[T][m] = X[T][d] . dequant(W[m][d])^T; argument order of q4_gemm_f32
  * (expert_ffn.c:201) plus the stream.  From jm_get_q4_gemm_min_tokens()
- * tokens the product runs on the int8 matrix cores (when m, d and group
+ * tokens the product runs on the matrix cores (when m, d and group
  * allow it and scales is 16-byte aligned; when its 32-token tiles x 256-row
  * blocks are fewer than 256, the contraction is split over up to 8 blocks
  * and the partial sums are added in split order), below on the v_dot8 digit

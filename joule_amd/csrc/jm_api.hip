@@ -780,8 +780,8 @@ int jm_q4_gemm_f32(float* out, const float* X, int T, const uint8_t* packed, con
     if (!aligned(packed, 16) || !aligned(X, 16)) return fail(JM_ERR_ARG, "packed and X must be 16-byte aligned");
     if (T == 0 || m == 0) return 0;
     hipStream_t st = (hipStream_t)stream;
-    // from jm_set_q4_gemm_min_tokens tokens on the matrix cores (int8 digit
-    // pairs of X)
+    // from jm_set_q4_gemm_min_tokens tokens on the matrix cores (fp6 digit
+    // planes of X)
     const bool mfma = T >= g_q4_gemm_min_t.load(std::memory_order_relaxed) && jm::q4_gemm_mfma_ok(m, d, group) &&
                       aligned(scales, 16);
     const size_t ng = (size_t)d / group;
