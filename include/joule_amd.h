@@ -114,7 +114,7 @@ int jm_store_info(const jm_store* s, int* L, int* E, int* d, int* m, int* topk, 
  * slots takes the MFMA branch (32-token tiles on the fp6 matrix cores: the
  * nibbles q against each activation's four base-16 digits), the others the
  * wave-item GEMV kernels.  0 restores the default (8, or 3 in calls with fewer
- * than 16 slots per expert); a value above B * topk keeps every expert on the
+ * than 16 slots per expert on a store with 4 digit planes); a value above B * topk keeps every expert on the
  * GEMV kernels.  No counterpart in the
  * reference, whose batch is at most 16 tokens (decode_kernel.c:1522). */
 int jm_store_set_dense_min(jm_store* s, int min_tokens);

@@ -366,8 +366,10 @@ int ffn_enqueue(jm_store* s, int layer, const float* x, int B, float* out, const
     r.first_slot = w.first_slot; r.comb = w.comb;
     r.work = w.work; r.umax = umax; r.rec = s->rec;
     r.key0 = (long long)layer * E;
-    const int dense_min = s->dense_min ? s->dense_min
-                        : nslot < JM_DENSE_FEW_SLOTS * E ? JM_DENSE_MIN_FEW : JM_DENSE_MIN_DEFAULT;
+    // (a store with 5 digit planes asked for more precision than the MFMA
+    // branch's records hold: its small experts stay on the wave items)
+    const bool few = nslot < JM_DENSE_FEW_SLOTS * E && s->ndig == JM_NDIG;
+    const int dense_min = s->dense_min ? s->dense_min : few ? JM_DENSE_MIN_FEW : JM_DENSE_MIN_DEFAULT;
     r.tiles = w.tiles; r.n_tiles = w.n_tiles; r.small = w.small;
     r.skip_topk = dec && jm::gateup_topk(B, E);
     r.ndig = s->ndig;

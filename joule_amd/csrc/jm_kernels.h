@@ -28,7 +28,7 @@
 // in tiles of this many tokens (fp6 matrix-core operands, jm_mx.h).
 #define JM_DENSE_TILE 32
 // By default (jm_store_set_dense_min): 8 slots, and 3 when a call has fewer
-// than 16 slots per expert, where the experts of 3 to 7 slots are many and
+// than 16 slots per expert (and the store 4 digit planes), where the experts of 3 to 7 slots are many and
 // their tokens one by one bound the call (their tiles cost the same HBM bytes
 // and a thirty-second of the work).  us per block at 3 vs 8, Qwen3 shape: 33
 // tokens 117.6 vs 118.9, 52 116.9 vs 153.9, 80 124.2 vs 177.0, 128 124.3 vs

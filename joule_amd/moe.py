@@ -154,7 +154,8 @@ class HbmExpertStore:
 
     def set_dense_min(self, min_tokens: int) -> None:
         """Segment size from which an expert takes the MFMA branch (batches
-        with more than 256 slots); 0 restores the default."""
+        with more than 256 slots); 0 restores the default: 8, or 3 in calls
+        with fewer than 16 slots per expert on a store with 4 digit planes."""
         _lib.check(_lib.lib().jm_store_set_dense_min(self._h, int(min_tokens)), "jm_store_set_dense_min")
 
     def set_act_digits(self, ndig: int) -> None:

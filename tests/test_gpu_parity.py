@@ -754,6 +754,34 @@ def test_block_five_digits_zipf_and_stages(qwen64):
     assert errs[5] <= 2e-5 and errs[5] * 4 <= errs[4]
 
 
+@pytest.mark.parametrize("B", [40, 128])
+def test_block_five_digits_default_threshold(qwen64, B):
+    """A store with 5 digits keeps every expert under 8 slots on the 5-digit
+    GEMV kernels at the default dense_min, also in batches with fewer than 16
+    slots per expert (where a 4-digit store's threshold is 3): the tokens
+    whose experts all have fewer than 8 slots keep test_block_five_digits' bar."""
+    layer, st = qwen64, qwen64.store
+    banner(f"five digits, default threshold B={B}")
+    x = activations(B, layer.shape.d, seed=5)
+    rout, rtop, _ = layer.oracle(0).forward(x, n_threads=8)
+    counts = np.bincount(rtop.ravel(), minlength=layer.shape.E)
+    tiles = {}
+    for nd, least in ((4, 3), (5, 8)):
+        try:
+            st.set_act_digits(nd)
+            out, top, _ = _run_block(layer, 0, x)
+            tiles[nd] = st.dense_tiles()
+        finally:
+            st.set_act_digits(0)
+        assert np.array_equal(top, rtop)
+        assert tiles[nd] == int(((counts + TILE - 1) // TILE)[counts >= least].sum())
+    light = (counts[rtop] < 8).all(axis=1)        # (at B=128 every token meets an expert of 8 slots)
+    assert light.all() or B == 128
+    err = _rel(out[light], rout[light]) if light.any() else 0.0
+    print(f"  tiles {tiles}, {int(light.sum())} tokens without a tile: normwise {err:.3e}", flush=True)
+    assert err <= 2e-5
+
+
 def test_act_digits_setting_errors(qwen64):
     banner("act digits setting")
     st = qwen64.store
