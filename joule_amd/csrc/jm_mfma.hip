@@ -20,8 +20,11 @@
 // (64 columns') sums already scaled per token; per element the epilogue is
 // one multiply-add by the row's group scale:
 //   acc += P * s_row
-// on top of the -8 of the Q4 code, for all groups at once: a product of
-// the tokens' group corrections (three bf16 terms) and the row scales (two).
+// The -8 of the Q4 code is what a group's sum starts from: the tokens' group
+// corrections, three bf16 terms each, spread over the columns by a product
+// with ones.  Added to the largest digits first, a group's partial sums need
+// no more bits than float32 has (see group_mfma), so tokens of one sign lose
+// nothing to the cancellation.
 //
 // A wave takes 32 tokens x 64 weight rows (two 32-row blocks, which share the
 // token operands), a block 4 waves; two blocks share a CU and stay for several
@@ -72,7 +75,7 @@ constexpr int RING = 4 * 6 * PIECE; // LDS bytes of a super-stage's token operan
 // compiler sees that reading one does not wait for the loads into another.
 struct Rings {
     uint8_t* r[3];      // the third for an odd count of super-stages
-    uint8_t* corr;      // [steps][3][PIECE] the unit's correction operands
+    uint8_t* corr;      // the unit's group corrections (CorrTok)
 };
 
 // Where a wave's product's operands come from: K columns in nss super-stages,
@@ -169,90 +172,58 @@ __device__ __forceinline__ void stage_tokens(const Operands& op, int S, uint8_t*
     }
 }
 
-// The unit's group corrections on their way to LDS (three bf16 terms each, in
-// the operand order of the correction product): wave w holds steps w, w + 4,
-// ... of 16 groups, lane l groups 16 st + 8 (l / 32) .. + 7 of token l % 32.
-template <int CSTEPS>
+// The unit's group corrections on their way to LDS, three bf16 terms each
+// (exact: 24 bits).  Thread t holds blocks t / 32 + 8 r of 4 groups of token
+// t % 32; in LDS [block][term][token][4 groups].
+constexpr int CBLOCK = 3 * MT * 8;                // LDS bytes of a block of 4 groups
+template <int CR>
 struct CorrTok {
-    static_assert(CSTEPS <= NWAVE, "a step per wave");
-    float4 c[2];
+    float4 c[CR];
     __device__ __forceinline__ void load(const float* corr, int ng) {
-        const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
 #pragma unroll
-        for (int q = 0; q < 2; q++) {
-            const int g = 16 * w + 8 * (l >> 5) + 4 * q;
-            c[q] = *(const float4*)(corr + (g < ng ? g : 0));
+        for (int r = 0; r < CR; r++) {
+            const int b = (threadIdx.x >> 5) + 8 * r;
+            c[r] = *(const float4*)(corr + (4 * b < ng ? 4 * b : 0));
         }
     }
     __device__ __forceinline__ void store(int ng, uint8_t* cl) const {
-        const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
-        if (16 * w >= ng) return;
-        uint32_t t[3][4];
 #pragma unroll
-        for (int q = 0; q < 2; q++) {
-            const bool in = 16 * w + 8 * (l >> 5) + 4 * q < ng;
-            const float v[4] = {in ? c[q].x : 0.0f, in ? c[q].y : 0.0f, in ? c[q].z : 0.0f, in ? c[q].w : 0.0f};
+        for (int r = 0; r < CR; r++) {
+            const int b = (threadIdx.x >> 5) + 8 * r;
+            if (4 * b >= ng) continue;
+            const float v[4] = {c[r].x, c[r].y, c[r].z, c[r].w};
+            uint32_t t[3][2];
 #pragma unroll
             for (int e = 0; e < 2; e++) {
-                const float a = v[2 * e], b = v[2 * e + 1];
-                uint32_t hi, lo;
-                split_bf16x2(a, b, hi, lo);
-                t[0][2 * q + e] = hi;
-                t[1][2 * q + e] = lo;
-                t[2][2 * q + e] = pack_bf16x2(
-                    __fsub_rn(__fsub_rn(a, __uint_as_float(hi << 16)), __uint_as_float(lo << 16)),
-                    __fsub_rn(__fsub_rn(b, __uint_as_float(hi & 0xFFFF0000u)), __uint_as_float(lo & 0xFFFF0000u)));
+                const float x = v[2 * e], y = v[2 * e + 1];
+                split_bf16x2(x, y, t[0][e], t[1][e]);
+                // (half the third term: its lanes meet two ones)
+                t[2][e] = pack_bf16x2(
+                    __fmul_rn(0.5f, __fsub_rn(__fsub_rn(x, __uint_as_float(t[0][e] << 16)), __uint_as_float(t[1][e] << 16))),
+                    __fmul_rn(0.5f, __fsub_rn(__fsub_rn(y, __uint_as_float(t[0][e] & 0xFFFF0000u)),
+                                              __uint_as_float(t[1][e] & 0xFFFF0000u))));
             }
+#pragma unroll
+            for (int k = 0; k < 3; k++)
+                *(uint2*)(cl + b * CBLOCK + (k * MT + (threadIdx.x & 31)) * 8) = make_uint2(t[k][0], t[k][1]);
         }
-#pragma unroll
-        for (int k = 0; k < 3; k++)
-            *(uint4*)(cl + (3 * w + k) * PIECE + 16 * l) = make_uint4(t[k][0], t[k][1], t[k][2], t[k][3]);
     }
 };
 
-// The row scales of one row block for the correction product: lane l groups
-// 16 st + 8 (l / 32) .. + 7 of row l % 32, steps st of 16 groups.
-template <int CSTEPS>
-struct CorrScales {
-    uint2 v[CSTEPS][2];
-    __device__ __forceinline__ void load(const Operands& op, const uint8_t* sc) {
-        const int l = threadIdx.x & 63;
-#pragma unroll
-        for (int st = 0; st < CSTEPS; st++)
-#pragma unroll
-            for (int q = 0; q < 2; q++) {
-                const int g = 16 * st + 8 * (l >> 5) + 4 * q;
-                v[st][q] = load_as<uint2>(lane_at(sc, (uint32_t)(l & 31) * op.srow + 2 * (g < op.ng ? g : 0)));
-            }
-    }
-};
-
-// acc += sum over the groups of correction x row scale
-template <int CSTEPS>
-__device__ __forceinline__ void add_corr(floatx16& acc, const Operands& op, const CorrScales<CSTEPS>& sc, const uint8_t* cl) {
+// A block's 4 groups as the operand of v_mfma_f32_32x32x16_bf16: lane half 0
+// the first and second terms, half 1 the third twice.
+__device__ __forceinline__ bf16x8 corr_operand(const uint8_t* cl, int b) {
     const int l = threadIdx.x & 63, h = l >> 5;
-#pragma unroll
-    for (int st = 0; st < CSTEPS; st++) {
-        if (16 * st >= op.ng) break;
-        uint32_t hi[4], lo[4];
-#pragma unroll
-        for (int q = 0; q < 2; q++) {
-            const bool in = 16 * st + 8 * h + 4 * q < op.ng;
-            const uint32_t x = in ? sc.v[st][q].x : 0u, y = in ? sc.v[st][q].y : 0u;
-            split_bf16x2(fp16_hw((uint16_t)x), fp16_hw((uint16_t)(x >> 16)), hi[2 * q], lo[2 * q]);
-            split_bf16x2(fp16_hw((uint16_t)y), fp16_hw((uint16_t)(y >> 16)), hi[2 * q + 1], lo[2 * q + 1]);
-        }
-        const bf16x8 wh = __builtin_bit_cast(bf16x8, make_uint4(hi[0], hi[1], hi[2], hi[3]));
-        const bf16x8 wl = __builtin_bit_cast(bf16x8, make_uint4(lo[0], lo[1], lo[2], lo[3]));
-        const bf16x8 c0 = __builtin_bit_cast(bf16x8, *(const uint4*)(cl + (3 * st + 0) * PIECE + 16 * l));
-        const bf16x8 c1 = __builtin_bit_cast(bf16x8, *(const uint4*)(cl + (3 * st + 1) * PIECE + 16 * l));
-        const bf16x8 c2 = __builtin_bit_cast(bf16x8, *(const uint4*)(cl + (3 * st + 2) * PIECE + 16 * l));
-        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(c2, wh, acc, 0, 0, 0);
-        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(c1, wl, acc, 0, 0, 0);
-        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(c1, wh, acc, 0, 0, 0);
-        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(c0, wl, acc, 0, 0, 0);
-        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(c0, wh, acc, 0, 0, 0);
-    }
+    const uint8_t* const p = cl + b * CBLOCK + (2 * h * MT + (l & 31)) * 8;
+    const uint2 x = *(const uint2*)p, y = *(const uint2*)(p + (h ? 0 : MT * 8));
+    return __builtin_bit_cast(bf16x8, make_uint4(x.x, x.y, y.x, y.y));
+}
+
+// The correction of group g of the block for every column: ones at both terms
+template <int GI>
+__device__ __forceinline__ floatx16 corr_init(const bf16x8& c) {
+    constexpr uint32_t one = GI & 1 ? 0x3F800000u : 0x3F80u, lo = GI < 2 ? one : 0u, hi = GI < 2 ? 0u : one;
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(c, __builtin_bit_cast(bf16x8, make_uint4(lo, hi, lo, hi)), floatx16{}, 0, 0, 0);
 }
 
 // Two dwords of each of the 4 sixteen-lane rows exchanged: x = rows (x0, x1,
@@ -310,47 +281,57 @@ __device__ __forceinline__ floatx16 mfma_f6(const int8v& a, const int8v& b, cons
     return __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a, b, c, 2, 2, SA, (int)sa, SB, (int)sb);
 }
 
-// One stage's products: P[rb][group] from the stage's token operands in LDS
-template <int G, int CS>
-__device__ __forceinline__ void stage_mfma(floatx16 (&P)[2][64 / G], const uint8_t* ring, const int8v (&b)[2][64 / G],
-                                           const typename WStage<G>::ExT& ex, uint32_t sb) {
-    // piece k, half h: chunk 12 CS + 2 k + h of token l % 32 (opaque: the
-    // addresses are made here instead of being kept in registers)
+// A piece of a stage's token operands in LDS, this lane's: piece k, half h is
+// chunk 12 CS + 2 k + h of token l % 32, at `at` for chunk h.
+template <int CS>
+__device__ __forceinline__ uint4 token_piece(const uint8_t* ring, uint32_t at, int k) {
+    const int c = 12 * CS + 2 * k;
+    return *(const uint4*)(ring + (c >> 4) * (32 * 256) + (at ^ (16 * (c & 15))));
+}
+
+// One group's products: P[rb] from the stage's token operands in LDS, on top
+// of the group's correction (corr: the operand of the block of 4 groups it
+// lies in).  The digits' planes come largest first: with |a| <= 65535 the
+// correction -8 sum(a) is a multiple of 8 under 2^25, the sums with the planes
+// of 16^3 and 16^2 stay multiples of 8 under 2^27, with the plane of 16 under
+// 2^26, all of which float32 holds; the last, sum a (q - 8), is rounded only
+// past 2^24.
+template <int G, int CS, int GI>
+__device__ __forceinline__ void group_mfma(floatx16 (&P)[2], const uint8_t* ring, const int8v& b0, const int8v& b1,
+                                           const typename WStage<G>::ExT& ex, uint32_t sb, const bf16x8& corr) {
+    // (opaque: the addresses are made here instead of being kept in registers)
     const int l = threadIdx.x & 63;
     uint32_t at = (l & 31) * 256 + 16 * ((l >> 5) ^ (l & 15));
     __asm__ volatile("" : "+v"(at));
-    uint4 p[6];
-#pragma unroll
-    for (int k = 0; k < 6; k++) {
-        const int c = 12 * CS + 2 * k;
-        p[k] = *(const uint4*)(ring + (c >> 4) * (32 * 256) + (at ^ (16 * (c & 15))));
-    }
-    const int8v a0 = {(int)p[0].x, (int)p[0].y, (int)p[0].z, (int)p[0].w, (int)p[4].x, (int)p[4].y, 0, 0};
-    const int8v a1 = {(int)p[1].x, (int)p[1].y, (int)p[1].z, (int)p[1].w, (int)p[4].z, (int)p[4].w, 0, 0};
-    const int8v a2 = {(int)p[2].x, (int)p[2].y, (int)p[2].z, (int)p[2].w, (int)p[5].x, (int)p[5].y, 0, 0};
-    const int8v a3 = {(int)p[3].x, (int)p[3].y, (int)p[3].z, (int)p[3].w, (int)p[5].z, (int)p[5].w, 0, 0};
+    // operands 2 o and 2 o + 1
+    const auto pair = [&](int o, int8v& x, int8v& y) __attribute__((always_inline)) {
+        const uint4 p = token_piece<CS>(ring, at, 2 * o), q = token_piece<CS>(ring, at, 2 * o + 1), r = token_piece<CS>(ring, at, 4 + o);
+        x = int8v{(int)p.x, (int)p.y, (int)p.z, (int)p.w, (int)r.x, (int)r.y, 0, 0};
+        y = int8v{(int)q.x, (int)q.y, (int)q.z, (int)q.w, (int)r.z, (int)r.w, 0, 0};
+    };
     if constexpr (G == 64) {
-#pragma unroll
-        for (int rb = 0; rb < 2; rb++) P[rb][0] = mfma_f6<CS, 0>(a0, b[rb][0], floatx16{}, ex, sb);
-#pragma unroll
-        for (int rb = 0; rb < 2; rb++) P[rb][0] = mfma_f6<CS, 1>(a1, b[rb][0], P[rb][0], ex, sb);
-#pragma unroll
-        for (int rb = 0; rb < 2; rb++) P[rb][0] = mfma_f6<CS, 2>(a2, b[rb][0], P[rb][0], ex, sb);
-#pragma unroll
-        for (int rb = 0; rb < 2; rb++) P[rb][0] = mfma_f6<CS, 3>(a3, b[rb][0], P[rb][0], ex, sb);
+        int8v a0, a1, a2, a3;
+        pair(1, a2, a3);
+        pair(0, a0, a1);
+        const floatx16 c = corr_init<CS>(corr);
+        P[0] = mfma_f6<CS, 3>(a3, b0, c, ex, sb);
+        P[1] = mfma_f6<CS, 3>(a3, b1, c, ex, sb);
+        P[0] = mfma_f6<CS, 2>(a2, b0, P[0], ex, sb);
+        P[1] = mfma_f6<CS, 2>(a2, b1, P[1], ex, sb);
+        P[0] = mfma_f6<CS, 1>(a1, b0, P[0], ex, sb);
+        P[1] = mfma_f6<CS, 1>(a1, b1, P[1], ex, sb);
+        P[0] = mfma_f6<CS, 0>(a0, b0, P[0], ex, sb);
+        P[1] = mfma_f6<CS, 0>(a0, b1, P[1], ex, sb);
     } else {
         const uint32_t e = CS < 2 ? ex.x : ex.y;
-        constexpr int B0 = 2 * (CS & 1);
-#pragma unroll
-        for (int rb = 0; rb < 2; rb++) {
-            P[rb][0] = mfma_f6<B0, 0>(a0, b[rb][0], floatx16{}, e, sb);
-            P[rb][1] = mfma_f6<B0 + 1, 0>(a2, b[rb][1], floatx16{}, e, sb);
-        }
-#pragma unroll
-        for (int rb = 0; rb < 2; rb++) {
-            P[rb][0] = mfma_f6<B0, 1>(a1, b[rb][0], P[rb][0], e, sb);
-            P[rb][1] = mfma_f6<B0 + 1, 1>(a3, b[rb][1], P[rb][1], e, sb);
-        }
+        constexpr int B0 = 2 * (CS & 1) + GI;
+        int8v a0, a1;
+        pair(GI, a0, a1);
+        const floatx16 c = corr_init<B0>(corr);
+        P[0] = mfma_f6<B0, 1>(a1, b0, c, e, sb);
+        P[1] = mfma_f6<B0, 1>(a1, b1, c, e, sb);
+        P[0] = mfma_f6<B0, 0>(a0, b0, P[0], e, sb);
+        P[1] = mfma_f6<B0, 0>(a0, b1, P[1], e, sb);
     }
 }
 
@@ -365,9 +346,9 @@ __device__ __forceinline__ void pin(floatx16 (&acc)[2]) {
     __asm__ volatile("" : "+v"(acc[0]), "+v"(acc[1]) : : "memory");
 }
 
-// 16-group steps of the correction product: of 256 or 768 columns for one or
-// three super-stages, else of up to KMAX
-constexpr int corr_steps(int G, int nss) { return ((nss ? nss * SSC : KMAX) / G + 15) / 16; }
+// blocks of 4 groups of a contraction: of 256 or 768 columns for one or three
+// super-stages, else of up to KMAX
+constexpr int corr_blocks(int G, int nss) { return (nss ? nss * SSC : KMAX) / G / 4; }
 
 // A wave's running state over a block's units (a unit: one token tile against
 // the block's rows): the operands of the unit being computed and the next
@@ -376,27 +357,13 @@ template <int G, int NSS>
 struct Pipe {
     using W = WStage<G>;
     static constexpr int NG = 64 / G;
-    static constexpr int CSTEPS = corr_steps(G, NSS);
-    // the correction's scales are kept from the unit before, or (more than
-    // the registers hold) read when they are needed
-    static constexpr bool CS_AHEAD = CSTEPS <= 2;
     W w;
     floatx16 acc[2];
-    CorrScales<CSTEPS> cs[2];
-    CorrTok<CSTEPS> ct;
-
-    // the next unit's corrections on their way
-    __device__ __forceinline__ void next_corr(const Operands& op, const float* corr) {
-        if constexpr (CS_AHEAD) {
-#pragma unroll
-            for (int rb = 0; rb < 2; rb++) cs[rb].load(op, op.sc[rb]);
-        }
-        ct.load(corr, op.ng);
-    }
+    CorrTok<(corr_blocks(G, NSS) + 7) / 8> ct;
 
     // the first unit's operands
     __device__ __forceinline__ void start(const Operands& op, const Rings& rg, const float* corr) {
-        next_corr(op, corr);
+        ct.load(corr, op.ng);
         stage_tokens(op, 0, rg.r[0]);
         w.load_half(op, 0, 0);
         w.load_half(op, 0, 1);
@@ -404,11 +371,11 @@ struct Pipe {
         ct.store(op.ng, rg.corr);
     }
 
-    // Super-stage S from `ring`; the next one's operands (nop's super-stage
-    // nS) are requested into nring and the weight registers.  hook() runs
-    // once every wave's operands of S are there.
+    // Super-stage S from `ring` (its corrections at cl); the next one's
+    // operands (nop's super-stage nS) are requested into nring and the weight
+    // registers.  hook() runs once every wave's operands of S are there.
     template <class Hook>
-    __device__ __forceinline__ void step(const uint8_t* ring, uint8_t* nring, Hook&& hook) {
+    __device__ __forceinline__ void step(const uint8_t* ring, const uint8_t* cl, uint8_t* nring, Hook&& hook) {
         const uint32_t h = (threadIdx.x >> 5) & 1;
         // the planes' scales: 2^6 for the two operands' eighths, times 16^plane
         const uint32_t sb = G == 64 ? 0x918D8985u : h ? 0x9189u : 0x8D85u;
@@ -426,14 +393,19 @@ struct Pipe {
         __builtin_amdgcn_sched_barrier(0);
         const typename W::ScT sc[2] = {w.sc[0], w.sc[1]};
         const typename W::ExT ex = w.ex;
+        bf16x8 corr = corr_operand(cl, 0);
         auto stage = [&](auto cs_, const int8v (&b)[2][NG]) __attribute__((always_inline)) {
             constexpr int CS = decltype(cs_)::value;
-            floatx16 P[2][NG];
-            stage_mfma<G, CS>(P, ring, b, ex, sb);
-#pragma unroll
-            for (int rb = 0; rb < 2; rb++)
-#pragma unroll
-                for (int g = 0; g < NG; g++) group_acc(acc[rb], P[rb][g], sc_at<G>(sc[rb], NG * CS + g));
+            if (G == 32 && CS == 2) corr = corr_operand(cl, 1);
+            floatx16 P[2];
+            group_mfma<G, CS, 0>(P, ring, b[0][0], b[1][0], ex, sb, corr);
+            group_acc(acc[0], P[0], sc_at<G>(sc[0], NG * CS));
+            group_acc(acc[1], P[1], sc_at<G>(sc[1], NG * CS));
+            if constexpr (G == 32) {
+                group_mfma<G, CS, 1>(P, ring, b[0][1], b[1][1], ex, sb, corr);
+                group_acc(acc[0], P[0], sc_at<G>(sc[0], NG * CS + 1));
+                group_acc(acc[1], P[1], sc_at<G>(sc[1], NG * CS + 1));
+            }
         };
         auto half = [&](auto u) __attribute__((always_inline)) {
             constexpr int U = decltype(u)::value;
@@ -447,6 +419,7 @@ struct Pipe {
                 __builtin_amdgcn_sched_barrier(0);
                 const int8v b0[2][NG] = {{t0[0]}, {t1[0]}}, b1[2][NG] = {{t0[1]}, {t1[1]}};
                 stage(std::integral_constant<int, 2 * U>{}, b0);
+                pin(acc);                     // (one stage's operands at a time: registers)
                 stage(std::integral_constant<int, 2 * U + 1>{}, b1);
                 pin(acc);
             } else {
@@ -475,38 +448,35 @@ struct Pipe {
     // loads): they find the next unit and fill in its operands.
     template <class Early, class Late>
     __device__ __forceinline__ void unit(const Operands& op, Operands& nop, const Rings& rg, Early&& early, Late&& late) {
+        constexpr int CSS = SSC / G / 4 * CBLOCK;     // LDS bytes of a super-stage's corrections
         auto first = [&]() __attribute__((always_inline)) {
-#pragma unroll
-            for (int rb = 0; rb < 2; rb++) {
-                if constexpr (!CS_AHEAD) cs[rb].load(op, op.sc[rb]);
-                acc[rb] = floatx16{};
-                add_corr(acc[rb], op, cs[rb], rg.corr);
-            }
+            acc[0] = floatx16{};
+            acc[1] = floatx16{};
             early();
         };
         if constexpr (NSS == 1) {
-            step(rg.r[0], nullptr, [&](int& nS) __attribute__((always_inline)) -> Operands {
+            step(rg.r[0], rg.corr, nullptr, [&](int& nS) __attribute__((always_inline)) -> Operands {
                 first();
                 late(nop);
                 nS = 0;
                 return nop;
             });
-            wave_meet();                      // every wave is done with the only buffer
+            wave_meet();                      // every wave is done with the only buffer and the corrections
             stage_tokens(nop, 0, rg.r[0]);
         } else if constexpr (NSS == 3) {
-            step(rg.r[0], rg.r[1], [&](int& nS) __attribute__((always_inline)) -> Operands { first(); nS = 1; return op; });
-            step(rg.r[1], rg.r[2], [&](int& nS) __attribute__((always_inline)) -> Operands { late(nop); nS = 2; return op; });
-            step(rg.r[2], rg.r[0], [&](int& nS) __attribute__((always_inline)) -> Operands { nS = 0; return nop; });
+            step(rg.r[0], rg.corr, rg.r[1], [&](int& nS) __attribute__((always_inline)) -> Operands { first(); nS = 1; return op; });
+            step(rg.r[1], rg.corr + CSS, rg.r[2], [&](int& nS) __attribute__((always_inline)) -> Operands { late(nop); nS = 2; return op; });
+            step(rg.r[2], rg.corr + 2 * CSS, rg.r[0], [&](int& nS) __attribute__((always_inline)) -> Operands { nS = 0; return nop; });
         } else {
 #pragma unroll 1
             for (int S = 0; S < op.nss; S += 2) {
-                step(rg.r[0], rg.r[1], [&](int& nS) __attribute__((always_inline)) -> Operands {
+                step(rg.r[0], rg.corr + S * CSS, rg.r[1], [&](int& nS) __attribute__((always_inline)) -> Operands {
                     if (S == 0) first();
                     nS = S + 1;
                     return op;
                 });
                 const bool last = S + 2 == op.nss;
-                step(rg.r[1], rg.r[0], [&](int& nS) __attribute__((always_inline)) -> Operands {
+                step(rg.r[1], rg.corr + (S + 1) * CSS, rg.r[0], [&](int& nS) __attribute__((always_inline)) -> Operands {
                     if (S == 0) late(nop);
                     nS = last ? 0 : S + 2;
                     return last ? nop : op;
@@ -614,7 +584,7 @@ __global__ void __launch_bounds__(MTHREADS, 2)
 k_gateup_mfma(ExpertArgs a) {
     __shared__ __align__(16) uint8_t ring0[RING];
     __shared__ __align__(16) uint8_t ring1[RING];
-    __shared__ __align__(16) uint8_t corr_l[corr_steps(G, 0) * 3 * PIECE];
+    __shared__ __align__(16) uint8_t corr_l[corr_blocks(G, 0) * CBLOCK];
     __shared__ __align__(16) float act[MT * ACT_RP];
     const Rings rg{{ring0, ring1, nullptr}, corr_l};
     const int nrb = a.m / GU_ROWS, nb = gridDim.x;
@@ -639,10 +609,10 @@ k_gateup_mfma(ExpertArgs a) {
                     sn = tile_slot(a, tn);
                 },
                 [&](Operands& o) __attribute__((always_inline)) { gateup_op<G>(o, a, tn, un % nrb, sn); });
-            p.next_corr(nop, a.xc + (size_t)(sn / a.topk) * nop.ng);
+            p.ct.load(a.xc + (size_t)(sn / a.topk) * nop.ng, nop.ng);
             gateup_out<G>(a, p.acc, ti, u % nrb, sl, act);
             if (un == u) break;
-            p.ct.store(nop.ng, corr_l);
+            p.ct.store(nop.ng, corr_l);           // (every wave met in gateup_out, past its last read of the old ones)
             u = un;
             ti = tn;
             sl = sn;
@@ -707,7 +677,7 @@ k_down_mfma(ExpertArgs a) {
     __shared__ __align__(16) uint8_t ring0[RING];
     __shared__ __align__(16) uint8_t ring1[NSS == 1 ? 16 : RING];
     __shared__ __align__(16) uint8_t ring2[NSS == 3 ? RING : 16];
-    __shared__ __align__(16) uint8_t corr_l[corr_steps(G, NSS) * 3 * PIECE];
+    __shared__ __align__(16) uint8_t corr_l[corr_blocks(G, NSS) * CBLOCK];
     const Rings rg{{ring0, ring1, ring2}, corr_l};
     const int nrb = a.d / DN_ROWS, nb = gridDim.x;
     int u = blockIdx.x;
@@ -733,9 +703,10 @@ k_down_mfma(ExpertArgs a) {
                 },
                 [&](Operands& o) __attribute__((always_inline)) { down_op<G>(o, a, tn, un % nrb, sn); });
             const float twn = a.tw[sn];
-            p.next_corr(nop, a.ac + (size_t)sn * nop.ng);
+            p.ct.load(a.ac + (size_t)sn * nop.ng, nop.ng);
             down_out(a, p.acc, ti, u % nrb, sl, tw);
             if (un == u) break;
+            if (NSS != 1) wave_meet();            // every wave has read the unit's corrections
             p.ct.store(nop.ng, corr_l);
             u = un;
             ti = tn;
@@ -767,7 +738,7 @@ k_q4_gemm_mfma(const uint8_t* __restrict__ packed, const uint16_t* __restrict__ 
     __shared__ __align__(16) uint8_t ring0[RING];
     __shared__ __align__(16) uint8_t ring1[NSS == 1 ? 16 : RING];
     __shared__ __align__(16) uint8_t ring2[NSS == 3 ? RING : 16];
-    __shared__ __align__(16) uint8_t corr_l[corr_steps(G, NSS) * 3 * PIECE];
+    __shared__ __align__(16) uint8_t corr_l[corr_blocks(G, NSS) * CBLOCK];
     const Rings rg{{ring0, ring1, ring2}, corr_l};
     const int tid = threadIdx.x, lane = tid & 63;
     const int w = scalar(tid >> 6);

@@ -10,9 +10,9 @@
 // a_j = rint(x_j / 2^E), |a_j| <= 65535, with E the smallest exponent that
 // allows it: the step is at most max|x| / 32767.  The 4 digits of a_j go to 4
 // planes; the products of a plane are scaled by 2^E 16^plane in the matrix
-// core (E8M0 block scales), so that 4 accumulating instructions give
-// sum_j a_j q_j 2^E in float32.  The -8 of the Q4 code is added once per row
-// and token as sum over the groups of (-8 sum_j a_j 2^E) x row scale.
+// core (E8M0 block scales), so that 4 accumulating instructions, starting from
+// the group's correction -8 sum_j a_j 2^E (the -8 of the Q4 code), give
+// sum_j a_j (q_j - 8) 2^E in float32.
 //
 // Lane layout (checked on the device): A[i][k] at lane i % 32, B[k][n] at
 // lane n % 32, k = 32 (l / 32) + j, field j at bit 6 j of 6 dwords; D
@@ -40,8 +40,8 @@ typedef float floatx16 __attribute__((ext_vector_type(16)));
 
 constexpr int F6_STAGE = 192;           // record bytes per 64 columns
 
-// bytes of the records of `rows` rows of K columns, of their exponents and
-// of their group corrections
+// bytes of the records of `rows` rows of K columns (their exponents and group
+// corrections are arrays of their own, one value per group)
 __host__ __device__ constexpr size_t f6_rec_bytes(size_t rows, int K) { return rows * (size_t)K * 3; }
 
 // 16 nibbles (w: values 0..7, v: values 8..15, value i in bits 4 i) as 16

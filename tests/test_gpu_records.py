@@ -1,0 +1,74 @@
+"""The matrix-core product on digit planes (jm_mx.h, jm_mfma.hip) against
+float64, through the plugin product: its sums, its encoding and its range.
+
+Shapes: 2048 columns split over 8 blocks of one super-stage (256 columns) and
+unsplit, 768 columns unsplit (three super-stages) and split, 512 unsplit; Q4
+groups of 64 and 32; a ragged last token tile."""
+
+import numpy as np
+import pytest
+import torch
+
+from conftest import banner
+from joule_amd import q4_store as Q
+from joule_amd.backend import HipBackend
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [(768, 2048, 40), (8192, 2048, 257), (8192, 768, 257), (2048, 768, 33), (4096, 512, 513)]
+
+
+class Product:
+    """One random Q4 matrix on the GPU, its nibbles and scales in float64."""
+
+    def __init__(self, m, d, group, seed=0):
+        g = torch.Generator(device="cuda")
+        g.manual_seed(1000 * group + m + d + seed)
+        self.m, self.d, self.group = m, d, group
+        self.packed = torch.randint(0, 256, (m * d // 2,), generator=g, device="cuda", dtype=torch.uint8)
+        self.scales = (torch.rand(m * d // group, generator=g, device="cuda") * 0.01 + 0.002).to(torch.float16)
+        n = self.packed.cpu().numpy()
+        sc = self.scales.cpu().numpy().view(np.uint16)
+        self.W = torch.from_numpy(Q.dequantize(sc, n, m * d, group).reshape(m, d)).cuda().double()
+
+    def __call__(self, X):
+        out = torch.empty((X.shape[0], self.m), device="cuda")
+        HipBackend().q4_gemm(out, X.contiguous(), self.packed, self.scales.view(torch.int16), self.m, self.d, self.group)
+        torch.cuda.synchronize()
+        return out
+
+    def terms(self, X):
+        """[groups, T, m] the groups' exact contributions."""
+        T, ng = X.shape[0], self.d // self.group
+        x = X.double().view(T, ng, self.group).transpose(0, 1)
+        w = self.W.view(self.m, ng, self.group).permute(1, 2, 0)
+        return torch.stack([x[g] @ w[g].contiguous() for g in range(ng)])
+
+
+@pytest.mark.parametrize("group", [64, 32])
+@pytest.mark.parametrize("m,d,T", SHAPES)
+@pytest.mark.parametrize("sign", ["one", "mixed"])
+def test_sums_round_like_float32(gpu, m, d, T, group, sign):
+    """Integer tokens of 15 bits, which the encoding holds exactly, so that
+    only the sums round.  Bound per element: a group's sum is rounded at most
+    twice (the last plane, the scale's multiply-add) and a running sum over
+    consecutive groups once per group and per column split (at most 8):
+    2^-24 (2 sum |term| + (groups + 8) R), R the largest sum over consecutive
+    groups.  Tokens of one sign need the -8 of the nibbles inside the groups:
+    taken once for all groups, the running sum is up to 100 R."""
+    banner(f"records sums {m}x{d} T={T} G={group} {sign}")
+    p = Product(m, d, group)
+    g = torch.Generator(device="cuda")
+    g.manual_seed(3)
+    X = torch.randint(28000, 32768, (T, d), generator=g, device="cuda").float()
+    if sign == "mixed":
+        X = X * (torch.randint(0, 2, (T, d), generator=g, device="cuda") * 2 - 1)
+    X = X / 32768
+    got = p(X)
+    t = p.terms(X)
+    pre = torch.cat([torch.zeros_like(t[:1]), t.cumsum(0)])
+    R = pre.amax(0) - pre.amin(0)
+    bound = 2.0 ** -24 * (2 * t.abs().sum(0) + (t.shape[0] + 8) * R)
+    over = ((got.double() - pre[-1]).abs() / bound).max().item()
+    print(f"  largest error / bound {over:.3f}", flush=True)
+    assert over <= 1.0
