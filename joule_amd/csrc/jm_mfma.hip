@@ -291,11 +291,11 @@ __device__ __forceinline__ uint4 token_piece(const uint8_t* ring, uint32_t at, i
 
 // One group's products: P[rb] from the stage's token operands in LDS, on top
 // of the group's correction (corr: the operand of the block of 4 groups it
-// lies in).  The digits' planes come largest first: with |a| <= 65535 the
-// correction -8 sum(a) is a multiple of 8 under 2^25, the sums with the planes
-// of 16^3 and 16^2 stay multiples of 8 under 2^27, with the plane of 16 under
-// 2^26, all of which float32 holds; the last, sum a (q - 8), is rounded only
-// past 2^24.
+// lies in).  The digits' planes come largest first: the correction -8 sum(a)
+// and the sums with the planes of 32^3, 32^2 and 32 are multiples of 8, which
+// float32 holds up to 2^27, so they round only in groups whose values are
+// nearly all of one sign and within half of the largest (|sum a| over 2^24);
+// the last, sum a (q - 8), is rounded past 2^24.
 template <int G, int CS, int GI>
 __device__ __forceinline__ void group_mfma(floatx16 (&P)[2], const uint8_t* ring, const int8v& b0, const int8v& b1,
                                            const typename WStage<G>::ExT& ex, uint32_t sb, const bf16x8& corr) {
@@ -377,8 +377,8 @@ struct Pipe {
     template <class Hook>
     __device__ __forceinline__ void step(const uint8_t* ring, const uint8_t* cl, uint8_t* nring, Hook&& hook) {
         const uint32_t h = (threadIdx.x >> 5) & 1;
-        // the planes' scales: 2^6 for the two operands' eighths, times 16^plane
-        const uint32_t sb = G == 64 ? 0x918D8985u : h ? 0x9189u : 0x8D85u;
+        // the planes' scales: 2^6 for the two operands' eighths, times 32^plane
+        const uint32_t sb = G == 64 ? 0x948F8A85u : h ? 0x948Au : 0x8F85u;
         // this super-stage's tokens and weights have arrived (waited for by
         // count the tokens alone would do, but the compiler then waits for
         // the next ones' loads to LDS before it takes the weights; and the

@@ -2,17 +2,19 @@
 // v_mfma_scale_f32_32x32x64_f8f6f4) of the dense expert branch and the
 // plugin product (jm_mfma.hip), and the encoding of activations for them.
 //
-// A 6-bit float e2m3 with code n = 0..15 is n / 8 (the subnormals and the
-// first binade are one linear range), bit 5 its sign.  So an unsigned Q4
-// nibble q, zero-extended, is the operand q / 8, and one hexadecimal digit of
-// an integer with the integer's sign is an operand as well.  An activation
-// group (the columns one weight scale covers) is written as integers
-// a_j = rint(x_j / 2^E), |a_j| <= 65535, with E the smallest exponent that
-// allows it: the step is at most max|x| / 32767.  The 4 digits of a_j go to 4
-// planes; the products of a plane are scaled by 2^E 16^plane in the matrix
-// core (E8M0 block scales), so that 4 accumulating instructions, starting from
-// the group's correction -8 sum_j a_j 2^E (the -8 of the Q4 code), give
-// sum_j a_j (q_j - 8) 2^E in float32.
+// A 6-bit float e2m3 with code n = 0..16 is n / 8 (the subnormals and the
+// first binade are one linear range, 16 the next binade's first), bit 5 its
+// sign.  So an unsigned Q4 nibble q, zero-extended, is the operand q / 8, and a
+// balanced digit -16..15 of base 32 is an operand as well.  An activation group
+// (the columns one weight scale covers) is written as integers
+// a_j = rint(x_j / 2^E), |a_j| <= 507375 = 15 (1 + 32 + 32^2 + 32^3), with E the
+// smallest exponent that allows it: a value is held to half a step, at most
+// max|x| / 507374.  (Sixteen-valued digits under one sign, the form before, held
+// it to max|x| / 65534.)  The 4 digits of a_j go to 4 planes; the products of a
+// plane are scaled by 2^E 32^plane in the matrix core (E8M0 block scales), so
+// that 4 accumulating instructions, starting from the group's correction
+// -8 sum_j a_j 2^E (the -8 of the Q4 code), give sum_j a_j (q_j - 8) 2^E in
+// float32.
 //
 // Lane layout (checked on the device): A[i][k] at lane i % 32, B[k][n] at
 // lane n % 32, k = 32 (l / 32) + j, field j at bit 6 j of 6 dwords; D
@@ -53,6 +55,18 @@ __device__ __forceinline__ void f6_spread(uint32_t w, uint32_t v, uint32_t& d0, 
     d2 = (w & 0x00F00F00u) | ((v << 2) & 0x3C03C03Cu);
 }
 
+// the value each field of f6_spread's dwords holds
+constexpr int F6_ORDER[16] = {0, 1, 3, 4, 6, 7, 9, 10, 12, 13, 15, 8, 2, 11, 5, 14};
+constexpr int F6_AMAX = 15 * (1 + 32 + 1024 + 32768);       // the largest integer of 4 balanced digits
+constexpr int F6_BIAS = 16 * (1 + 32 + 1024 + 32768);       // + a: every digit as digit + 16, 0..31
+
+// Five digits, digit + 16 in 5 bits at bits 6 i, as operand codes: the sign in
+// bit 5, the magnitude below.
+__device__ __forceinline__ uint32_t f6_codes(uint32_t u) {
+    const uint32_t n = ~(u >> 4) & 0x01041041u;             // 1 per negative digit
+    return (((u & 0x0F3CF3CFu) ^ ((n << 4) - n)) + n) | (n << 5);
+}
+
 // Encode 16 consecutive columns (block c16 of a row: columns 16 c16 ..) held
 // by one thread; the G / 16 threads of a group are aligned neighbours, and
 // all must call this.  Writes the thread's dwords of the row's record, and
@@ -77,40 +91,30 @@ __device__ __forceinline__ void f6_encode16(const float (&x)[16], int c16, bool 
         bad |= dpp_i<DPP_XOR2>(bad);
     }
     // (values below 2^-120 lose digits rather than leave the exponent's range)
-    int E = (int)(__float_as_uint(mx) >> 23) - (127 + 15);
+    int E = (int)(__float_as_uint(mx) >> 23) - (127 + 18);
     E = E < -120 ? -120 : E;
-    if (rintf(__builtin_ldexpf(mx, -E)) > 65535.0f) E++;
-    int mag[16], sum = 0;
-    uint32_t sw = 0, sv = 0;
+    if (rintf(__builtin_ldexpf(mx, -E)) > (float)F6_AMAX) E++;
+    uint32_t u[16];
+    int sum = 0;
 #pragma unroll
     for (int j = 0; j < 16; j++) {
         const int q = bad ? 0 : (int)rintf(__builtin_ldexpf(x[j], -E));
         sum += q;
-        mag[j] = q < 0 ? -q : q;
-        const uint32_t s = (uint32_t)q >> 31;
-        if (j < 8) sw |= s << (4 * j);
-        else sv |= s << (4 * (j - 8));
+        u[j] = (uint32_t)(q + F6_BIAS);
     }
     sum += dpp_i<DPP_XOR1>(sum);
     if (G == 64) sum += dpp_i<DPP_XOR2>(sum);
-    uint32_t s0, s1, s2;
-    f6_spread(sw, sv, s0, s1, s2);
-    s2 = __builtin_amdgcn_alignbit(s2, s1, 27);             // bit 0 of each field to its bit 5
-    s1 = __builtin_amdgcn_alignbit(s1, s0, 27);
-    s0 <<= 5;
     const int c = c16 & 3, b = c & 1;
     uint8_t* const st = rec + (size_t)(c16 >> 2) * F6_STAGE;
 #pragma unroll
     for (int p = 0; p < 4; p++) {
-        uint32_t w = 0, v = 0;
+        uint32_t f[4] = {0, 0, 0, 0};                       // fields 0..4, 5..9, 10..14 and 15
 #pragma unroll
-        for (int j = 0; j < 8; j++) {
-            w |= (((uint32_t)mag[j] >> (4 * p)) & 15u) << (4 * j);
-            v |= (((uint32_t)mag[8 + j] >> (4 * p)) & 15u) << (4 * j);
-        }
-        uint32_t d0, d1, d2;
-        f6_spread(w, v, d0, d1, d2);
-        d0 |= s0; d1 |= s1; d2 |= s2;
+        for (int i = 0; i < 16; i++) f[i / 5] |= ((u[F6_ORDER[i]] >> (5 * p)) & 31u) << (6 * (i % 5));
+#pragma unroll
+        for (int k = 0; k < 4; k++) f[k] = f6_codes(f[k]);
+        f[3] &= 63u;                                        // (its other fields are absent, not -16)
+        const uint32_t d0 = f[0] | (f[1] << 30), d1 = (f[1] >> 2) | (f[2] << 28), d2 = (f[2] >> 4) | (f[3] << 26);
         const int o = G == 64 ? p : 2 * (c >> 1) + p / 2, h = G == 64 ? c >> 1 : p & 1;
         uint32_t* const hd = (uint32_t*)(st + o * 32 + h * 16);
         if (!store) continue;

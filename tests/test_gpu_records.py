@@ -45,17 +45,24 @@ class Product:
         return torch.stack([x[g] @ w[g].contiguous() for g in range(ng)])
 
 
+def _float32_bound(t):
+    """Rounding of the sums alone, per element: a group's sum is rounded at
+    most twice (the last plane, the scale's multiply-add), a running sum over
+    consecutive groups once per group and per column split (at most 8): 2^-24
+    (2 sum |term| + (groups + 8) R), R the largest sum over consecutive
+    groups."""
+    pre = torch.cat([torch.zeros_like(t[:1]), t.cumsum(0)])
+    R = pre.amax(0) - pre.amin(0)
+    return 2.0 ** -24 * (2 * t.abs().sum(0) + (t.shape[0] + 8) * R)
+
+
 @pytest.mark.parametrize("group", [64, 32])
 @pytest.mark.parametrize("m,d,T", SHAPES)
 @pytest.mark.parametrize("sign", ["one", "mixed"])
 def test_sums_round_like_float32(gpu, m, d, T, group, sign):
     """Integer tokens of 15 bits, which the encoding holds exactly, so that
-    only the sums round.  Bound per element: a group's sum is rounded at most
-    twice (the last plane, the scale's multiply-add) and a running sum over
-    consecutive groups once per group and per column split (at most 8):
-    2^-24 (2 sum |term| + (groups + 8) R), R the largest sum over consecutive
-    groups.  Tokens of one sign need the -8 of the nibbles inside the groups:
-    taken once for all groups, the running sum is up to 100 R."""
+    only the sums round.  Tokens of one sign need the -8 of the nibbles inside
+    the groups: taken once for all groups, the running sum is up to 100 R."""
     banner(f"records sums {m}x{d} T={T} G={group} {sign}")
     p = Product(m, d, group)
     g = torch.Generator(device="cuda")
@@ -66,9 +73,58 @@ def test_sums_round_like_float32(gpu, m, d, T, group, sign):
     X = X / 32768
     got = p(X)
     t = p.terms(X)
-    pre = torch.cat([torch.zeros_like(t[:1]), t.cumsum(0)])
-    R = pre.amax(0) - pre.amin(0)
-    bound = 2.0 ** -24 * (2 * t.abs().sum(0) + (t.shape[0] + 8) * R)
-    over = ((got.double() - pre[-1]).abs() / bound).max().item()
+    over = ((got.double() - t.sum(0)).abs() / _float32_bound(t)).max().item()
     print(f"  largest error / bound {over:.3f}", flush=True)
+    assert over <= 1.0
+
+
+@pytest.mark.parametrize("group", [64, 32])
+@pytest.mark.parametrize("m,d,T", [(768, 2048, 40), (8192, 768, 257)])
+@pytest.mark.parametrize("kind", ["spikes", "constant"])
+def test_values_are_held_to_half_a_step(gpu, m, d, T, group, kind):
+    """A value is held to half a step, at most its group's largest / 507374.
+    With one value per group that is the error of its term; in a row of one
+    value every group holds it alike, and the result is off by that factor.
+    On top, the sums' rounding."""
+    banner(f"records step {m}x{d} T={T} G={group} {kind}")
+    p = Product(m, d, group)
+    g = torch.Generator(device="cuda")
+    g.manual_seed(7)
+    if kind == "constant":
+        X = (1.0 + torch.rand((T, 1), generator=g, device="cuda")).expand(T, d).contiguous()
+    else:
+        X = torch.zeros((T, d // group, group), device="cuda")
+        at = torch.randint(0, group, (T, d // group, 1), generator=g, device="cuda")
+        X.scatter_(2, at, 1.0 + torch.rand((T, d // group, 1), generator=g, device="cuda"))
+        X = X.view(T, d)
+    got = p(X)
+    t = p.terms(X)
+    held = t.sum(0).abs() if kind == "constant" else t.abs().sum(0)
+    over = ((got.double() - t.sum(0)).abs() / (held / 507374 + _float32_bound(t))).max().item()
+    print(f"  largest error / bound {over:.3f}", flush=True)
+    assert over <= 1.0
+
+
+@pytest.mark.parametrize("group", [64, 32])
+@pytest.mark.parametrize("mean", [0.0, 3.0])
+def test_product_error(gpu, group, mean):
+    """N(mean, 1) tokens.  Each value's rounding is uniform within half a step,
+    at most max / 507374 of its group, and independent: the error of an
+    element has the variance sum of (max / 507374)^2 / 3 w^2, and the largest
+    of 10^5 lies within 6 of its standard deviations; on top, the sums'
+    rounding.  A lost digit plane, plane scale or correction is 30 times
+    this at the least (a step of the plane above)."""
+    banner(f"records error G={group} mean={mean}")
+    m, d, T = 2048, 2048, 70
+    p = Product(m, d, group)
+    g = torch.Generator(device="cuda")
+    g.manual_seed(11)
+    X = torch.randn((T, d), generator=g, device="cuda") + mean
+    got = p(X)
+    t = p.terms(X)
+    mx = X.double().abs().view(T, d // group, group).amax(2)
+    sd = ((mx / 507374) ** 2 / 3 @ p.W.view(m, d // group, group).square().sum(2).T.contiguous()).sqrt()
+    over = ((got.double() - t.sum(0)).abs() / (6 * sd + _float32_bound(t))).max().item()
+    rel = ((got.double() - t.sum(0)).norm() / t.sum(0).norm()).item()
+    print(f"  largest error / bound {over:.3f}, rel err {rel:.2e}", flush=True)
     assert over <= 1.0
