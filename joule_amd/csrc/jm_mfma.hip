@@ -340,6 +340,9 @@ __device__ __forceinline__ void group_acc(floatx16& acc, const floatx16& P, floa
     for (int v = 0; v < 16; v++) acc[v] = __builtin_fmaf(P[v], ws, acc[v]);
 }
 
+// A result from its accumulator (exact but at the ends of the float32 range)
+__device__ __forceinline__ float full(float acc) { return __fmul_rn(acc, (float)(1 << F6_SHIFT)); }
+
 // What acc depends on comes before what follows in the source (else the
 // operands of later stages are read first, into registers there are not).
 __device__ __forceinline__ void pin(floatx16 (&acc)[2]) {
@@ -377,8 +380,9 @@ struct Pipe {
     template <class Hook>
     __device__ __forceinline__ void step(const uint8_t* ring, const uint8_t* cl, uint8_t* nring, Hook&& hook) {
         const uint32_t h = (threadIdx.x >> 5) & 1;
-        // the planes' scales: 2^6 for the two operands' eighths, times 32^plane
-        const uint32_t sb = G == 64 ? 0x948F8A85u : h ? 0x948Au : 0x8F85u;
+        // the planes' scales: 2^6 for the two operands' eighths, times 32^plane, 2^F6_SHIFT times smaller
+        constexpr uint32_t sh = 0x01010101u * F6_SHIFT;
+        const uint32_t sb = G == 64 ? 0x948F8A85u - sh : h ? 0x948Au - (sh & 0xFFFFu) : 0x8F85u - (sh & 0xFFFFu);
         // this super-stage's tokens and weights have arrived (waited for by
         // count the tokens alone would do, but the compiler then waits for
         // the next ones' loads to LDS before it takes the weights; and the
@@ -543,7 +547,7 @@ __device__ __forceinline__ void gateup_out(const ExpertArgs& a, const floatx16 (
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, n = lane & 31, h = lane >> 5;
     const int m = a.m, r0 = rblk * GU_ROWS;
 #pragma unroll
-    for (int v = 0; v < 16; v++) act[(8 * (v / 4) + 4 * h + (v % 4)) * ACT_RP + 32 * w + n] = swiglu(acc[0][v], acc[1][v]);
+    for (int v = 0; v < 16; v++) act[(8 * (v / 4) + 4 * h + (v % 4)) * ACT_RP + 32 * w + n] = swiglu(full(acc[0][v]), full(acc[1][v]));
     __builtin_amdgcn_s_waitcnt(0xC07F);           // lgkmcnt(0)
     wave_meet();
     const int it = tid >> 3, rr = 16 * (tid & 7);
@@ -652,8 +656,8 @@ __device__ __forceinline__ void down_out(const ExpertArgs& a, const floatx16 (&a
         const float t = __shfl(tw, i, JM_WAVE);
         if (i < ti.z) {
             float* const y = a.y + (size_t)slot * a.d + row;
-            y[0] = __fmul_rn(t, acc[0][v]);
-            y[32] = __fmul_rn(t, acc[1][v]);
+            y[0] = __fmul_rn(t, full(acc[0][v]));
+            y[32] = __fmul_rn(t, full(acc[1][v]));
         }
     }
 }
@@ -769,8 +773,8 @@ k_q4_gemm_mfma(const uint8_t* __restrict__ packed, const uint16_t* __restrict__ 
         const int i = 8 * (v / 4) + 4 * h + (v % 4);
         if (i < nt) {
             float* const y = o + (size_t)(t0 + i) * m + row0 + i0;
-            y[0] = p.acc[0][v];
-            y[32] = p.acc[1][v];
+            y[0] = full(p.acc[0][v]);
+            y[32] = full(p.acc[1][v]);
         }
     }
 }

@@ -16,6 +16,12 @@
 // -8 sum_j a_j 2^E (the -8 of the Q4 code), give sum_j a_j (q_j - 8) 2^E in
 // float32.
 //
+// The corrections and products are all taken 2^F6_SHIFT times smaller, and the
+// kernels' results that much larger: 8 sum|x| of a group may pass the float32
+// range where its sum over the weights does not.  At the other end E stops at
+// -126 (the third bf16 term of a correction, 2^(E - 2) 8 / 2, is normal
+// there): groups under 2^-108 lose digits one by one, to 16 bits at 2^-111.
+//
 // Lane layout (checked on the device): A[i][k] at lane i % 32, B[k][n] at
 // lane n % 32, k = 32 (l / 32) + j, field j at bit 6 j of 6 dwords; D
 // register v of lane l = (i = 8 (v / 4) + 4 (l / 32) + v % 4, n = l % 32).
@@ -58,6 +64,7 @@ __device__ __forceinline__ void f6_spread(uint32_t w, uint32_t v, uint32_t& d0, 
 // the value each field of f6_spread's dwords holds
 constexpr int F6_ORDER[16] = {0, 1, 3, 4, 6, 7, 9, 10, 12, 13, 15, 8, 2, 11, 5, 14};
 constexpr int F6_AMAX = 15 * (1 + 32 + 1024 + 32768);       // the largest integer of 4 balanced digits
+constexpr int F6_SHIFT = 2;
 constexpr int F6_BIAS = 16 * (1 + 32 + 1024 + 32768);       // + a: every digit as digit + 16, 0..31
 
 // Five digits, digit + 16 in 5 bits at bits 6 i, as operand codes: the sign in
@@ -72,7 +79,7 @@ __device__ __forceinline__ uint32_t f6_codes(uint32_t u) {
 // all must call this.  Writes the thread's dwords of the row's record, and
 // for the group its E8M0 exponent (0xFF: NaN, when the group holds a
 // non-finite value, so that it propagates) and its correction
-// -8 sum(a) 2^E.  Only when `store`.
+// -8 sum(a) 2^(E - F6_SHIFT).  Only when `store`.
 template <int G>
 __device__ __forceinline__ void f6_encode16(const float (&x)[16], int c16, bool store, uint8_t* __restrict__ rec,
                                             uint8_t* __restrict__ exps, float* __restrict__ corr) {
@@ -92,7 +99,7 @@ __device__ __forceinline__ void f6_encode16(const float (&x)[16], int c16, bool 
     }
     // (values below 2^-120 lose digits rather than leave the exponent's range)
     int E = (int)(__float_as_uint(mx) >> 23) - (127 + 18);
-    E = E < -120 ? -120 : E;
+    E = E < -126 ? -126 : E;
     if (rintf(__builtin_ldexpf(mx, -E)) > (float)F6_AMAX) E++;
     uint32_t u[16];
     int sum = 0;
@@ -129,7 +136,7 @@ __device__ __forceinline__ void f6_encode16(const float (&x)[16], int c16, bool 
     if (store && (threadIdx.x & (G / 16 - 1)) == 0) {
         const int g = c16 / (G / 16);
         exps[g] = bad ? 0xFF : (uint8_t)(E + 127);
-        corr[g] = __builtin_ldexpf((float)(-8 * sum), E);
+        corr[g] = __builtin_ldexpf((float)(-8 * sum), E - F6_SHIFT);
     }
 }
 

@@ -128,3 +128,55 @@ def test_product_error(gpu, group, mean):
     rel = ((got.double() - t.sum(0)).norm() / t.sum(0).norm()).item()
     print(f"  largest error / bound {over:.3f}, rel err {rel:.2e}", flush=True)
     assert over <= 1.0
+
+
+@pytest.mark.parametrize("scale", [4e-34, 1e-30, 1e30, 1e36])
+@pytest.mark.parametrize("kind", ["constant", "normal"])
+def test_product_over_the_float_range(gpu, scale, kind):
+    """test_product_error's bound and test_values_are_held_to_half_a_step's at
+    the ends of the float32 range: a step is at least 2^-126, and the sums over
+    unsigned nibbles and their correction stay finite where the result is."""
+    banner(f"records range {scale} {kind}")
+    m, d, T, group = 768, 2048, 40, 64
+    p = Product(m, d, group)
+    g = torch.Generator(device="cuda")
+    g.manual_seed(13)
+    if kind == "constant":
+        X = (1.0 + torch.rand((T, 1), generator=g, device="cuda")).expand(T, d)
+    else:
+        X = torch.randn((T, d), generator=g, device="cuda")
+    X = (X.double() * scale).float().contiguous()
+    got = p(X)
+    t = p.terms(X)
+    half = (X.double().abs().view(T, d // group, group).amax(2) / 507374).clamp_min(2.0 ** -127)
+    if kind == "constant":
+        held = t.sum(0).abs() * (half / X.double().abs().view(T, d // group, group).amax(2)).amax(1, keepdim=True)
+    else:
+        held = 6 * ((half ** 2 / 3) @ p.W.view(m, d // group, group).square().sum(2).T.contiguous()).sqrt()
+    assert torch.isfinite(got).all()
+    over = ((got.double() - t.sum(0)).abs() / (held + _float32_bound(t))).max().item()
+    rel = ((got.double() - t.sum(0)).norm() / t.sum(0).norm()).item()
+    print(f"  largest error / bound {over:.3f}, rel err {rel:.2e}", flush=True)
+    assert over <= 1.0
+    # the block integers of the int8 form, 16 bits, at the lower end too
+    assert rel <= 2.0 ** -15
+
+
+@pytest.mark.parametrize("value", [float("nan"), float("inf"), -float("inf")])
+@pytest.mark.parametrize("group", [64, 32])
+def test_non_finite_values_stay_in_their_row(gpu, group, value):
+    """A non-finite value makes its token's whole row non-finite (every weight
+    row reads it) and leaves the other rows as they are."""
+    banner(f"records non-finite {value} G={group}")
+    p = Product(768, 2048, group)
+    g = torch.Generator(device="cuda")
+    g.manual_seed(17)
+    X = torch.randn((70, 2048), generator=g, device="cuda")
+    clean = p(X)
+    bad = [0, 33, 69]
+    for i, b in enumerate(bad):
+        X[b, (0, 1000, 2047)[i]] = value
+    got = p(X)
+    assert not torch.isfinite(got[bad]).any()
+    keep = [i for i in range(70) if i not in bad]
+    assert torch.equal(got[keep], clean[keep])
