@@ -1,7 +1,8 @@
 """The matrix-core product on digit planes (jm_mx.h, jm_mfma.hip) against
-float64, through the plugin product: its sums, its encoding and its range.
+float64: its sums, its encoding and its range through the plugin product, and
+the expert block whose products all take it.
 
-Shapes: 2048 columns split over 8 blocks of one super-stage (256 columns) and
+Plugin shapes: 2048 columns split over 8 blocks of one super-stage (256 columns) and
 unsplit, 768 columns unsplit (three super-stages) and split, 512 unsplit; Q4
 groups of 64 and 32; a ragged last token tile."""
 
@@ -12,6 +13,8 @@ import torch
 from conftest import banner
 from joule_amd import q4_store as Q
 from joule_amd.backend import HipBackend
+from joule_amd.moe import HbmExpertStore, MoEShape
+from joule_amd.synth import activations, router_weights, torch_store
 
 pytestmark = pytest.mark.gpu
 
@@ -180,3 +183,79 @@ def test_non_finite_values_stay_in_their_row(gpu, group, value):
     assert not torch.isfinite(got[bad]).any()
     keep = [i for i in range(70) if i not in bad]
     assert torch.equal(got[keep], clean[keep])
+
+
+class Block:
+    """A one-layer block whose experts all take the matrix-core branch."""
+
+    def __init__(self, d, m, group):
+        self.shape = MoEShape(d, m, 16, 8, True, f"d{d}-m{m}")
+        blob, offsets = torch_store(self.shape, 1, group)
+        self.group = group
+        self.store = HbmExpertStore(self.shape, 1, blob, offsets, group)
+        self.store.set_router(torch.from_numpy(router_weights(self.shape, 0)[None]).cuda())
+        self.store.set_dense_min(1)
+
+    def __call__(self, x):
+        sh = self.shape
+        self.top = torch.empty((x.shape[0], sh.topk), dtype=torch.int32, device="cuda")
+        self.tw = torch.empty((x.shape[0], sh.topk), device="cuda")
+        out = self.store.layer_ffn_batch(0, x, topk_idx=self.top, topk_w=self.tw)
+        torch.cuda.synchronize()
+        return out
+
+    def exact(self, x):
+        """float64, with the routing of the call before."""
+        sh, out = self.shape, torch.zeros(x.shape, dtype=torch.float64, device="cuda")
+        for e in range(sh.E):
+            W = [torch.from_numpy(Q.dequantize(sc.cpu().numpy().view(np.uint16), pk.cpu().numpy(), n, self.group)
+                                  .reshape(r)).cuda().double()
+                 for (sc, pk, n), r in zip(self.store.ensure(0, e), ((sh.m, sh.d), (sh.m, sh.d), (sh.d, sh.m)))]
+            tok, slot = torch.where(self.top == e)
+            xe = x[tok].double()
+            act = torch.nn.functional.silu(xe @ W[0].T) * (xe @ W[1].T)
+            out.index_add_(0, tok, self.tw[tok, slot].double().unsqueeze(1) * (act @ W[2].T))
+        return out
+
+
+@pytest.mark.parametrize("d,m,group,B", [(512, 256, 32, 40), (1024, 256, 64, 70), (2048, 768, 32, 65), (2048, 768, 64, 130),
+                                         (1024, 512, 64, 97), (2048, 2048, 64, 33)])
+@pytest.mark.parametrize("mean", [0.0, 2.0])
+def test_block_error(gpu, d, m, group, B, mean):
+    """Largest error of a token over its largest output at most 2e-5, the bar
+    of the five-digit kernels (whose step, max / 489335, lies between the
+    records' max / 507375 and max / 253688).  A lost plane, scale or
+    correction in either product costs at least 32 steps."""
+    banner(f"records block d={d} m={m} G={group} B={B} mean={mean}")
+    blk = Block(d, m, group)
+    try:
+        x = torch.from_numpy(activations(B, d, seed=d + m)).cuda() + mean
+        got = blk(x).double()
+        assert blk.store.dense_tiles() == int(((torch.bincount(blk.top.flatten().long()) + 31) // 32).sum())
+        want = blk.exact(x)
+        err = ((got - want).abs().amax(1) / want.abs().amax(1)).max().item()
+        print(f"  max rel err {err:.2e}", flush=True)
+        assert err <= 2e-5
+    finally:
+        blk.store.close()
+
+
+@pytest.mark.parametrize("group", [64, 32])
+def test_block_non_finite_tokens(gpu, group):
+    """On the matrix-core branch: a token whose act leaves the float32 range
+    comes out non-finite as a whole (every hidden row reads it), a NaN token is
+    routed nowhere and comes out 0, and the other tokens keep their bits."""
+    banner(f"records block non-finite G={group}")
+    blk = Block(1024, 768, group)
+    try:
+        x = torch.from_numpy(activations(70, 1024, seed=3)).cuda()
+        clean = blk(x)
+        x[5] *= 1e25
+        x[40, 100] = float("nan")
+        got = blk(x)
+        assert not torch.isfinite(got[5]).any()
+        assert (blk.top[40] == -1).all() and (got[40] == 0).all()
+        keep = [b for b in range(70) if b not in (5, 40)]
+        assert torch.equal(got[keep], clean[keep])
+    finally:
+        blk.store.close()
