@@ -450,6 +450,15 @@ int jm_q4_gemm_f32(float* out, const float* X, int T, const uint8_t* packed, con
 int jm_set_q4_gemm_min_tokens(int tokens);
 int jm_get_q4_gemm_min_tokens(void);
 
+/* How the bf16 projections of B tokens run (decode and prefill calls, dense
+ * FFNs): rows0 + rows1 + rows2 weight rows (0 for an absent matrix) of K
+ * columns.  Returns 0 for the 128-row GEMM tile and 1 for the 256-row one,
+ * *slices (may be NULL) the column ranges that it is split into; JM_ERR_SHAPE
+ * for products that are not GEMMs (fewer than 33 tokens, row counts or K not
+ * multiples of 128).  Reads no device memory.  No counterpart in the
+ * reference. */
+int jm_gemm_plan(int rows0, int rows1, int rows2, int K, int B, int* slices);
+
 #ifdef __cplusplus
 }
 #endif

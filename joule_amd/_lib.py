@@ -60,6 +60,7 @@ SIGNATURES = {
     "jm_q4_gemm_f32": ([_vp, _vp, _i, _vp, _vp, _i, _i, _i, _vp], _i),
     "jm_set_q4_gemm_min_tokens": ([_i], _i),
     "jm_get_q4_gemm_min_tokens": ([], _i),
+    "jm_gemm_plan": ([_i] * 5 + [_vp], _i),
 }
 
 

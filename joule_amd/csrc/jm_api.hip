@@ -815,6 +815,17 @@ int jm_set_q4_gemm_min_tokens(int tokens) {
 
 int jm_get_q4_gemm_min_tokens(void) { return g_q4_gemm_min_t.load(std::memory_order_relaxed); }
 
+int jm_gemm_plan(int rows0, int rows1, int rows2, int K, int B, int* slices) {
+    const long long n = (long long)rows0 + rows1 + rows2;
+    jm::GemvArgs a{};
+    a.rows[0] = rows0; a.rows[1] = rows1; a.rows[2] = rows2;
+    a.K = K; a.N = (int)n; a.B = B;
+    if (rows0 <= 0 || rows1 < 0 || rows2 < 0 || n > INT32_MAX || K <= 0 || B < JM_GEMM_MIN_B || !jm::gemm_shape_ok(a))
+        return fail(JM_ERR_SHAPE, "no GEMM: %d + %d + %d rows of %d columns, %d tokens", rows0, rows1, rows2, K, B);
+    if (slices) *slices = jm::gemm_slices(a);
+    return jm::gemm_wide(a) ? 1 : 0;
+}
+
 // ------------------------------------------------- block stages one by one
 
 int jm_expert_gateup(jm_store* s, int layer, const float* x, const int32_t* top, int B, float* act, void* stream) {

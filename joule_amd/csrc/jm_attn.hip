@@ -295,19 +295,20 @@ k_gemm_bf16(GemvArgs a) {
     }
 }
 
-// The same product where the blocks outnumber the CUs: block (256-row tile,
+// The same product for the larger grids (gemm_plan): block (256-row tile,
 // 64-token tile, column range), 4 waves of 64 tokens x 64 rows each, which
 // read 6 operands from LDS per 8 MFMAs where k_gemm_bf16's 32 x 32 waves read
 // 12, and two blocks per CU instead of one, so that one multiplies while the
 // other waits for its stage.  The stage is 64 columns, so that a weight row's
 // part is a whole 128-byte line (32-column stages fetched each line twice:
-// 152 us against 141 for the case below), in one LDS buffer.  At 301 tokens,
-// us per launch, against k_gemm_bf16: rows x columns 24576 x 4096 141 vs 191
-// (860 TFLOP/s executed), 4096 x 12288 112 vs 140, 6144 x 4096 45 vs 56, 4096
-// x 4096 42 vs 50.  What bounds it: a stage's loads, LDS writes and reads take
-// about 2.05 us for a pair of blocks, of which the MFMAs are 0.85; reading the
-// next stage's operands ahead from a third LDS buffer measured 158 for the
-// first case, and two stages in registers no better.
+// 152 us against 141 for the first case below), in one LDS buffer.  At 301
+// tokens, weights from HBM, us per launch in its best column ranges, against
+// k_gemm_bf16 in its own: rows x columns 24576 x 4096 146 (1) vs 181 (1), 4096
+// x 12288 94 (4) vs 110 (1), 4096 x 4096 37 (4) vs 41 (1).  What bounds it: a
+// stage's loads, LDS writes and reads take about 1.7 us for a pair of blocks,
+// of which the MFMAs are 0.85; reading the next stage's operands ahead from a
+// third LDS buffer measured 158 for the first case, and two stages in registers
+// no better.
 constexpr int GW_R = 256;           // weight rows per block
 
 struct GwStage {
@@ -492,13 +493,23 @@ static int gemm_slices_narrow(const GemvArgs& a) {
 }
 
 // Which kernel takes a, and in how many column ranges.  Both are priced in
-// microseconds as they measured here, for the 64-column stages of a block and
-// the blocks a CU gets: k_gemm_bf16 0.74 per stage and 3 per block, one block
-// at a time; the wide tile 2.05 per stage of two blocks sharing a CU or 1.25
-// of one alone, 8 per such round and 4 once.  Each further slice is written
-// and read again at about 5 TB/s.  The wide tile has to be 5% ahead: measured
-// where it is not, us narrow vs wide, 512 tokens 5120 x 2048 39 vs 41 and 2048
-// x 4096 28 vs 33.
+// microseconds, for the 64-column stages of a block and the blocks a CU gets:
+// k_gemm_bf16, in gemm_slices_narrow's ranges, 0.6 per stage and 3.5 per block,
+// one block at a time; the wide tile 1.71 per stage of two blocks sharing a CU
+// or 1.32 of one alone, 6 per such round and 1.5 once.  Each slice is written
+// here and read by the consumer, together at about 2.2 TB/s.  The constants are
+// fitted to both kernels' times in 1, 2 and 4 ranges on cold weights: rows x
+// columns 2048 x 2048, 2048 x 4096, 4096 x 4096, 4096 x 12288, 5120 x 2048,
+// 6144 x 2048, 6144 x 4096 and 24576 x 4096 at 16 token counts of 33 to 512.
+// Over these 128 the rule is within 0.4% of the better kernel on average and
+// never behind k_gemm_bf16 alone (slices' cost included), 2.4% ahead of it.  Some
+// lines, us, narrow (ranges) vs wide (ranges) with the slices' cost: 24576 x
+// 4096 at 64 tokens 54 (1) vs 56 (1), 65 76 (2) vs 71 (2), 129 118 (2) vs 115
+// (4), 257 180 (1) vs 145 (1); 4096 x 12288 at 256 tokens 75 (2) vs 82 (4), 257
+// 110 (1) vs 96 (4); 6144 x 4096 at 128 tokens 27 (2) vs 35 (4), 129 43 (1) vs
+// 36 (4).  At 6144 x 4096 and 256 to 320 tokens it keeps the narrow kernel, 46 to
+// 51, where 4 wide ranges take 43 to 47; 5120 x 2048 goes wide from 448 tokens
+// (39 vs 38).
 struct GemmPlan {
     bool wide;
     int kz;
@@ -509,13 +520,13 @@ static GemmPlan gemm_plan(const GemvArgs& a) {
     GemmPlan p{false, gemm_slices_narrow(a)};
     // (the wide kernel sums squares only where it applies a norm weight)
     if (a.rows[0] % GW_R != 0 || a.rows[1] % GW_R != 0 || a.rows[2] % GW_R != 0 || (a.rss && !a.norm_w)) return p;
-    const double slice = (double)a.B * a.N * 4 / 5e6;
+    const double slice = (double)a.B * a.N * 4 / 2.2e6;
     const long long nb = ((long long)(a.N / GM_R) * tt * p.kz + ncu - 1) / ncu;
-    double best = 0.95 * ((double)nb * (0.74 * nstage / p.kz + 3.0) + slice * p.kz);
+    double best = (double)nb * (0.6 * nstage / p.kz + 3.5) + slice * p.kz;
     for (int kz : {1, 2, 4}) {
         if (nstage % (2 * kz) != 0) continue;
         const long long n = ((long long)(a.N / GW_R) * tt * kz + ncu - 1) / ncu;
-        const double t = (double)nstage / kz * (2.05 * (n / 2) + 1.25 * (n % 2)) + 8.0 * ((n + 1) / 2) + 4.0 + slice * kz;
+        const double t = (double)nstage / kz * (1.71 * (n / 2) + 1.32 * (n % 2)) + 6.0 * ((n + 1) / 2) + 1.5 + slice * kz;
         if (t < best) {
             best = t;
             p = {true, kz};
@@ -525,6 +536,7 @@ static GemmPlan gemm_plan(const GemvArgs& a) {
 }
 
 int gemm_slices(const GemvArgs& a) { return gemm_plan(a).kz; }
+bool gemm_wide(const GemvArgs& a) { return gemm_plan(a).wide; }
 
 hipError_t launch_gemm_bf16(const GemvArgs& a, hipStream_t st) {
     if (a.B == 0 || a.N == 0) return hipSuccess;

@@ -209,7 +209,7 @@ struct GemvArgs {
     int K, N, B;              // N = rows[0] + rows[1] + rows[2]
     float* part;              // [K / gemv_slice_cols(K)][B][N]
     float* rss;               // [slices][B] receives the sums of x[b][k]^2 over each slice's columns
-                              // (the GEMM: one slice of all K), or NULL: not wanted
+                              // (the GEMM: its column ranges), or NULL: not wanted
 };
 // the decoder's projections take K a multiple of 1024 up to 8192; the
 // kernel takes any multiple of its slice width: 512 columns, 1024 from
@@ -217,11 +217,13 @@ struct GemvArgs {
 bool gemv_shape_ok(int K);
 int gemv_slice_cols(int K);
 hipError_t launch_gemv_part(const GemvArgs& a, hipStream_t st);
-// many tokens (a prefill chunk): the whole sum into part[0] (one slice);
-// every row count a multiple of 128, K a multiple of 128
+// many tokens (a prefill chunk): gemm_slices(a) column ranges' sums into
+// part[0..]; every row count a multiple of 128, K a multiple of 128
 bool gemm_shape_ok(const GemvArgs& a);
 // the K slices the GEMM writes for a (1, 2 or 4; the consumer sums them)
 int gemm_slices(const GemvArgs& a);
+// whether the 256-row tile takes it
+bool gemm_wide(const GemvArgs& a);
 hipError_t launch_gemm_bf16(const GemvArgs& a, hipStream_t st);
 // from this many tokens the projections take the GEMM
 #define JM_GEMM_MIN_B 33
