@@ -1614,7 +1614,7 @@ hipError_t launch_attn(const AttnArgs& a, int qpk, float* att, hipStream_t st) {
         hipError_t e0 = hipGetLastError();
         if (e0 != hipSuccess) return e0;
     }
-    const bool tile = !a.append && a.shared && !a.kv_f32 && (long long)a.B * a.KH >= JM_ATTN_TILE_MIN;
+    const bool tile = !a.append && a.shared && !a.kv_f32 && attn_tile_takes(a.B, a.KH, qpk);
     if (qpk != 1 && qpk != 2 && qpk != 4 && qpk != 8) return hipErrorInvalidValue;
     if (!a.append) {
         // (the partial outputs' buffer, unused by k_attn_tile, holds the query heads for it)

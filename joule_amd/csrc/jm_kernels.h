@@ -261,18 +261,23 @@ struct AttnArgs {
     uint16_t* qhl;            // [B][H][2][128] finished query heads for k_attn_tile (launch_attn sets it)
     float* part_ml;           // [B][KH][S][H/KH][2]
 };
-// tokens x KV heads of one prompt's call over bf16 caches from which it takes
-// the query-tiled kernel (k_attn_tile).  Below, too few of its blocks (one
-// per KV head and 64 query rows) share the prefix.  A layer at prefixes of
-// 200 / 1000 / 4000 positions, per-position form vs tiled, us: 4 KV heads, 64
-// tokens 58.9 / 71.2 / 115.8 vs 61.2 / 72.2 / 118.0, 96 tokens 64.8 / 83.1 /
-// 150.1 vs 63.9 / 75.1 / 120.7; 8 KV heads, 32 tokens 48.9 / 60.1 / 100.3 vs
-// 49.8 / 63.6 / 108.9, 48 tokens 59.4 / 76.0 / 135.8 vs 60.7 / 73.4 / 118.5;
-// 16 KV heads, 16 tokens 41.2 / 50.2 / 86.9 vs 41.9 / 53.0 / 99.0, 20 tokens
-// 44.6 / 56.2 / 102.7 vs 44.2 / 55.6 / 103.0.
-#ifndef JM_ATTN_TILE_MIN
-#define JM_ATTN_TILE_MIN 320
-#endif
+// Whether one prompt's call over bf16 caches (qpk query heads per KV head)
+// takes the query-tiled kernel, k_attn_tile.  Below, too few of its blocks (one
+// per KV head and 64 query rows) share the prefix, and with under 16 tokens the
+// blocks' tiles are mostly padding that a long prefix repeats.  A layer at
+// prefixes of 0 / 200 / 1000 / 4000 positions, per-position form vs tiled, us,
+// query / KV heads: 32/4, 80 tokens 58.7 / 61.8 / 76.8 / 133.6 vs 57.9 / 61.9 /
+// 73.6 / 119.5; 32/8, 40 tokens 55.6 / 58.4 / 71.6 / 121.6 vs 55.6 / 58.1 / 72.0
+// / 117.0; 32/16, 20 tokens 45.9 / 48.8 / 60.4 / 108.6 vs 45.6 / 48.3 / 60.4 /
+// 108.1; 64/8, 40 tokens 66.0 / 69.4 / 85.1 / 145.8 vs 65.3 / 68.0 / 81.4 /
+// 127.8; one head each, 16/16, 20 tokens 41.6 / 44.1 / 55.5 / 101.7 vs 40.7 /
+// 42.9 / 55.0 / 102.3; 8/8, 40 tokens 47.1 / 49.7 / 62.6 / 107.6 vs 46.6 / 49.2
+// / 63.7 / 109.8, 50 tokens 47.8 / 51.6 / 67.5 / 123.2 vs 47.7 / 50.2 / 64.7 /
+// 110.6; 32/32, 10 tokens 44.1 / 46.7 / 57.6 / 110.0 vs 42.9 / 45.0 / 56.6 /
+// 126.9, 16 tokens 44.8 / 48.4 / 67.1 / 147.2 vs 43.6 / 45.4 / 57.1 / 127.7.
+constexpr bool attn_tile_takes(int B, int KH, int qpk) {
+    return B >= 16 && (long long)B * KH >= (qpk == 1 ? 352 : 320);
+}
 // the projections finished (q out, k and v appended), partial attention,
 // then the merge into att [B][H*128]
 hipError_t launch_attn(const AttnArgs& a, int qpk, float* att, hipStream_t st);

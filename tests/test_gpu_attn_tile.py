@@ -65,3 +65,10 @@ def test_non_finite_token_stays_causal(bad, value):
     assert np.array_equal(got[:bad], clean[:bad])
     assert not np.isfinite(got[bad:]).all(axis=1).any()
     dec.store.close()
+
+
+@pytest.mark.parametrize("H,KH,B,p0", [(32, 32, 15, 300), (32, 32, 16, 300), (8, 8, 43, 130), (8, 8, 44, 130)])
+def test_one_head_each_on_both_sides_of_the_rule(H, KH, B, p0):
+    """One query head per KV head takes the tiled kernel from 16 tokens and 352
+    tokens x KV heads."""
+    test_tiles_match_oracle(H, KH, 1, B, p0)
