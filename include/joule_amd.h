@@ -146,13 +146,14 @@ int jm_layer_ffn_batch(jm_store* s, int layer, const float* x, int B, float* out
 /* jm_layer_ffn_batch for callers that cannot allocate device memory: code
  * under HIP graph capture, tight serving loops, harnesses that forbid
  * hipMalloc.  No counterpart in the reference.  The same kernels and
- * results as jm_layer_ffn_batch, with the workspace in a fixed array of
- * JM_NOALLOC_SCRATCH_BYTES on each device (reserved when the library first
- * creates a store on that device, kept until the process ends) instead of
- * the store's own: the call allocates nothing and fails with JM_ERR_SHAPE
- * when B tokens of the store's shape need more workspace than the array
- * holds (about 140 KB per token for the Qwen3-30B-A3B block: up to ~110
- * tokens).  Every call on a device shares that device's array: calls that
+ * results as jm_layer_ffn_batch, with the workspace in a fixed array on each
+ * device (9/8 of JM_NOALLOC_SCRATCH_BYTES, 18 MiB; reserved when the library
+ * first creates a store on that device, kept until the process ends) instead
+ * of the store's own: the call allocates nothing and fails with JM_ERR_SHAPE
+ * when B tokens of the store's shape count for more than
+ * JM_NOALLOC_SCRATCH_BYTES (about 130 KB per token for the Qwen3-30B-A3B
+ * block: up to 129 tokens; the array's eighth above it is for operands that
+ * the count leaves out).  Every call on a device shares that device's array: calls that
  * overlap on one GPU (other streams, other stores, other threads) race and
  * must be serialised by the caller.  jm_store_copy_workspace does not see
  * this workspace. */

@@ -154,85 +154,89 @@ int check_group_shape(int d, int m, int group) {
 
 namespace {
 
-// Sizes of the Ws fields for B tokens, in field order.
-constexpr int WS_NF = 25;
-void ws_sizes(const jm_store* s, int B, size_t (&sz)[WS_NF]) {
+// The Ws fields by name, in field order: what follows pairs sizes and pointers
+// by name.
+#define JM_WS_FIELDS(X)                                                                                       \
+    X(logits) X(top) X(tw) X(xdig) X(xscale) X(seg_off) X(seg_slot) X(active) X(n_active) X(first_slot) X(comb) \
+    X(work) X(tiles) X(n_tiles) X(small) X(act) X(adig) X(ascale) X(y) X(aq) X(xq) X(xc) X(ac) X(xe) X(ae)
+
+// Bytes of the Ws fields for B tokens.
+struct WsSizes {
+#define JM_X(f) size_t f;
+    JM_WS_FIELDS(JM_X)
+#undef JM_X
+    size_t total() const {
+        size_t t = 0;
+#define JM_X(f) t += align256(f);
+        JM_WS_FIELDS(JM_X)
+#undef JM_X
+        return t;
+    }
+};
+static_assert(sizeof(jm::Ws) / sizeof(void*) == sizeof(WsSizes) / sizeof(size_t), "a size for every workspace field");
+
+WsSizes ws_sizes(const jm_store* s, int B) {
     const int E = s->E, d = s->d, m = s->m, k = s->topk, G = s->group;
     const size_t nslot = (size_t)B * k;
     // digit planes: room for the most (jm_store_set_act_digits)
     const size_t words_d = (size_t)(d / G) * JM_NDIG_MAX * (G / 8);
     const size_t words_m = (size_t)(m / 8) * JM_NDIG_MAX;
-    const size_t max_tiles = nslot / JM_DENSE_TILE + E;
-    const size_t v[WS_NF] = {
-        (size_t)B * E * 4,            // logits
-        nslot * 4,                    // top
-        nslot * 4,                    // tw
-        (size_t)B * words_d * 4,      // xdig
-        (size_t)B * (d / G) * 4,      // xscale
-        (size_t)(E + 1) * 4,          // seg_off
-        nslot * 4,                    // seg_slot
-        (size_t)E * 4,                // active
-        4,                            // n_active
-        (size_t)E * 4,                // first_slot
-        nslot * 4,                    // comb
-        (size_t)E * sizeof(jm::ExpertWork),   // work table
-        (max_tiles + 1) * 16,         // dense tiles
-        8,                            // n_tiles (tiles, small experts)
-        (size_t)E * 4,                // small
-        nslot * m * 4,                // act
-        nslot * words_m * 4,          // adig
-        nslot * (m / 32) * 4,         // ascale
-        nslot * d * 4,                // y
-        nslot * m * 3,                // aq
-        (size_t)B * d * 3,            // xq
-        (size_t)B * (d / G) * 4,      // xc
-        nslot * (m / G) * 4,          // ac
-        (size_t)B * (d / G),          // xe
-        nslot * (m / G),              // ae
-    };
-    for (int i = 0; i < WS_NF; i++) sz[i] = v[i];
+    WsSizes z;
+    z.logits = (size_t)B * E * 4;
+    z.top = nslot * 4;
+    z.tw = nslot * 4;
+    z.xdig = (size_t)B * words_d * 4;
+    z.xscale = (size_t)B * (d / G) * 4;
+    z.seg_off = (size_t)(E + 1) * 4;
+    z.seg_slot = nslot * 4;
+    z.active = (size_t)E * 4;
+    z.n_active = 4;
+    z.first_slot = (size_t)E * 4;
+    z.comb = nslot * 4;
+    z.work = (size_t)E * sizeof(jm::ExpertWork);
+    z.tiles = (nslot / JM_DENSE_TILE + E + 1) * sizeof(int4);
+    z.n_tiles = 8;                      // tiles, small experts
+    z.small = (size_t)E * 4;
+    z.act = nslot * m * 4;
+    z.adig = nslot * words_m * 4;
+    z.ascale = nslot * (m / 32) * 4;
+    z.y = nslot * d * 4;
+    z.aq = nslot * m * 3;
+    z.xq = (size_t)B * d * 3;
+    z.xc = (size_t)B * (d / G) * 4;
+    z.ac = nslot * (m / G) * 4;
+    z.xe = (size_t)B * (d / G);
+    z.ae = nslot * (m / G);
+    return z;
 }
 
 }  // namespace
 
-size_t jm::ws_bytes(const jm_store* s, int B) {
-    size_t sz[WS_NF];
-    ws_sizes(s, B, sz);
-    size_t total = 0;
-    for (size_t v : sz) total += align256(v);
-    return total;
-}
+size_t jm::ws_bytes(const jm_store* s, int B) { return ws_sizes(s, B).total(); }
 
-// jm_layer_ffn_batch_noalloc's bound was set when the dense branch's operands
-// took 2 bytes per value, a scale and a sum per group, and a tile 8 bytes; it is kept, so that the
-// batches the call takes and refuses are what they were.  The layout above is
-// at most an eighth larger (3 bytes per value, of 17 or more in all).
+// jm_layer_ffn_batch_noalloc's bound counts the dense branch's operands at 2
+// bytes per value with a scale and a sum per group, and a tile at 8 bytes, so
+// that the batches the call takes do not depend on their layout.  The layout
+// above takes 3 bytes per value, 5 per group and 16 per tile.  What it adds is
+// under an eighth of the counted bytes: 1 byte per act value of 8.6 (act, 5
+// digit planes and the counted 2) with y's 4 d beside them, 1 per token value
+// of the 4.5 and more beside at least 4 of y, 8 per tile and expert of 100.
 size_t jm::ws_noalloc_bytes(const jm_store* s, int B) {
-    const size_t G = s->group, nslot = (size_t)B * s->topk;
-    size_t sz[WS_NF];
-    ws_sizes(s, B, sz);
-    size_t total = 0;
-    sz[12] = (nslot / JM_DENSE_TILE + s->E) * 8;      // dense tiles
-    for (int i = 0; i < WS_NF - 6; i++) total += align256(sz[i]);
-    return total + 2 * align256(nslot * s->m) + 2 * align256((size_t)B * s->d) + 2 * align256(B * (s->d / G) * 4) +
-           2 * align256(nslot * (s->m / G) * 4);
+    const size_t d = s->d, m = s->m, G = s->group, nslot = (size_t)B * s->topk;
+    WsSizes z = ws_sizes(s, B);
+    z.tiles = (nslot / JM_DENSE_TILE + s->E) * 8;
+    z.aq = z.xq = z.xc = z.ac = z.xe = z.ae = 0;
+    return z.total() + 2 * align256(nslot * m) + 2 * align256(B * d) + 2 * align256(B * (d / G) * 4) +
+           2 * align256(nslot * (m / G) * 4);
 }
 
 void jm::ws_layout(const jm_store* s, int B, char* base, Ws* w) {
-    size_t sz[WS_NF];
-    ws_sizes(s, B, sz);
-    void** slots[WS_NF] = {(void**)&w->logits, (void**)&w->top, (void**)&w->tw, (void**)&w->xdig,
-                           (void**)&w->xscale, (void**)&w->seg_off, (void**)&w->seg_slot,
-                           (void**)&w->active, (void**)&w->n_active, (void**)&w->first_slot,
-                           (void**)&w->comb, (void**)&w->work, (void**)&w->tiles,
-                           (void**)&w->n_tiles, (void**)&w->small, (void**)&w->act, (void**)&w->adig,
-                           (void**)&w->ascale, (void**)&w->y, (void**)&w->aq, (void**)&w->xq,
-                           (void**)&w->xc, (void**)&w->ac, (void**)&w->xe, (void**)&w->ae};
-    static_assert(sizeof(Ws) == WS_NF * sizeof(void*), "a size for every workspace field");
-    for (int i = 0; i < WS_NF; i++) {
-        *slots[i] = base;
-        base += align256(sz[i]);
-    }
+    const WsSizes z = ws_sizes(s, B);
+#define JM_X(f)                             \
+    w->f = (decltype(w->f))base;            \
+    base += align256(z.f);
+    JM_WS_FIELDS(JM_X)
+#undef JM_X
 }
 
 int jm::store_reserve(jm_store* s, int B) {
@@ -663,10 +667,13 @@ int jm_layer_ffn_batch_noalloc(jm_store* s, int layer, const float* x, int B, fl
     if (B == 0) return 0;
     if (!x || !out) return fail(JM_ERR_ARG, "x and out must be non-NULL");
     if (!aligned(x, 16) || !aligned(out, 16)) return fail(JM_ERR_ARG, "x and out must be 16-byte aligned");
-    const size_t need = jm::ws_noalloc_bytes(s, B);
-    if (need > (size_t)JM_NOALLOC_SCRATCH_BYTES || jm::ws_bytes(s, B) > SCRATCH_BYTES)
-        return fail(JM_ERR_SHAPE, "B=%d needs %zu bytes of workspace; the fixed no-allocation workspace holds %zu "
+    const size_t need = jm::ws_noalloc_bytes(s, B), bytes = jm::ws_bytes(s, B);
+    if (need > (size_t)JM_NOALLOC_SCRATCH_BYTES)
+        return fail(JM_ERR_SHAPE, "B=%d needs %zu bytes of workspace; a no-allocation call takes up to %zu "
                     "(use jm_layer_ffn_batch, or fewer tokens per call)", B, need, (size_t)JM_NOALLOC_SCRATCH_BYTES);
+    if (bytes > SCRATCH_BYTES)
+        return fail(JM_ERR_SHAPE, "B=%d needs %zu bytes of workspace; the fixed no-allocation workspace holds %zu "
+                    "(use jm_layer_ffn_batch, or fewer tokens per call)", B, bytes, SCRATCH_BYTES);
     void* base = (s->device >= 0 && s->device < MAX_DEVICES) ? scratch_ptr[s->device] : nullptr;
     if (!base) return fail(JM_ERR_ARG, "the no-allocation workspace of device %d is not resolved", s->device);
     JM_HIP(hipSetDevice(s->device), "hipSetDevice");

@@ -13,7 +13,7 @@ import torch
 
 from conftest import banner
 from joule_amd import _lib
-from joule_amd.moe import QWEN3, HbmExpertStore
+from joule_amd.moe import OLMOE, QWEN3, HbmExpertStore, MoEShape
 from joule_amd.synth import activations, router_weights, torch_store
 
 pytestmark = pytest.mark.gpu
@@ -68,3 +68,27 @@ def test_noalloc_refuses_batches_beyond_its_workspace(store):
     want = _call(L.jm_layer_ffn_batch, store, 0, x8)
     got = _call(L.jm_layer_ffn_batch_noalloc, store, 0, x8)
     assert np.array_equal(got[0].view(np.uint32), want[0].view(np.uint32))
+
+
+@pytest.mark.parametrize("shape,group,most", [(QWEN3, 64, 129), (QWEN3, 32, 128), (OLMOE, 64, 113),
+                                              (MoEShape(512, 256, 16, 8, True, "d512-m256"), 32, 450)])
+def test_noalloc_largest_batch(gpu, shape, group, most):
+    """The largest batch the call takes, which fills the array's last bytes,
+    gives the allocating call's bits; one token more is refused."""
+    banner(f"no-allocation block: {shape.name} G={group}, {most} tokens")
+    L = _lib.lib()
+    blob, offsets = torch_store(shape, 1, group)
+    st = HbmExpertStore(shape, 1, blob, offsets, group)
+    try:
+        st.set_router(torch.from_numpy(router_weights(shape, 0)[None]).cuda())
+        x = torch.from_numpy(activations(most + 1, shape.d, seed=9)).cuda()
+        want, got = (torch.full((most, shape.d), float("nan"), device="cuda") for _ in range(2))
+        for fn, out in ((L.jm_layer_ffn_batch, want), (L.jm_layer_ffn_batch_noalloc, got)):
+            _lib.check(fn(st._h, 0, _lib.ptr(x), most, _lib.ptr(out), None, None, _lib.stream_handle()), fn.__name__)
+        torch.cuda.synchronize()
+        assert torch.isfinite(want).all() and torch.equal(got, want)
+        out = torch.empty_like(x)
+        rc = L.jm_layer_ffn_batch_noalloc(st._h, 0, _lib.ptr(x), most + 1, _lib.ptr(out), None, None, _lib.stream_handle())
+        assert rc == -2 and b"no-allocation" in L.jm_last_error()
+    finally:
+        st.close()
