@@ -2,6 +2,7 @@
 entries report, the per-call percentiles, the block's algorithmic bytes and
 the refusal of more than one GPU (before anything touches a GPU)."""
 
+import json
 import subprocess
 import sys
 from pathlib import Path
@@ -86,3 +87,23 @@ def test_more_than_one_gpu_is_refused_before_the_gpu_is_touched():
     assert p.returncode == 2
     assert "one GPU only" in p.stderr
     assert p.stdout == ""
+
+
+def test_result_line_is_short_and_keeps_the_numbers():
+    par = {"ok": True, "normwise_max": 5.123456789e-05}
+    res = {"metric": "m", "value": 45678.123456789, "ms_per_step": 0.0412345678901, "steps": 20, "vs_baseline": None,
+           "config": {"batch": 8}, "parity": {"ok": True, "configs": {"qwen3_B1": par}},
+           "sweep": {"qwen3_B1": {"tok_per_s": 1 / 3, "parity": par}, "other": {"parity": par},
+                     "plugin_q4_gemm": {"queued_ahead": True, "sizes": {"T1": {"us_per_call": 5.3, "path": "dot8_digits",
+                                                                             "bytes": 846848, "GBs": 160.3, "tflops_equiv": 0.6,
+                                                                             "queued_ahead": True}}}}}
+    before = json.dumps(res)
+    line = bench.result_line(res)
+    assert json.dumps(res) == before and "\n" not in line and " " not in line
+    got = json.loads(line)
+    assert got["value"] == pytest.approx(res["value"], rel=1e-5) and got["ms_per_step"] == pytest.approx(res["ms_per_step"], rel=1e-5)
+    assert got["steps"] == 20 and got["vs_baseline"] is None and got["config"] == {"batch": 8}
+    assert got["parity"]["configs"]["qwen3_B1"]["normwise_max"] == pytest.approx(par["normwise_max"], rel=1e-5)
+    assert "parity" not in got["sweep"]["qwen3_B1"] and "parity" in got["sweep"]["other"]
+    assert got["sweep"]["plugin_q4_gemm"] == {"queued_ahead": True, "sizes": {"T1": {"us_per_call": 5.3, "path": "dot8_digits"}}}
+    assert bench.result_line({"value": 1.0}) == '{"value":1.0}'
