@@ -112,11 +112,11 @@ int jm_store_info(const jm_store* s, int* L, int* E, int* d, int* m, int* topk, 
 
 /* Batches with B * topk > 256 slots: an expert routed at least min_tokens
  * slots takes the MFMA branch (32-token tiles on the fp6 matrix cores: the
- * nibbles q against each activation's four base-16 digits), the others the
- * wave-item GEMV kernels.  0 restores the default (8, or 3 in calls with fewer
- * than 16 slots per expert on a store with 4 digit planes); a value above B * topk keeps every expert on the
- * GEMV kernels.  No counterpart in the
- * reference, whose batch is at most 16 tokens (decode_kernel.c:1522). */
+ * nibbles q against each activation's four balanced base-32 digits), the
+ * others the wave-item GEMV kernels.  0 restores the default (8, or 3 in calls
+ * with fewer than 16 slots per expert on a store with 4 digit planes); a value
+ * above B * topk keeps every expert on the GEMV kernels.  No counterpart in
+ * the reference, whose batch is at most 16 tokens (decode_kernel.c:1522). */
 int jm_store_set_dense_min(jm_store* s, int min_tokens);
 
 /* Base-16 digit planes per activation value on the GEMV (wave-item)
@@ -125,8 +125,9 @@ int jm_store_set_dense_min(jm_store* s, int min_tokens);
  * group's largest magnitude / R, R = 30583 for 4 digits, 489335 for 5).  4
  * (the default; 0 restores it) keeps about 15 bits per group, 5 about 19 bits
  * at more dot products per row.  Router indices and weights do not depend on
- * it.  The MFMA branch's digit planes are not affected.  No counterpart in
- * the reference, whose activations are float32. */
+ * it.  The MFMA branch's digit planes (a value held to its group's largest /
+ * 507374) are not affected; with 5 it takes experts from 8 slots on by
+ * default.  No counterpart in the reference, whose activations are float32. */
 int jm_store_set_act_digits(jm_store* s, int ndig);
 /* The store's digit planes (4 or 5), -1 for a NULL store. */
 int jm_store_act_digits(const jm_store* s);
@@ -153,10 +154,10 @@ int jm_layer_ffn_batch(jm_store* s, int layer, const float* x, int B, float* out
  * when B tokens of the store's shape count for more than
  * JM_NOALLOC_SCRATCH_BYTES (about 130 KB per token for the Qwen3-30B-A3B
  * block: up to 129 tokens; the array's eighth above it is for operands that
- * the count leaves out).  Every call on a device shares that device's array: calls that
- * overlap on one GPU (other streams, other stores, other threads) race and
- * must be serialised by the caller.  jm_store_copy_workspace does not see
- * this workspace. */
+ * the count leaves out).  Every call on a device shares that device's array:
+ * calls that overlap on one GPU (other streams, other stores, other threads)
+ * race and must be serialised by the caller.  jm_store_copy_workspace does
+ * not see this workspace. */
 #define JM_NOALLOC_SCRATCH_BYTES (16u << 20)
 int jm_layer_ffn_batch_noalloc(jm_store* s, int layer, const float* x, int B, float* out,
                                int32_t* topk_idx, float* topk_w, void* stream);

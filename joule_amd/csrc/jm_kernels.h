@@ -183,7 +183,10 @@ hipError_t launch_down_mfma(const ExpertArgs& a, int max_tiles, hipStream_t st);
 // q4_gemm_mfma_ws bytes
 bool q4_gemm_mfma_ok(int m, int d, int group);
 // default token count from which jm_q4_gemm_f32 takes the matrix cores
-// (jm_set_q4_gemm_min_tokens changes it): the measured crossover
+// (jm_set_q4_gemm_min_tokens changes it): the measured crossover with groups of
+// 64 (768 x 2048, us, dot8 vs matrix cores: 6 tokens 9.8 vs 10.4, 7 tokens 10.7
+// vs 10.4); with groups of 32 it lies at 13 (7 tokens 7.9 vs 10.9, 16 12.5 vs
+// 11.2)
 #ifndef JM_Q4_GEMM_MIN_T
 #define JM_Q4_GEMM_MIN_T 7
 #endif

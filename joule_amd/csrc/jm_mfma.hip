@@ -35,20 +35,23 @@
 // tile entry, slots, corrections and first operands are requested during the
 // unit before.
 //
-// Bound.  512 Zipf-routed Qwen3 tokens (1122 gate/up units, 214 MB of records):
-// a block's super-stage takes 2.7 to 4 us, of which its arithmetic alone is 1.2
-// (per wave 330 vector instructions and 32 MFMAs of 34 cycles) and the rest the
-// records' arrival, 3 to 4.2 TB/s while every block streams; the unit's SwiGLU
-// and encode take 3 to 5; and 1122 units on 512 resident blocks leave the third
-// round a fifth full.  Gate/up 134 -> 99 us, down 64 -> 56 (203 OLMoE tokens: 80
-// -> 66 and 46 -> 38).  The form before (int8 digit pairs, exact int32 group
-// sums, 4 instructions per element for two float scales) moved 56 16-byte LDS
-// reads and writes per wave and super-stage, 3584 LDS cycles of the 3600 that a
-// pair of waves took.  Measured on the way: blocks of one unit 117 and 69 (each
-// waited 7 to 14 us for its chain of loads), three such blocks per CU 108 and
-// 64 (168 registers, spills), tokens staged 32 bytes per lane pair 113 (64
-// address cycles per load instead of 16); the units' column order rotated by
-// expert and row block made no difference.
+// Bound.  512 Zipf-routed Qwen3 tokens (183 tiles, 1098 gate/up units, 214 MB
+// of records): gate/up takes 98 us and reads 475 MB past the L2, at 4.85 TB/s as
+// fast as a large copy on this card, because an expert of several tiles reads
+// its records once per tile; down takes 51 us for 214 MB.  The matrix cores are
+// busy 17%, the VALU 37% (per wave and super-stage 32 fp6 MFMAs of 34 cycles, 4
+// for the corrections and 625 vector instructions, the unit's epilogue included).  The
+// unit's SwiGLU and encode take 3 to 5 us, and the units leave the third round
+// of the 512 resident blocks a seventh full.  The form before (int8 digit pairs,
+// exact int32 group sums, 4 instructions per element for two float scales): 134
+// and 64 us; it moved 56 16-byte LDS reads and writes per wave and super-stage,
+// 3584 LDS cycles of the 3600 that a pair of waves took.  Measured on the way:
+// blocks of one unit 117 and 69 (each waited 7 to 14 us for its chain of loads),
+// three such blocks per CU 108 and 64 (168 registers, spills), tokens staged 32
+// bytes per lane pair 113 (64 address cycles per load instead of 16); the units'
+// column order rotated by expert and row block made no difference; the -8 of
+// all groups as one product of the corrections and the row scales at the unit's
+// start 99 and 56 (it rounds: up to 15 times the error on tokens of one sign).
 #include <algorithm>
 #include <type_traits>
 

@@ -162,7 +162,8 @@ class HbmExpertStore:
         """Base-16 digit planes per activation value on the GEMV kernels: 4
         (the default; 0 restores it, about 15 bits per Q4 group) or 5 (about
         19 bits, more dot products per weight row).  Routing does not depend
-        on it; the MFMA branch's digit planes are not affected."""
+        on it; the MFMA branch's digit planes are not affected (with 5 it takes
+        experts from 8 slots on by default)."""
         _lib.check(_lib.lib().jm_store_set_act_digits(self._h, int(ndig)), "jm_store_set_act_digits")
 
     @property

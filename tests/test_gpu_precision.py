@@ -93,7 +93,7 @@ def test_mfma_beyond_fp16_range(qwen1, case):
     """Every expert on the MFMA branch (dense_min 1, B=64) with two tokens
     whose activations leave the fp16 range: their x itself (a few channels
     at 1e5) or only their SwiGLU outputs (channels at 2e4: act passes
-    65504).  The branch's int8 digit pairs carry one scale per token and Q4
+    65504).  The branch's digit planes carry one scale per token and Q4
     group, so any finite magnitude is taken; the block must stay finite and
     within tolerance of the oracle, and the case must really occur (act read
     back from the workspace)."""
