@@ -217,10 +217,10 @@ size_t jm::ws_bytes(const jm_store* s, int B) { return ws_sizes(s, B).total(); }
 // jm_layer_ffn_batch_noalloc's bound counts the dense branch's operands at 2
 // bytes per value with a scale and a sum per group, and a tile at 8 bytes, so
 // that the batches the call takes do not depend on their layout.  The layout
-// above takes 3 bytes per value, 5 per group and 16 per tile.  What it adds is
-// under an eighth of the counted bytes: 1 byte per act value of 8.6 (act, 5
-// digit planes and the counted 2) with y's 4 d beside them, 1 per token value
-// of the 4.5 and more beside at least 4 of y, 8 per tile and expert of 100.
+// above takes 3 bytes per value, 5 per group and 16 per tile: over the shapes
+// that jm_store_create takes, at most 1.1095 times JM_NOALLOC_SCRATCH_BYTES for
+// a batch that counts for no more than that (2048 x 64, one expert per token,
+// 886 tokens), so SCRATCH_BYTES holds every batch that is accepted.
 size_t jm::ws_noalloc_bytes(const jm_store* s, int B) {
     const size_t d = s->d, m = s->m, G = s->group, nslot = (size_t)B * s->topk;
     WsSizes z = ws_sizes(s, B);
